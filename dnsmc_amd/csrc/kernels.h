@@ -81,6 +81,9 @@ struct TraceArgs {
     const int4* slotinfo;       // processing slot -> {tally slot, cell, bricked index, i|j<<10|k<<20}
     float2* pray;               // per-ray (E, A) for the deterministic tally modes
     unsigned* claim;            // 8 super-chunk counters (one per XCD, 32 words apart), zero at launch
+    int retire_steps;           // a wave with a ray beyond this many crossings stops claiming work
+    unsigned retire_from;       // from this claim of its XCD's share on,
+    unsigned retire_most;       // at most this many waves of the launch (claim word 16 counts them)
     long long slot0;            // first slot of this batch
     int snap;
     // tallies

@@ -600,6 +600,65 @@ __device__ __forceinline__ bool long_candidate(const A& P, uint32_t q, uint32_t 
 // cand_cap).  A block takes tiles of kCandTile rays of one range and stages
 // the tile's hits in LDS: one global atomic per tile.
 constexpr uint32_t kCandTile = 4096;
+constexpr int kQuads = 16;   // rays a wave follows in the drain, four lanes each
+constexpr int kDrain = 16;   // crossings a ray moves ahead per batch of the drain (a multiple of 4)
+
+// Value of another lane of the quad (4 consecutive lanes): lane j of the quad
+// reads lane (CTRL >> 2 j) & 3.
+template <int CTRL>
+__device__ __forceinline__ int quad_i(int v)
+{
+    return __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true);
+}
+template <int CTRL>
+__device__ __forceinline__ float quad_f(float v)
+{
+    return __int_as_float(quad_i<CTRL>(__float_as_int(v)));
+}
+constexpr int kQuadXor1 = 0xB1, kQuadXor2 = 0x4E, kQuadPrev = 0x93;
+// Minimum over the quad (no NaN): v_min_f32 with the permuted operand; s_nop 1
+// gives the two wait states between a VALU write and its DPP read.
+__device__ __forceinline__ float quad_min(float v)
+{
+    float r;
+    asm("s_nop 1\n\tv_min_f32_dpp %0, %1, %1 quad_perm:[1,0,3,2] row_mask:0xf bank_mask:0xf\n\t"
+        "s_nop 1\n\tv_min_f32_dpp %0, %0, %0 quad_perm:[2,3,0,1] row_mask:0xf bank_mask:0xf"
+        : "=&v"(r)
+        : "v"(v));
+    return r;
+}
+// acc = fma(x of lane j of the quad, y_j, acc) for j = 0..3 in turn (s_nop 1:
+// the two wait states before the first DPP read of x); t: acc after each.
+#define DN_QFMA(x, y, j) "v_fmac_f32_dpp %0, " x ", " y " quad_perm:[" j "," j "," j "," j "] row_mask:0xf bank_mask:0xf\n\t"
+__device__ __forceinline__ void quad_fma(float& acc, float x, float y0, float y1, float y2, float y3)
+{
+    asm("s_nop 1\n\t" DN_QFMA("%1", "%2", "0") DN_QFMA("%1", "%3", "1") DN_QFMA("%1", "%4", "2") DN_QFMA("%1", "%5", "3")
+        : "+&v"(acc)
+        : "v"(x), "v"(y0), "v"(y1), "v"(y2), "v"(y3));
+}
+__device__ __forceinline__ void quad_fma_t(float& acc, float x, const float* y, float* t)
+{
+    asm("s_nop 1\n\t" DN_QFMA("%4", "%5", "0") "v_mov_b32 %1, %0\n\t" DN_QFMA("%4", "%6", "1") "v_mov_b32 %2, %0\n\t"
+        DN_QFMA("%4", "%7", "2") "v_mov_b32 %3, %0\n\t" DN_QFMA("%4", "%8", "3")
+        : "+&v"(acc), "=&v"(t[0]), "=&v"(t[1]), "=&v"(t[2])
+        : "v"(x), "v"(y[0]), "v"(y[1]), "v"(y[2]), "v"(y[3]));
+    t[3] = acc;
+}
+__device__ __forceinline__ int quad_sum(int v)
+{
+    v += quad_i<kQuadXor1>(v);
+    return v + quad_i<kQuadXor2>(v);
+}
+__device__ __forceinline__ int quad_max(int v)
+{
+    v = max(v, quad_i<kQuadXor1>(v));
+    return max(v, quad_i<kQuadXor2>(v));
+}
+__device__ __forceinline__ int quad_min_i(int v)
+{
+    v = min(v, quad_i<kQuadXor1>(v));
+    return min(v, quad_i<kQuadXor2>(v));
+}
 __global__ __launch_bounds__(256) void cand_scan(TraceArgs P, uint32_t nfin, uint32_t* list)
 {
     __shared__ uint32_t s_q[kCandTile];
@@ -971,13 +1030,80 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         return rd;
     };
 
+    // Retiring: a wave asked to claim more work near the launch's end (its last
+    // claim at retire_from or later) while one of its rays is beyond
+    // retire_steps crossings stops claiming, so that it reaches the drain below
+    // (over four times faster per crossing) while the other waves trace the
+    // rest.  At most retire_most waves of the launch do (asked once per wave,
+    // counted in claim word 16): the others remain to claim what is left.
+    uint32_t last_c = 0;
+    bool may_retire = P.retire_most > 0u;
+    auto retire = [&]() -> bool {
+        if (!may_retire || last_c < P.retire_from || !__ballot(alive && rsteps > P.retire_steps)) return false;
+        may_retire = false;
+        uint32_t k = 0;
+        if (lane == 0) k = atomicAdd(P.claim + 16, 1u);
+        return __builtin_amdgcn_readfirstlane(k) < P.retire_most;
+    };
+    // kappa and Ib of a ray's (band, g) rows at a field value
+    auto table_at = [&](float T, int kr, int ir, float& kap, float& ibj) {
+        if (SPEC == kSpecGreyT4) {
+            const float t2 = T * T;
+            kap = P.kappa_grey;
+            ibj = t2 * t2;
+            return;
+        }
+        int w;
+        float fr;
+        if (TAB == kTabSliced) {
+            w = (int)T;
+            w = w > nw - 2 ? nw - 2 : w;
+            fr = T - (float)w;
+        } else {
+            float pos = fmaf(T, P.inv_dT, P.mT0);
+            pos = fminf(fmaxf(pos, 0.0f), (float)(nT - 1));
+            w = (int)pos;
+            w = w > nT - 2 ? nT - 2 : w;
+            fr = pos - (float)w;
+        }
+        const float k0 = TAB == kTabSliced ? s_kq[kr + w] : kq[kr + w];
+        const float k1 = TAB == kTabSliced ? s_kq[kr + w + 1] : kq[kr + w + 1];
+        const float i0 = ibt[ir + w], i1 = ibt[ir + w + 1];
+        kap = fmaf(fr, k1 - k0, k0);
+        ibj = fmaf(fr, i1 - i0, i0);
+    };
+    // adaptive mesh coarsening (code/mc_gpu.cu:193-207): the lane's ray goes on
+    // in the next coarser level
+    auto coarser = [&]() {
+        ++lev;
+        const int* L = s_lev + lev * kLevWords;
+        n0 = L[0]; n1 = L[1]; n2 = L[2];
+        fo0 = L[3]; fo1 = L[4]; fo2 = L[5]; maxs = L[6];
+        oo0 = L[11]; oo1 = L[12]; oo2 = L[13];
+        Tl = lev_T(L);
+        if (GEN) Tl += (size_t)rsnap * (uint32_t)L[14];
+        // ic = (ic + r - 1) / r with r = 2: every level halves each axis
+        // (level g has n >> g cells)
+        cx = (cx + 1) >> 1;
+        cy = (cy + 1) >> 1;
+        cz = (cz + 1) >> 1;
+        fx = face_at(fo0, cx - (fl & 1));
+        fy = face_at(fo1, cy - ((fl >> 1) & 1));
+        fz = face_at(fo2, cz - ((fl >> 2) & 1));
+        idx = off_at(oo0, cx) + off_at(oo1, cy) + off_at(oo2, cz);
+        Tc = load_T(Tl, idx);
+        cnt = 0;
+    };
+
     for (;;) {
         const bool idle = !alive;
         const unsigned long long m_idle = __ballot(idle);
         const int ni = __popcll(m_idle);
         const int na = 64 - ni;
         const bool have_rays = more || cur < cend || ghead < gn || (int)cand < 0;
-        if (na == 0 && !have_rays) break;
+        // nothing left to hand out and few rays alive: the drain follows them
+        // (on the last level; coarsening has few crossings before it)
+        if (!have_rays && na <= kQuads && (!AMC || !__ballot(alive && lev + 1 < P.nlev))) break;
         if (have_rays && (ni >= P.refill_k || na == 0)) {
             // ---- tally the rays finished since the last refill
             if (!QUEUE && TMODE == 0) flush_wave(P, fin && rslot != aslot && aslot >= 0, aslot, aE, aA, aQ, lane);
@@ -1056,6 +1182,10 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                 ghead += t1;
                 if (t1 < (uint32_t)ni) {
                     bool drawn = false;
+                    if (GEN == 1 && (int)cand < 0 && retire()) {
+                        more = false;
+                        cand &= 0x7FFFFFFFu;
+                    }
                     if (GEN == 1 && (int)cand < 0) {
                         // the next (up to) 64 listed long rays, all of the last
                         // snapshot, from this XCD's list first; no ring entries (their
@@ -1081,6 +1211,10 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                             break;
                         }
                     }
+                    if (!drawn && cur >= cend && more && retire()) {
+                        more = false;
+                        cand &= 0x7FFFFFFFu;
+                    }
                     if (!drawn && cur >= cend && more) {
                         // claim the next super-chunk, from this XCD's share first,
                         // then from the following XCDs' shares.  Claim c of XCD X is
@@ -1098,6 +1232,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                             const uint32_t sn = c / per_x;
                             const uint32_t lc = X * per_x + (c - sn * per_x);
                             if (lc >= cps) continue;   // past the snapshot's last chunk
+                            last_c = c;
                             csnap = sn;
                             cur = lc * S;
                             cend = cur + S < nrays ? cur + S : nrays;
@@ -1204,6 +1339,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                 const uint32_t avail = cend - cur;
                 uint32_t q = 0xFFFFFFFFu, qs = csnap;
                 if (idle && rank < avail) q = cur + rank;
+                if (avail < (uint32_t)ni && more && retire()) more = false;
                 if (avail < (uint32_t)ni && more) {
                     // the current super-chunk runs out: claim the next one (as above)
                     bool got = false;
@@ -1220,6 +1356,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                         const uint32_t sn = c / per_x;
                         const uint32_t lc = X * per_x + (c - sn * per_x);
                         if (lc >= cps) continue;   // past the snapshot's last chunk
+                        last_c = c;
                         nsn = sn;
                         nstart = lc * S;
                         nend = nstart + S < nrays ? nstart + S : nrays;
@@ -1352,29 +1489,228 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
             alive = false; fin = true; endt = cut ? 0 : 1; Dfin = 1.0f;
         } else if (cap) {
             if (AMC && lev + 1 < P.nlev) {
-                // adaptive mesh coarsening (code/mc_gpu.cu:193-207)
-                ++lev;
-                const int* L = s_lev + lev * kLevWords;
-                n0 = L[0]; n1 = L[1]; n2 = L[2];
-                fo0 = L[3]; fo1 = L[4]; fo2 = L[5]; maxs = L[6];
-                oo0 = L[11]; oo1 = L[12]; oo2 = L[13];
-                Tl = lev_T(L);
-                if (GEN) Tl += (size_t)rsnap * (uint32_t)L[14];
-                // ic = (ic + r - 1) / r with r = 2: every level halves each axis
-                // (level g has n >> g cells)
-                cx = (cx + 1) >> 1;
-                cy = (cy + 1) >> 1;
-                cz = (cz + 1) >> 1;
-                fx = face_at(fo0, cx - (fl & 1));
-                fy = face_at(fo1, cy - ((fl >> 1) & 1));
-                fz = face_at(fo2, cz - ((fl >> 2) & 1));
-                idx = off_at(oo0, cx) + off_at(oo1, cy) + off_at(oo2, cz);
-                Tc = load_T(Tl, idx);
-                cnt = 0;
+                coarser();
             } else {
                 alive = false; fin = true; endt = 2; Dfin = 1.0f - tra;
             }
         }
+    }
+    // ---- drain: nothing is left to hand out and at most 16 of the wave's rays
+    // run on, on the last level.  Such a ray is a serial chain (along the walls
+    // in a thin bin up to the step cap, 1e5 crossings): one crossing per
+    // iteration of the loop above takes 350 ns, 840 cycles, of which 380 issue
+    // its 95 instructions and the rest waits for LDS and the field; a
+    // 64x96x64 solve of 2e8 rays spent 36 of its 46 ms here.  So four lanes
+    // follow one ray.  The cells a ray crosses do not depend on the field:
+    // lane a of the quad holds axis a (lane 3 none) and the quad moves kDrain
+    // crossings ahead, the nearest face by quad permutes, the two faces behind
+    // the exit face read ahead.  Then the batch's field loads and table
+    // lookups run in parallel, crossing 4 k + j on lane j, and tau and G
+    // follow in crossing order with the main loop's arithmetic (a crossing
+    // past the ray's end has length 0 and adds 0): 122 ns per crossing, the
+    // solve 46 -> 24 ms (18 to 24 with retiring waves, above).
+    if (__ballot(alive)) {
+        __builtin_amdgcn_s_setprio(3);   // ahead of the waves that still trace the bulk
+        const unsigned long long am = __ballot(alive);
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(am >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)am, 0u));
+        // the lane of the ray that this quad follows: its rank-th alive lane
+        // (each alive lane sends its number to lane 4 rank, the others to 63)
+        int src = quad_i<0>(__builtin_amdgcn_ds_permute(alive ? 16 * rank : 4 * 63, lane));
+        const int a = lane & 3;
+        const bool ax3 = a == 3;
+        bool run = (lane >> 2) < __popcll(am);
+        src = run ? src : 0;
+        auto axis_f = [&](float x, float y, float z, float w) -> float {
+            const float vx = __shfl(x, src), vy = __shfl(y, src), vz = __shfl(z, src);
+            return a == 0 ? vx : (a == 1 ? vy : (a == 2 ? vz : w));
+        };
+        // (lane 3 is never the nearest face: distance 3e38)
+        float qp = axis_f(px, py, pz, 0.0f), qs = axis_f(sx, sy, sz, 0.0f), qi = axis_f(ix, iy, iz, 1.0f);
+        float qf = axis_f(fx, fy, fz, 3.0e38f);
+        int qc;                                          // 0-based cell
+        {
+            const int vx = __shfl(cx, src), vy = __shfl(cy, src), vz = __shfl(cz, src);
+            // (a quad without a ray stays frozen in cell 0: lane 0's last ray may
+            // have ended on a finer level, whose cells this level does not have)
+            qc = !run ? 0 : (a == 0 ? vx - 1 : (a == 1 ? vy - 1 : (a == 2 ? vz - 1 : 0)));
+        }
+        const bool neg = (__shfl(fl, src) >> a) & 1;     // (fl has 3 bits)
+        const int st = neg ? -1 : 1;
+        float qtau = __shfl(tau, src), qtra = __shfl(tra, src), qG = __shfl(G, src);
+        const int qkrow = __shfl(krow, src), qibrow = __shfl(ibrow, src), qband = __shfl(band, src);
+        int qcnt = __shfl(cnt, src), qsteps = __shfl(rsteps, src), qend = 0;
+        float qD = 1.0f;
+        uint32_t qhash = REC ? (uint32_t)__shfl((int)hash, src) : 0u;
+        const int bcbit = 2 * a + (neg ? 0 : 1);         // the boundary this axis runs into
+        const bool per = (P.bc_periodic >> bcbit) & 1;
+        // the last level: cells along this axis, LDS bytes of the face behind the
+        // exit face of cell 0 and of its brick offset
+        const int* L = s_lev + (P.nlev - 1) * kLevWords;
+        const int qn = ax3 ? 0x7FFFFFFF : L[a], qmaxs = L[6];
+        const int gb = L[3 + (ax3 ? 0 : a)] + (neg ? -4 : 8), ob = L[11 + (ax3 ? 0 : a)] + 4;
+        const int qstride = a == 0 ? 1 : (a == 1 ? L[0] : (a == 2 ? L[0] * L[1] : 0));
+        gfloat* qT = lev_T(L);
+        if (GEN) qT += (size_t)(uint32_t)__shfl((int)rsnap, src) * (uint32_t)L[14];
+        // face i behind (+) or before (-) the exit face of cell c: word c + i st of
+        // the face table from gb - st (a word past the axis's faces is one of its
+        // LDS neighbours and is not used)
+        auto face_w = [&](int byte, int i) -> float { return *(const float*)((const char*)s_face + byte + (i << 2)); };
+        while (__ballot(run)) {
+            int lim = run ? min(kDrain, qmaxs - qcnt) : 0;
+            int wall = -1;
+            // a frozen quad (no ray, or its ray hit a wall inside the batch) has
+            // length-0 crossings and does not move
+            unsigned long long live = __ballot(run);
+            int nlive = __popcll(live) >> 2;
+            qs = run ? qs : 0.0f;
+            qi = run ? qi : 0.0f;
+            float dsv[kDrain];
+            int oid[kDrain / 4], lin[kDrain / 4];
+            float g = face_w(gb, qc), h = face_w(gb + 4 * st, qc);
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                int ov[4];
+                oid[k] = lin[k] = 0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int u = 4 * k + j;
+                    ov[j] = off_at(ob, qc);
+                    const float d = (qf - qp) * qi;
+                    const float ds = quad_min(d);
+                    dsv[u] = ds;
+                    unsigned long long em = __ballot(d == ds) & live;
+                    qp = __builtin_amdgcn_inverse_ballot_w64(em) ? qf : fmaf(ds, qs, qp);
+                    // of several axes at the same distance the last one moves
+                    if (__builtin_expect(__popcll(em) != nlive, 0))
+                        em &= ~((em >> 1) | ((em >> 2) & 0x1111111111111111ull));
+                    const bool mv = __builtin_amdgcn_inverse_ballot_w64(em);
+                    if (REC) {
+                        const int l = quad_sum(qc * qstride);
+                        lin[k] = a == j ? l : lin[k];
+                    }
+                    qc += mv ? st : 0;
+                    qf = mv ? g : qf;
+                    g = mv ? h : g;
+                    const bool out = (uint32_t)qc >= (uint32_t)qn;
+                    if (__builtin_expect(__ballot(out) != 0ull, 0)) {
+                        int w = -1;
+                        if (out) {
+                            if (per) {
+                                qc = neg ? qn - 1 : 0;
+                                qp = face_w(gb - 8 * st, neg ? qn - 1 : 0);
+                            } else {
+                                w = bcbit;
+                                qc -= st;
+                            }
+                            qf = face_w(gb - 4 * st, qc);
+                            g = face_w(gb, qc);
+                        }
+                        w = quad_max(w);
+                        const bool hit = w >= 0;
+                        wall = hit && u < lim ? w : wall;
+                        lim = hit ? min(lim, u + 1) : lim;
+                        qs = hit ? 0.0f : qs;
+                        qi = hit ? 0.0f : qi;
+                        live &= ~__ballot(hit);
+                        nlive = __popcll(live) >> 2;
+                        __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0) here, not on the common path)
+                    }
+                    h = face_w(gb + 4 * st, qc);
+                }
+                // the cells' field offsets: crossing 4 k + j to lane j
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int ou = quad_sum(ax3 ? 0 : ov[j]);
+                    oid[k] = a == j ? ou : oid[k];
+                }
+            }
+            if (__ballot(run && lim < kDrain)) {             // the step cap inside the batch
+#pragma unroll
+                for (int u = 0; u < kDrain; ++u) dsv[u] = u < lim ? dsv[u] : 0.0f;
+            }
+            // the cells' temperatures and lookups
+            float Tv[kDrain / 4], kap[kDrain / 4], ibv[kDrain / 4], tk[kDrain / 4], dg[kDrain / 4];
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) Tv[k] = load_T(qT, oid[k]);
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) table_at(Tv[k], qkrow, qibrow, kap[k], ibv[k]);
+            // optical depth in crossing order (every lane of the quad), kept by
+            // the crossing's lane
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                float t[4];
+                quad_fma_t(qtau, kap[k], dsv + 4 * k, t);
+                tk[k] = a == 0 ? t[0] : (a == 1 ? t[1] : (a == 2 ? t[2] : t[3]));
+            }
+            // transmissivities; the first crossing past the cut-off
+            int first = kDrain;
+            float before = qtra;   // transmissivity before this group of four
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                const bool cut = tk[k] >= P.tau_cut;
+                const float t1 = __expf(-tk[k]);
+                const float t0 = quad_f<kQuadPrev>(t1);      // (every lane of the quad takes part)
+                const float tp = a == 0 ? before : t0;
+                dg[k] = cut ? tp : tp - t1;
+                first = min(first, cut ? 4 * k + a : kDrain);
+                before = quad_f<0xFF>(t1);
+            }
+            bool cutq = false;
+            int taken = lim;
+            if (__ballot(first < lim)) {
+                first = quad_min_i(first);
+                cutq = first < lim;
+                taken = cutq ? first + 1 : lim;
+#pragma unroll
+                for (int k = 0; k < kDrain / 4; ++k) dg[k] = 4 * k + a < taken ? dg[k] : 0.0f;
+            }
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                quad_fma(qG, dg[k], quad_f<0x00>(ibv[k]), quad_f<0x55>(ibv[k]), quad_f<0xAA>(ibv[k]), quad_f<0xFF>(ibv[k]));
+            }
+            if (REC) {
+                const uint32_t lb = (uint32_t)(P.nlev - 1) << 28;
+#pragma unroll
+                for (int k = 0; k < kDrain / 4; ++k) {
+                    const uint32_t l0 = (uint32_t)quad_i<0x00>(lin[k]), l1 = (uint32_t)quad_i<0x55>(lin[k]);
+                    const uint32_t l2 = (uint32_t)quad_i<0xAA>(lin[k]), l3 = (uint32_t)quad_i<0xFF>(lin[k]);
+                    if (4 * k < taken) qhash = (qhash ^ (lb ^ l0)) * 16777619u;
+                    if (4 * k + 1 < taken) qhash = (qhash ^ (lb ^ l1)) * 16777619u;
+                    if (4 * k + 2 < taken) qhash = (qhash ^ (lb ^ l2)) * 16777619u;
+                    if (4 * k + 3 < taken) qhash = (qhash ^ (lb ^ l3)) * 16777619u;
+                }
+            }
+            qtra = before;   // (not used after a cut-off)
+            qcnt += taken;
+            qsteps += taken;
+            const bool hitw = run && !cutq && wall >= 0;
+            if (hitw) qG = fmaf(qtra, s_ibw[wall * P.nB + qband], qG);
+            if (run && (cutq || hitw)) {
+                run = false;
+                qend = cutq ? 0 : 1;
+                qtau = 0.0f;   // (the quad idles below the cut-off: it adds 0)
+                qtra = 1.0f;
+            } else if (run && qcnt >= qmaxs) {
+                run = false;
+                qend = 2;
+                qD = 1.0f - qtra;
+            }
+        }
+        // back to the lanes that held the rays
+        const int from = alive ? 4 * rank : lane;
+        const float rG = __shfl(qG, from), rD = __shfl(qD, from);
+        const int rsn = __shfl(qsteps, from), ren = __shfl(qend, from);
+        const uint32_t rh = REC ? (uint32_t)__shfl((int)qhash, from) : 0u;
+        if (alive) {
+            G = rG;
+            Dfin = rD;
+            rsteps = rsn;
+            endt = ren;
+            if (REC) hash = rh;
+            alive = false;
+            fin = true;
+        }
+        __builtin_amdgcn_s_setprio(0);
     }
     // a ray that ended after the last refill (nothing was left to hand out)
     if (!QUEUE && TMODE == 0) flush_wave(P, fin && rslot != aslot && aslot >= 0, aslot, aE, aA, aQ, lane);
