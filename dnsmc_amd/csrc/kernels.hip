@@ -1030,6 +1030,17 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         return rd;
     };
 
+    // Next claim of XCD X's share (nclaim or more: none left).  Another XCD's
+    // counter is read first: in a small launch every wave visits all eight at
+    // the end, and reads of a used-up counter do not queue as atomics do.
+    auto claim_of = [&](uint32_t X) -> uint32_t {
+        uint32_t c = 0;
+        if (lane == 0) {
+            if (xi > 0u) c = __hip_atomic_load(P.claim + 32u * X, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            if (c < nclaim) c = atomicAdd(P.claim + 32u * X, 1u);
+        }
+        return __builtin_amdgcn_readfirstlane(c);
+    };
     // Retiring: a wave asked to claim more work near the launch's end (its last
     // claim at retire_from or later) while one of its rays is beyond
     // retire_steps crossings stops claiming, so that it reaches the drain below
@@ -1222,9 +1233,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                         bool got = false;
                         while (xi < nparts) {
                             const uint32_t X = (xcd + xi) % nparts;
-                            uint32_t c = 0;
-                            if (lane == 0) c = atomicAdd(P.claim + 32u * X, 1u);
-                            c = __builtin_amdgcn_readfirstlane(c);
+                            const uint32_t c = claim_of(X);
                             if (c >= nclaim) {
                                 ++xi;
                                 continue;
@@ -1346,9 +1355,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                     uint32_t nstart = 0, nend = 0, nsn = 0;
                     while (xi < nparts) {
                         const uint32_t X = (xcd + xi) % nparts;
-                        uint32_t c = 0;
-                        if (lane == 0) c = atomicAdd(P.claim + 32u * X, 1u);
-                        c = __builtin_amdgcn_readfirstlane(c);
+                        const uint32_t c = claim_of(X);
                         if (c >= nclaim) {
                             ++xi;
                             continue;

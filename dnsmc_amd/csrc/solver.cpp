@@ -1046,8 +1046,14 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
         P.refill_k = rk ? atoi(rk) : (!det && !s->record ? rk_queue : 16);
         if (P.refill_k < 1) P.refill_k = 1;
         if (P.refill_k > 64) P.refill_k = 64;
+        // a small launch takes shorter super-chunks, so that its rays spread over
+        // the resident waves (about 16 per CU), four claims each: grey solves of
+        // 16x24x16 cells x 32 rays 0.57 ms with 512-ray chunks on a grid of 16
+        // chunks per block, 0.09 ms; 32x32x32 x 100 rays 0.96 and 0.51 ms
         const char* sc = getenv("DNSMC_SUPER");
-        P.super = sc ? atoi(sc) : (fused || snapwise ? 512 : 256);
+        const long long lrays = (fused ? std::min(fused_part, nslots) * c.nsnap : std::min(slots_per_batch, nslots)) * (long long)R;
+        const long long even = lrays / (4ll * 16 * s->ncu) / 64 * 64;
+        P.super = sc ? atoi(sc) : (int)std::max(64ll, std::min<long long>(fused || snapwise ? 512 : 256, even));
         P.super = std::max(64, (P.super + 63) / 64 * 64);
     }
     P.slotinfo = s->d_slotinfo.p;
@@ -1112,7 +1118,11 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
         if (lds_learn > s->lds_max) return fail(DNSMC_EINVAL, "too many (band, g) bins for the learned proposal");
     }
 
-    const int trace_blocks = s->ncu * 16;
+    // persistent grids, shrunk for small launches to one wave per 64 rays
+    // (blocks of four waves)
+    auto trace_cap = [&](long long rays) {
+        return (int)std::min<long long>((long long)s->ncu * 16, std::max<long long>(8, (rays + 255) / 256));
+    };
     s->first_batch_rays = 0;
     P.nsnap_launch = 1;
     P.tally_stride = 0;
@@ -1168,6 +1178,20 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
         }
         // long rays first (the plain in-kernel draw; DNSMC_LONG_FIRST=0: off)
         bool long_first = !lfused;
+        // a grey ray ends after tau_cut / kappa of path: with few crossings at
+        // most there is no long ray to list; nor is there an order to choose
+        // when every ray of the launch starts at once
+        if (spec == kSpecGreyT4) {
+            double cross = 0.0;
+            for (int a = 0; a < 3; ++a) {
+                const std::vector<float>& f = s->lev[0].faces[a];
+                float dmin = c.L[a];
+                for (size_t i = 1; i < f.size(); ++i) dmin = std::min(dmin, f[i] - f[i - 1]);
+                cross += (double)P.tau_cut / c.kappa_grey / dmin;
+            }
+            if (cross < 4096.0) long_first = false;
+        }
+        if (nslots * (long long)R * c.nsnap <= 16ll * 64 * s->ncu) long_first = false;
         if (const char* lf = getenv("DNSMC_LONG_FIRST")) long_first = long_first && atoi(lf) != 0;
         // the listed part, the final 1/long_part of each XCD range of the last
         // snapshot: a half in launches of several snapshots, a quarter in
@@ -1217,8 +1241,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
                 hipLaunchKernelGGL(cand_scan, dim3(nb), dim3(256), 0, ls, P, (uint32_t)nfin, cp.d_cand.p);
                 HIPCHK(hipGetLastError());
             }
-            const long long nsc = ((P.nrays + P.super - 1) / P.super) * c.nsnap;
-            const int tb_cap = (int)std::min<long long>(trace_blocks, std::max<long long>(8, (nsc + 15) / 16));
+            const int tb_cap = trace_cap(P.nrays * c.nsnap);
             EventPair* et = na ? nullptr : &next_event(s, 1);
             if (et) HIPCHK(hipEventRecord(et->a, ls));
             HIPCHK(launch_trace(spec, tab, lfused ? 2 : 1, false, false, amc, s->ncu, tb_cap, lds_trace, ls, P));
@@ -1270,8 +1293,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             P.claim = tp.d_claim.p;
             hipLaunchKernelGGL(fill_u32, dim3(1), dim3(256), 0, ts, tp.d_claim.p, 256ll, 0u);
             HIPCHK(hipGetLastError());
-            const long long nsc = (P.nrays + P.super - 1) / P.super;
-            const int tb_cap = (int)std::min<long long>(trace_blocks, std::max<long long>(8, (nsc + 15) / 16));
+            const int tb_cap = trace_cap(P.nrays);
             EventPair& et = next_event(s, 1);
             HIPCHK(hipEventRecord(et.a, ts));
             HIPCHK(launch_trace(spec, tab, false, false, false, amc, s->ncu, tb_cap, lds_trace, ts, P));
@@ -1325,9 +1347,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             P.Q2 = s->d_Q2.p + (size_t)snap * nslots;
             P.nrec = (s->record && snap == 0 && b0 == 0) ? s->nrec : 0;
             bool rec = P.nrec > 0;
-            // persistent grid, shrunk for small launches (about 4 super-chunks per wave)
-            const long long nsc = (nr + P.super - 1) / P.super;
-            const int tb_cap = (int)std::min<long long>(trace_blocks, std::max<long long>(8, (nsc + 15) / 16));
+            const int tb_cap = trace_cap(nr);
             P.claim = pp.d_claim.p;
             hipLaunchKernelGGL(fill_u32, dim3(1), dim3(256), 0, st, pp.d_claim.p, 256ll, 0u);
             HIPCHK(hipGetLastError());
