@@ -9,6 +9,7 @@
 namespace dn {
 
 constexpr int kLevWords = 16;   // per-level parameter words staged in LDS
+constexpr float kFaceEnd = 3.0e38f;   // before and after each axis's faces in the packed face buffer
 constexpr int kRing = 8;        // tally ring entries per wave (power of 2)
 constexpr int kLRowFloats = 2048;   // a learned proposal row in a wave's row buffer (4 chunks x 64 lanes x 8)
 
@@ -61,7 +62,7 @@ struct TraceArgs {
     const float* Ibw;           // wall Planck [(axis*2+side)*nB + b]
     const float* faces;         // all levels packed
     int nfaces;
-    const int* offs;            // per level and axis: brick-layout offset of 0-based cell index c
+    const int* offs;            // per level and axis: brick-layout byte offset of 0-based cell index c
     int noffs;
     const float* centres;       // level 0, x|y|z packed, ghost-inclusive
     int coff[3];
@@ -83,7 +84,7 @@ struct TraceArgs {
     unsigned* claim;            // 8 super-chunk counters (one per XCD, 32 words apart), zero at launch
     int retire_steps;           // a wave with a ray beyond this many crossings stops claiming work
     unsigned retire_from;       // from this claim of its XCD's share on,
-    unsigned retire_most;       // at most this many waves of the launch (claim word 16 counts them)
+    unsigned retire_most;       // at most this many waves of the launch (claim words 16 to 19 count them)
     long long slot0;            // first slot of this batch
     int snap;
     // tallies

@@ -357,13 +357,22 @@ __device__ __forceinline__ gfloat* lev_T(const int* L)
     return (gfloat*)u;
 }
 
-// Temperature of bricked cell index idx: a 32-bit byte offset from the level
-// base (fields stay below 4 GiB), so a uniform base addresses in one VGPR.
-__device__ __forceinline__ float load_T(gfloat* base, int idx)
+// Temperature at a byte offset from the level base (a level of one snapshot
+// stays within 4 GiB).
+__device__ __forceinline__ float load_T(gfloat* base, int byte)
 {
     typedef __attribute__((address_space(1))) const char gchar;
-    return *(gfloat*)((gchar*)base + (uint32_t)idx * 4u);
+    return *(gfloat*)((gchar*)base + (uint32_t)byte);
 }
+
+// Smallest of three numbers (none NaN).
+__device__ __forceinline__ float min3(float a, float b, float c)
+{
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+}
+
 
 // Wave-aggregated tally atomics: the lanes with `need` set hand their running
 // slot sums over, grouped by slot; each group is summed across the wave and
@@ -414,12 +423,12 @@ __device__ __forceinline__ void tally_ray(const TraceArgs& P, float er, float ar
     aQ += x * x;
 }
 
-// A drawn ray, as the refill hands it to a lane: bricked index and packed
-// (i, j, k) of the emitting cell, its tally slot, band | g << 16 | sign flags
+// A drawn ray, as the refill hands it to a lane: packed (i, j, k) of the
+// emitting cell, its tally slot, band | g << 16 | sign flags
 // << 24, its processing slot in the launch, emitter temperature, direction and
 // its reciprocals, weights, emission point (the cell centre).
 struct RayStart {
-    int idx, cell, six, bg, ps;
+    int cell, six, bg, ps;
     float Tc, sx, sy, sz, ix, iy, iz, rw, rwi, px, py, pz;
 };
 
@@ -427,7 +436,6 @@ struct RayStart {
 __device__ __forceinline__ RayStart pull_ray(const RayStart& r, int src)
 {
     RayStart o;
-    o.idx = __shfl(r.idx, src);
     o.cell = __shfl(r.cell, src);
     o.six = __shfl(r.six, src);
     o.bg = __shfl(r.bg, src);
@@ -600,6 +608,14 @@ __device__ __forceinline__ bool long_candidate(const A& P, uint32_t q, uint32_t 
 // cand_cap).  A block takes tiles of kCandTile rays of one range and stages
 // the tile's hits in LDS: one global atomic per tile.
 constexpr uint32_t kCandTile = 4096;
+// Crossings per iteration of the traversal, their field loads in flight together
+// (a wave's lanes meet an L2 miss nearly every crossing, and only four waves
+// per SIMD hide it).  A ray that ends inside an iteration wastes the rest.
+// 384x256x256 on one level: 403 / 371 / 378 / 386 / 398 ms at 1 / 2 / 3 / 4 / 6
+// (the loop before: 398; L2 reads per crossing 0.88 -> 0.64, VALU instructions
+// 2.19 -> 1.76); two coarsened 256x128x128 snapshots, five crossings on each
+// finer level: 48.0 / 47.3 / 45.6 / 49.0 / 42.8 ms at 1 / 2 / 3 / 4 / 5 (44.4).
+constexpr int kAheadFine = 2, kAheadLev = 5;
 constexpr int kQuads = 16;   // rays a wave follows in the drain, four lanes each
 constexpr int kDrain = 16;   // crossings a ray moves ahead per batch of the drain (a multiple of 4)
 
@@ -758,10 +774,13 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     float* s_face = (float*)(s_lev + 6 * kLevWords);
     int* s_off = (int*)(s_face + P.nfaces);     // brick offsets per level and axis
     float* s_ibw = (float*)(s_off + P.noffs);   // 6 * nB wall Planck values
-    // face i of the face table at byte offset fb, brick offset of 1-based
-    // cell c of the table at byte offset ob (both offsets from the level block)
-    auto face_at = [&](int fb, int i) -> float { return *(const float*)((const char*)s_face + fb + (i << 2)); };
-    auto off_at = [&](int ob, int c) -> int { return *(const int*)((const char*)s_off + ob + (c << 2)); };
+    // words of LDS by address (an address is one register, no base to add)
+    typedef __attribute__((address_space(3))) const float lfloat;
+    typedef __attribute__((address_space(3))) const int lint;
+    auto lds_at = [&](const void* q) -> int { return (int)(uint32_t)(uintptr_t)(lfloat*)q; };
+    auto lds_f = [&](int at) -> float { return *(lfloat*)(uintptr_t)(uint32_t)at; };
+    auto lds_i = [&](int at) -> int { return *(lint*)(uintptr_t)(uint32_t)at; };
+    const int face0 = lds_at(s_face), off0 = lds_at(s_off);
     float* s_ib = s_ibw + 6 * P.nB;             // Ib rows (nT or tab_nw nodes)
     const int nw = P.tab_nw;
     float* s_kq = s_ib + P.nB * nw;             // sliced kappa rows (kTabSliced)
@@ -772,9 +791,9 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     for (int i = threadIdx.x; i < P.nlev; i += blockDim.x) {
         int* L = s_lev + i * kLevWords;
         L[0] = P.lev[i].n[0]; L[1] = P.lev[i].n[1]; L[2] = P.lev[i].n[2];
-        // face and brick-offset table positions as byte offsets into s_face
-        // and s_off (the offsets' -1 of the 1-based cell index folded in)
-        L[3] = 4 * P.lev[i].foff[0]; L[4] = 4 * P.lev[i].foff[1]; L[5] = 4 * P.lev[i].foff[2];
+        // per axis: LDS address of face 0, and from a cell's low face (word
+        // c - 1 of 1-based cell c) to its word of the brick-offset table
+        L[3] = face0 + 4 * P.lev[i].foff[0]; L[4] = face0 + 4 * P.lev[i].foff[1]; L[5] = face0 + 4 * P.lev[i].foff[2];
         L[6] = P.lev[i].maxs;
         const float* tb = P.T[i] + (size_t)P.snap * P.lev[i].tstride;
         unsigned long long u = (unsigned long long)tb;
@@ -782,10 +801,11 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         L[8] = (int)(uint32_t)(u >> 32);
         L[9] = P.lev[i].nbx;
         L[10] = P.lev[i].nby;
-        L[11] = 4 * (P.lev[i].ooff[0] - 1);
-        L[12] = 4 * (P.lev[i].ooff[1] - 1);
-        L[13] = 4 * (P.lev[i].ooff[2] - 1);
+        for (int a = 0; a < 3; ++a) L[11 + a] = off0 - face0 + 4 * (P.lev[i].ooff[a] - P.lev[i].foff[a]);
         L[14] = (int)P.lev[i].tstride;
+        int before = 0;                          // crossings on the finer levels
+        for (int g = 0; g < i; ++g) before += P.lev[g].maxs;
+        L[15] = before;
     }
     for (int i = threadIdx.x; i < P.nfaces; i += blockDim.x) s_face[i] = P.faces[i];
     for (int i = threadIdx.x; i < P.noffs; i += blockDim.x) s_off[i] = P.offs[i];
@@ -819,6 +839,9 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     const float* ibt = TAB == kTabGlobal ? P.Ib : s_ib;
     gfloat* kq = (gfloat*)P.kq;
     const int rowlen = TAB == kTabSliced ? nw : P.nT;   // nodes per table row
+    // a ray's table rows: element indices, or (sliced) LDS word indices
+    const int kr0 = TAB == kTabSliced ? lds_at(s_kq) >> 2 : 0;
+    const int ir0 = TAB == kTabSliced ? lds_at(s_ib) >> 2 : 0;
 
     const int lane = threadIdx.x & 63;
     const unsigned nb = gridDim.x, b = blockIdx.x;
@@ -845,19 +868,21 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     float Dfin = 1.0f;
     float px = 0.f, py = 0.f, pz = 0.f, sx = 1.f, sy = 1.f, sz = 1.f, ix = 1.f, iy = 1.f, iz = 1.f;
     float fx = 0.f, fy = 0.f, fz = 0.f, tau = 0.f, tra = 1.f, G = 0.f, rw = 0.f, rwi = 0.f, Tc = 0.f;
-    int cx = 1, cy = 1, cz = 1, fl = 0, krow = 0, ibrow = 0, band = 0, lev = 0, cnt = 0, idx = 0, rsteps = 0;
+    // The ray's cell, as three LDS addresses: A_a of its exit face along axis a
+    // (bytes; + s_a, +-4, one cell further), and A_a + K_a its word of the
+    // axis's brick-offset table.
+    int A0 = s_lev[3], A1 = s_lev[4], A2 = s_lev[5], K0 = s_lev[11], K1 = s_lev[12], K2 = s_lev[13];
+    int s0 = 4, s1 = 4, s2 = 4;
+    int krow = 0, ibrow = 0, band = 0, lev = 0, cnt = 0, rsteps = 0;
     uint32_t hash = 2166136261u;
-    int n0 = s_lev[0], n1 = s_lev[1], n2 = s_lev[2];
-    int fo0 = s_lev[3], fo1 = s_lev[4], fo2 = s_lev[5], maxs = s_lev[6];
-    int oo0 = s_lev[11], oo1 = s_lev[12], oo2 = s_lev[13];
-    if (!AMC) {   // one level: its parameters are the same for every lane (scalar registers)
-        n0 = __builtin_amdgcn_readfirstlane(n0); n1 = __builtin_amdgcn_readfirstlane(n1);
-        n2 = __builtin_amdgcn_readfirstlane(n2);
-        fo0 = __builtin_amdgcn_readfirstlane(fo0); fo1 = __builtin_amdgcn_readfirstlane(fo1);
-        fo2 = __builtin_amdgcn_readfirstlane(fo2); maxs = __builtin_amdgcn_readfirstlane(maxs);
-        oo0 = __builtin_amdgcn_readfirstlane(oo0); oo1 = __builtin_amdgcn_readfirstlane(oo1);
-        oo2 = __builtin_amdgcn_readfirstlane(oo2);
-    }
+    int maxs = s_lev[6];
+    if (!AMC) maxs = __builtin_amdgcn_readfirstlane(maxs);
+    // level 0's LDS addresses (scalar registers: every ray starts there)
+    const int f00 = __builtin_amdgcn_readfirstlane(s_lev[3]), f01 = __builtin_amdgcn_readfirstlane(s_lev[4]);
+    const int f02 = __builtin_amdgcn_readfirstlane(s_lev[5]), k00 = __builtin_amdgcn_readfirstlane(s_lev[11]);
+    const int k01 = __builtin_amdgcn_readfirstlane(s_lev[12]), k02 = __builtin_amdgcn_readfirstlane(s_lev[13]);
+    // 0-based cell along axis a of the level block L
+    auto cell_of = [&](const int* L, int a, int A, int s) -> int { return ((A - L[3 + a]) >> 2) - (s > 0 ? 1 : 0); };
     gfloat* Tl = lev_T(s_lev);
     gfloat* T0 = Tl;
     uint32_t rsnap = 0;
@@ -922,7 +947,6 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         const uint32_t slot = fdiv(q, P.fd_R);
         const int4 si = P.slotinfo[P.slot0 + slot];
         rd.six = si.x;
-        rd.idx = si.z;
         rd.cell = si.w;
         rd.ps = (int)slot + (int)qs * nslot_l;
         rd.px = P.centres[P.coff[0] + (si.w & 1023) + 1];
@@ -1042,21 +1066,47 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         return __builtin_amdgcn_readfirstlane(c);
     };
     // Retiring: a wave asked to claim more work near the launch's end (its last
-    // claim at retire_from or later) while one of its rays is beyond
-    // retire_steps crossings stops claiming, so that it reaches the drain below
-    // (over four times faster per crossing) while the other waves trace the
-    // rest.  At most retire_most waves of the launch do (asked once per wave,
-    // counted in claim word 16): the others remain to claim what is left.
-    uint32_t last_c = 0;
-    bool may_retire = P.retire_most > 0u;
+    // claim at retire_from or later) while one of its rays is beyond ask_at
+    // crossings stops claiming, so that it reaches the drain below (over four
+    // times faster per crossing) while the other waves trace the rest.  At most
+    // retire_most waves of the launch do for rays beyond retire_steps (counted
+    // in claim word 16), as many beyond four times that for the waves that were
+    // refused (word 17), and so on up to word 19: the longest rays are not left
+    // out, and the other waves remain to claim what is left.
+    uint32_t last_c = 0, asked = 0;
+    int ask_at = P.retire_most > 0u ? P.retire_steps : 0x7FFFFFFF;
     auto retire = [&]() -> bool {
-        if (!may_retire || last_c < P.retire_from || !__ballot(alive && rsteps > P.retire_steps)) return false;
-        may_retire = false;
+        if (last_c < P.retire_from || !__ballot(alive && cnt > ask_at)) return false;
         uint32_t k = 0;
-        if (lane == 0) k = atomicAdd(P.claim + 16, 1u);
+        if (lane == 0) k = atomicAdd(P.claim + 16u + asked, 1u);
+        ++asked;
+        ask_at = asked < 4u ? 4 * ask_at : 0x7FFFFFFF;
         return __builtin_amdgcn_readfirstlane(k) < P.retire_most;
     };
-    // kappa and Ib of a ray's (band, g) rows at a field value
+    // kappa and Ib of a ray's (band, g) rows at a field value (sliced tables:
+    // rows by LDS word, the value is the table coordinate within the
+    // slice, below its last node)
+    auto table_nodes = [&](float T, int kr, int ir, float& k0, float& k1, float& i0, float& i1) -> float {
+        if (TAB == kTabSliced) {
+            const int w = (int)T;
+            lfloat* kp = (lfloat*)(uintptr_t)((uint32_t)(kr + w) << 2);
+            lfloat* ip = (lfloat*)(uintptr_t)((uint32_t)(ir + w) << 2);
+            k0 = kp[0];
+            k1 = kp[1];
+            i0 = ip[0];
+            i1 = ip[1];
+            return __builtin_amdgcn_fractf(T);
+        }
+        float pos = fmaf(T, P.inv_dT, P.mT0);
+        pos = fminf(fmaxf(pos, 0.0f), (float)(nT - 1));
+        int w = (int)pos;
+        w = w > nT - 2 ? nT - 2 : w;
+        k0 = kq[kr + w];
+        k1 = kq[kr + w + 1];
+        i0 = ibt[ir + w];
+        i1 = ibt[ir + w + 1];
+        return pos - (float)w;
+    };
     auto table_at = [&](float T, int kr, int ir, float& kap, float& ibj) {
         if (SPEC == kSpecGreyT4) {
             const float t2 = T * T;
@@ -1064,45 +1114,31 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
             ibj = t2 * t2;
             return;
         }
-        int w;
-        float fr;
-        if (TAB == kTabSliced) {
-            w = (int)T;
-            w = w > nw - 2 ? nw - 2 : w;
-            fr = T - (float)w;
-        } else {
-            float pos = fmaf(T, P.inv_dT, P.mT0);
-            pos = fminf(fmaxf(pos, 0.0f), (float)(nT - 1));
-            w = (int)pos;
-            w = w > nT - 2 ? nT - 2 : w;
-            fr = pos - (float)w;
-        }
-        const float k0 = TAB == kTabSliced ? s_kq[kr + w] : kq[kr + w];
-        const float k1 = TAB == kTabSliced ? s_kq[kr + w + 1] : kq[kr + w + 1];
-        const float i0 = ibt[ir + w], i1 = ibt[ir + w + 1];
+        float k0, k1, i0, i1;
+        const float fr = table_nodes(T, kr, ir, k0, k1, i0, i1);
         kap = fmaf(fr, k1 - k0, k0);
         ibj = fmaf(fr, i1 - i0, i0);
     };
     // adaptive mesh coarsening (code/mc_gpu.cu:193-207): the lane's ray goes on
     // in the next coarser level
     auto coarser = [&]() {
+        const int* F = s_lev + lev * kLevWords;
+        const int* L = F + kLevWords;
         ++lev;
-        const int* L = s_lev + lev * kLevWords;
-        n0 = L[0]; n1 = L[1]; n2 = L[2];
-        fo0 = L[3]; fo1 = L[4]; fo2 = L[5]; maxs = L[6];
-        oo0 = L[11]; oo1 = L[12]; oo2 = L[13];
+        maxs = L[6];
         Tl = lev_T(L);
         if (GEN) Tl += (size_t)rsnap * (uint32_t)L[14];
-        // ic = (ic + r - 1) / r with r = 2: every level halves each axis
-        // (level g has n >> g cells)
-        cx = (cx + 1) >> 1;
-        cy = (cy + 1) >> 1;
-        cz = (cz + 1) >> 1;
-        fx = face_at(fo0, cx - (fl & 1));
-        fy = face_at(fo1, cy - ((fl >> 1) & 1));
-        fz = face_at(fo2, cz - ((fl >> 2) & 1));
-        idx = off_at(oo0, cx) + off_at(oo1, cy) + off_at(oo2, cz);
-        Tc = load_T(Tl, idx);
+        // ic = (ic + r - 1) / r with r = 2 (0-based: half): every level halves
+        // each axis (level g has n >> g cells)
+        auto down = [&](int a, int& A, int& K, int s, float& f) {
+            A = L[3 + a] + ((cell_of(F, a, A, s) >> 1) << 2) + (s > 0 ? 4 : 0);
+            K = L[11 + a] + (s > 0 ? -4 : 0);
+            f = lds_f(A);
+        };
+        down(0, A0, K0, s0, fx);
+        down(1, A1, K1, s1, fy);
+        down(2, A2, K2, s2, fz);
+        Tc = load_T(Tl, lds_i(A0 + K0) + lds_i(A1 + K1) + lds_i(A2 + K2));
         cnt = 0;
     };
 
@@ -1119,6 +1155,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
             // ---- tally the rays finished since the last refill
             if (!QUEUE && TMODE == 0) flush_wave(P, fin && rslot != aslot && aslot >= 0, aslot, aE, aA, aQ, lane);
             if (fin) {
+                rsteps = s_lev[lev * kLevWords + 15] + cnt;   // (each finer level took its maxs)
                 if (QUEUE)
                     ring_tally(rw * Dfin, rwi * G);
                 else
@@ -1143,38 +1180,40 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
                 if (GEN) T0 = lev_T(s_lev) + (size_t)rsnap * (uint32_t)s_lev[14];
                 Tc = rd.Tc;
                 band = rd.bg & 0xFFFF;
-                fl = (rd.bg >> 24) & 7;
+                const int fl = rd.bg >> 24;
                 sx = rd.sx; sy = rd.sy; sz = rd.sz;
                 ix = rd.ix; iy = rd.iy; iz = rd.iz;
                 rw = rd.rw;
                 rwi = rd.rwi;
                 const int g = (rd.bg >> 16) & 0xFF;
-                cx = (rd.cell & 1023) + 1;
-                cy = ((rd.cell >> 10) & 1023) + 1;
-                cz = ((rd.cell >> 20) & 1023) + 1;
                 px = rd.px;
                 py = rd.py;
                 pz = rd.pz;
                 pslot = rd.ps;
-                if (AMC && lev != 0) {
+                if (AMC) {
                     lev = 0;
-                    n0 = s_lev[0]; n1 = s_lev[1]; n2 = s_lev[2];
-                    fo0 = s_lev[3]; fo1 = s_lev[4]; fo2 = s_lev[5]; maxs = s_lev[6];
-                    oo0 = s_lev[11]; oo1 = s_lev[12]; oo2 = s_lev[13];
+                    maxs = s_lev[6];
                 }
                 Tl = T0;
-                fx = face_at(fo0, cx - (fl & 1));
-                fy = face_at(fo1, cy - ((fl >> 1) & 1));
-                fz = face_at(fo2, cz - ((fl >> 2) & 1));
-                idx = rd.idx;
+                s0 = fl & 1 ? -4 : 4;
+                s1 = fl & 2 ? -4 : 4;
+                s2 = fl & 4 ? -4 : 4;
+                A0 = f00 + ((rd.cell & 1023) << 2) + (fl & 1 ? 0 : 4);
+                A1 = f01 + (((rd.cell >> 10) & 1023) << 2) + (fl & 2 ? 0 : 4);
+                A2 = f02 + (((rd.cell >> 20) & 1023) << 2) + (fl & 4 ? 0 : 4);
+                K0 = k00 + (fl & 1 ? 0 : -4);
+                K1 = k01 + (fl & 2 ? 0 : -4);
+                K2 = k02 + (fl & 4 ? 0 : -4);
+                fx = lds_f(A0);
+                fy = lds_f(A1);
+                fz = lds_f(A2);
                 tau = 0.0f;
                 tra = 1.0f;
                 G = 0.0f;
-                krow = (band * P.nQ + g) * rowlen;
-                ibrow = band * rowlen;
+                krow = kr0 + (band * P.nQ + g) * rowlen;
+                ibrow = ir0 + band * rowlen;
                 cnt = 0;
                 hash = 2166136261u;
-                rsteps = 0;
                 alive = true;
             };
             if (QUEUE) {
@@ -1395,112 +1434,100 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         }
         if (!alive) continue;
 
-        // ---------------------------------------------------- one crossing
-        float k0 = 0.f, k1 = 0.f, i0 = 0.f, i1 = 0.f, fr = 0.f;
-        if (SPEC == kSpecTable) {
-            if (TAB == kTabSliced) {
-                // Tc is the cell's table coordinate within the slice (t_to_u):
-                // node w of the slice and the lerp fraction
-                int w = (int)Tc;
-                w = w > nw - 2 ? nw - 2 : w;
-                fr = Tc - (float)w;
-                k0 = s_kq[krow + w];
-                k1 = s_kq[krow + w + 1];
-                i0 = s_ib[ibrow + w];
-                i1 = s_ib[ibrow + w + 1];
-            } else {
-                float pos = fmaf(Tc, P.inv_dT, P.mT0);
-                pos = fminf(fmaxf(pos, 0.0f), (float)(nT - 1));
-                int t0 = (int)pos;
-                t0 = t0 > nT - 2 ? nT - 2 : t0;
-                fr = pos - (float)t0;
-                k0 = kq[krow + t0];
-                k1 = kq[krow + t0 + 1];
-                i0 = ibt[ibrow + t0];
-                i1 = ibt[ibrow + t0 + 1];
+        // ------------------------------------------------ kAhead crossings
+        constexpr int kAhead = AMC ? kAheadLev : kAheadFine;
+        float dsv[kAhead], Tv[kAhead];
+        int lin[kAhead];
+        const int lim = AMC ? min(kAhead, maxs - cnt) : kAhead;
+        int wall = -1, wall_u = kAhead;         // the crossing that hits a wall
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            dsv[u] = Tv[u] = 0.0f;
+            lin[u] = 0;
+            if (AMC && u >= lim) continue;
+            if (REC) {
+                const int* L = s_lev + lev * kLevWords;
+                lin[u] = cell_of(L, 0, A0, s0) + L[0] * (cell_of(L, 1, A1, s1) + L[1] * cell_of(L, 2, A2, s2));
             }
-        }
-        if (REC) {
-            const int lin = (cx - 1) + n0 * ((cy - 1) + n1 * (cz - 1));
-            hash = (hash ^ (((uint32_t)lev << 28) ^ (uint32_t)lin)) * 16777619u;
-        }
-        const float d0 = (fx - px) * ix;
-        const float d1 = (fy - py) * iy;
-        const float d2 = (fz - pz) * iz;
-        float ds = d0;
-        ds = (ds > d1) ? d1 : ds;
-        ds = (ds > d2) ? d2 : ds;
-        px = (ds == d0) ? fx : fmaf(ds, sx, px);
-        py = (ds == d1) ? fy : fmaf(ds, sy, py);
-        pz = (ds == d2) ? fz : fmaf(ds, sz, pz);
-        const int ax = (d0 < d1) ? ((d0 < d2) ? 0 : 2) : ((d1 < d2) ? 1 : 2);
-        const bool m0 = ax == 0, m1 = ax == 1, m2 = ax == 2;
-        const int fla = (fl >> ax) & 1;
-        const int stp = fla ? -1 : 1;
-        int cm = (m0 ? cx : (m1 ? cy : cz)) + stp;
-        const int nm = m0 ? n0 : (m1 ? n1 : n2);
-        const int fo = m0 ? fo0 : (m1 ? fo1 : fo2);
-        // the domain boundary (cm = 0 or nm + 1): a periodic wrap, or a wall
-        // hit that keeps the old cell (the ray ends there).  Rare per lane, so
-        // a branch: most steps of a wave have no lane at the boundary.
-        int wall = -1;
-        if ((uint32_t)(cm - 1) >= (uint32_t)nm) {
-            const int side = cm != 0;
-            const int bcbit = ax * 2 + side;
-            if ((P.bc_periodic >> bcbit) & 1) {
-                const float pw = face_at(fo, side ? 0 : nm);
-                cm = side ? 1 : nm;
-                px = m0 ? pw : px;
-                py = m1 ? pw : py;
-                pz = m2 ? pw : pz;
-            } else {
-                wall = bcbit;
-                cm -= stp;
+            const float d0 = (fx - px) * ix;
+            const float d1 = (fy - py) * iy;
+            const float d2 = (fz - pz) * iz;
+            const float ds = min3(d0, d1, d2);
+            dsv[u] = ds;
+            const bool e0 = ds == d0, e1 = ds == d1, m2 = ds == d2;
+            px = e0 ? fx : fmaf(ds, sx, px);
+            py = e1 ? fy : fmaf(ds, sy, py);
+            pz = m2 ? fz : fmaf(ds, sz, pz);
+            // of several axes at the same distance the last one moves
+            const bool m1 = e1 && !m2, m0 = e0 && !e1 && !m2;
+            A0 += m0 ? s0 : 0;
+            A1 += m1 ? s1 : 0;
+            A2 += m2 ? s2 : 0;
+            float fnew = lds_f(m2 ? A2 : (m1 ? A1 : A0));
+            // (read with the face: one LDS latency before the field load; a ray that
+            // left the domain reads its neighbours' words here and its own below)
+            int o0 = lds_i(A0 + K0), o1 = lds_i(A1 + K1), o2 = lds_i(A2 + K2);
+            asm volatile("" : "+v"(fnew), "+v"(o0), "+v"(o1), "+v"(o2));   // (here, not sunk past the branch)
+            // past the domain's last face: a periodic wrap, or a wall hit that keeps
+            // the old cell (the ray ends there).  Rare per lane, so a branch.
+            if (fnew > kFaceEnd * 0.5f) {
+                const int ax = m2 ? 2 : (m1 ? 1 : 0);
+                const int sa = m2 ? s2 : (m1 ? s1 : s0);
+                const int side = sa > 0 ? 1 : 0;
+                const int bcbit = ax * 2 + side;
+                const int* L = s_lev + lev * kLevWords + ax;
+                const int fo = L[3], last = fo + (L[0] << 2);     // face 0, face n
+                int An = (m2 ? A2 : (m1 ? A1 : A0)) - sa;
+                if ((P.bc_periodic >> bcbit) & 1) {
+                    const float pw = lds_f(side ? fo : last);
+                    An = side ? fo + 4 : last - 4;
+                    px = m0 ? pw : px;
+                    py = m1 ? pw : py;
+                    pz = m2 ? pw : pz;
+                } else if (wall < 0) {
+                    wall = bcbit;
+                    wall_u = u;
+                }
+                A0 = m0 ? An : A0;
+                A1 = m1 ? An : A1;
+                A2 = m2 ? An : A2;
+                fnew = lds_f(An);
+                o0 = lds_i(A0 + K0);
+                o1 = lds_i(A1 + K1);
+                o2 = lds_i(A2 + K2);
             }
+            fx = m0 ? fnew : fx;
+            fy = m1 ? fnew : fy;
+            fz = m2 ? fnew : fz;
+            Tv[u] = load_T(Tl, o0 + o1 + o2);
         }
-        const float fnew = face_at(fo, cm - fla);
-        cx = m0 ? cm : cx;
-        cy = m1 ? cm : cy;
-        cz = m2 ? cm : cz;
-        fx = m0 ? fnew : fx;
-        fy = m1 ? fnew : fy;
-        fz = m2 ? fnew : fz;
-        idx = off_at(oo0, cx) + off_at(oo1, cy) + off_at(oo2, cz);
-        const float Tn = load_T(Tl, idx);
-        float kap, ibj;
-        if (SPEC == kSpecGreyT4) {
-            const float t2 = Tc * Tc;
-            kap = P.kappa_grey;
-            ibj = t2 * t2;
-        } else {
-            kap = fmaf(fr, k1 - k0, k0);
-            ibj = fmaf(fr, i1 - i0, i0);
-        }
-        ++cnt;
-        ++rsteps;
-        Tc = Tn;   // (read on every path, so the load is issued here, not sunk)
         // transport, branch-free on the common path: past the cut-off the
         // remaining energy is deposited here (tra), else the segment absorbs
         // tra - tra1; a wall absorbs what is left; the step cap ends the ray
         // (or moves it to the next coarser level)
-        const float tau1 = fmaf(kap, ds, tau);
-        const bool cut = tau1 >= P.tau_cut;
-        const float tra1 = __expf(-tau1);
-        G = fmaf(cut ? tra : tra - tra1, ibj, G);
-        tau = tau1;
-        tra = cut ? tra : tra1;
-        const bool hitw = !cut && wall >= 0;
-        if (hitw) G = fmaf(tra, s_ibw[wall * P.nB + band], G);
-        const bool cap = !cut && !hitw && cnt >= maxs;
-        if (cut || hitw) {
-            alive = false; fin = true; endt = cut ? 0 : 1; Dfin = 1.0f;
-        } else if (cap) {
-            if (AMC && lev + 1 < P.nlev) {
-                coarser();
-            } else {
-                alive = false; fin = true; endt = 2; Dfin = 1.0f - tra;
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (!alive || (AMC && u >= lim)) continue;
+            float kap, ibj;
+            table_at(Tc, krow, ibrow, kap, ibj);
+            if (REC) hash = (hash ^ (((uint32_t)lev << 28) ^ (uint32_t)lin[u])) * 16777619u;
+            ++cnt;
+            Tc = Tv[u];
+            tau = fmaf(kap, dsv[u], tau);
+            const bool cut = tau >= P.tau_cut, hit = u == wall_u;
+            const float tra1 = __expf(-tau);
+            G = fmaf(cut ? tra : tra - tra1, ibj, G);
+            tra = tra1;   // (not used after a cut-off)
+            if (cut || hit || cnt >= maxs) {
+                if (cut || hit) {
+                    if (!cut) G = fmaf(tra, s_ibw[wall * P.nB + band], G);
+                    alive = false; fin = true; endt = cut ? 0 : 1; Dfin = 1.0f;
+                } else if (!AMC || lev + 1 >= P.nlev) {
+                    alive = false; fin = true; endt = 2; Dfin = 1.0f - tra;
+                }
             }
         }
+        if (AMC && alive && cnt >= maxs) coarser();
     }
     // ---- drain: nothing is left to hand out and at most 16 of the wave's rays
     // run on, on the last level.  Such a ray is a serial chain (along the walls
@@ -1534,34 +1561,34 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         // (lane 3 is never the nearest face: distance 3e38)
         float qp = axis_f(px, py, pz, 0.0f), qs = axis_f(sx, sy, sz, 0.0f), qi = axis_f(ix, iy, iz, 1.0f);
         float qf = axis_f(fx, fy, fz, 3.0e38f);
+        const bool neg = axis_f(sx, sy, sz, 1.0f) < 0.0f;
+        const int* L = s_lev + (P.nlev - 1) * kLevWords; // the last level
         int qc;                                          // 0-based cell
         {
-            const int vx = __shfl(cx, src), vy = __shfl(cy, src), vz = __shfl(cz, src);
+            const int vx = __shfl(A0, src), vy = __shfl(A1, src), vz = __shfl(A2, src);
             // (a quad without a ray stays frozen in cell 0: lane 0's last ray may
             // have ended on a finer level, whose cells this level does not have)
-            qc = !run ? 0 : (a == 0 ? vx - 1 : (a == 1 ? vy - 1 : (a == 2 ? vz - 1 : 0)));
+            qc = !run || ax3 ? 0 : cell_of(L, a, a == 0 ? vx : (a == 1 ? vy : vz), neg ? -4 : 4);
         }
-        const bool neg = (__shfl(fl, src) >> a) & 1;     // (fl has 3 bits)
         const int st = neg ? -1 : 1;
         float qtau = __shfl(tau, src), qtra = __shfl(tra, src), qG = __shfl(G, src);
         const int qkrow = __shfl(krow, src), qibrow = __shfl(ibrow, src), qband = __shfl(band, src);
-        int qcnt = __shfl(cnt, src), qsteps = __shfl(rsteps, src), qend = 0;
+        int qcnt = __shfl(cnt, src), qend = 0;
         float qD = 1.0f;
         uint32_t qhash = REC ? (uint32_t)__shfl((int)hash, src) : 0u;
         const int bcbit = 2 * a + (neg ? 0 : 1);         // the boundary this axis runs into
         const bool per = (P.bc_periodic >> bcbit) & 1;
-        // the last level: cells along this axis, LDS bytes of the face behind the
-        // exit face of cell 0 and of its brick offset
-        const int* L = s_lev + (P.nlev - 1) * kLevWords;
+        // cells along this axis, LDS bytes of the face behind the exit face of
+        // cell 0 and of its brick offset
         const int qn = ax3 ? 0x7FFFFFFF : L[a], qmaxs = L[6];
-        const int gb = L[3 + (ax3 ? 0 : a)] + (neg ? -4 : 8), ob = L[11 + (ax3 ? 0 : a)] + 4;
+        const int gb = L[3 + (ax3 ? 0 : a)] + (neg ? -4 : 8), ob = L[3 + (ax3 ? 0 : a)] + L[11 + (ax3 ? 0 : a)];
         const int qstride = a == 0 ? 1 : (a == 1 ? L[0] : (a == 2 ? L[0] * L[1] : 0));
         gfloat* qT = lev_T(L);
         if (GEN) qT += (size_t)(uint32_t)__shfl((int)rsnap, src) * (uint32_t)L[14];
         // face i behind (+) or before (-) the exit face of cell c: word c + i st of
         // the face table from gb - st (a word past the axis's faces is one of its
         // LDS neighbours and is not used)
-        auto face_w = [&](int byte, int i) -> float { return *(const float*)((const char*)s_face + byte + (i << 2)); };
+        auto face_w = [&](int byte, int i) -> float { return lds_f(byte + (i << 2)); };
         while (__ballot(run)) {
             int lim = run ? min(kDrain, qmaxs - qcnt) : 0;
             int wall = -1;
@@ -1581,7 +1608,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     const int u = 4 * k + j;
-                    ov[j] = off_at(ob, qc);
+                    ov[j] = lds_i(ob + (qc << 2));
                     const float d = (qf - qp) * qi;
                     const float ds = quad_min(d);
                     dsv[u] = ds;
@@ -1689,7 +1716,6 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
             }
             qtra = before;   // (not used after a cut-off)
             qcnt += taken;
-            qsteps += taken;
             const bool hitw = run && !cutq && wall >= 0;
             if (hitw) qG = fmaf(qtra, s_ibw[wall * P.nB + qband], qG);
             if (run && (cutq || hitw)) {
@@ -1706,12 +1732,12 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         // back to the lanes that held the rays
         const int from = alive ? 4 * rank : lane;
         const float rG = __shfl(qG, from), rD = __shfl(qD, from);
-        const int rsn = __shfl(qsteps, from), ren = __shfl(qend, from);
+        const int rcn = __shfl(qcnt, from), ren = __shfl(qend, from);
         const uint32_t rh = REC ? (uint32_t)__shfl((int)qhash, from) : 0u;
         if (alive) {
             G = rG;
             Dfin = rD;
-            rsteps = rsn;
+            cnt = rcn;
             endt = ren;
             if (REC) hash = rh;
             alive = false;
@@ -1722,6 +1748,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     // a ray that ended after the last refill (nothing was left to hand out)
     if (!QUEUE && TMODE == 0) flush_wave(P, fin && rslot != aslot && aslot >= 0, aslot, aE, aA, aQ, lane);
     if (fin) {
+        rsteps = s_lev[lev * kLevWords + 15] + cnt;
         if (QUEUE)
             ring_tally(rw * Dfin, rwi * G);
         else
@@ -1860,8 +1887,8 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
                     const int lin = (c[0] - 1) + n[0] * ((c[1] - 1) + n[1] * (c[2] - 1));
                     hash = (hash ^ (((uint32_t)lev << 28) ^ (uint32_t)lin)) * 16777619u;
                 }
-                const int idx = s_off[oo[0] + c[0] - 1] + s_off[oo[1] + c[1] - 1] + s_off[oo[2] + c[2] - 1];
-                const double Tj = (double)T[idx];
+                const uint32_t off = (uint32_t)(s_off[oo[0] + c[0] - 1] + s_off[oo[1] + c[1] - 1] + s_off[oo[2] + c[2] - 1]);
+                const double Tj = (double)*(const float*)((const char*)T + off);
                 double kap, ibj;
                 if (SPEC == kSpecGreyT4) {
                     kap = (double)P.kappa_grey;

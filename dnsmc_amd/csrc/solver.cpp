@@ -190,7 +190,7 @@ struct dnsmc_solver {
     long long tstride[kMaxLev] = {0, 0, 0, 0, 0, 0};   // bricked floats per level and snapshot
     int nbx[kMaxLev] = {0, 0, 0, 0, 0, 0}, nby[kMaxLev] = {0, 0, 0, 0, 0, 0};
     std::vector<float> faces_packed, centres_packed;
-    std::vector<int> offs_packed;   // brick-layout offset of each cell index, per level and axis
+    std::vector<int> offs_packed;   // brick-layout byte offset of each cell index, per level and axis
     int foff[kMaxLev][3], coff[3], ooff[kMaxLev][3];
     DevBuf<int> d_offs;
     DevBuf<float> d_faces, d_centres;
@@ -341,11 +341,14 @@ static EventPair& next_event(dnsmc_solver* s, int kind)
 static int upload_geometry(dnsmc_solver* s)
 {
     if (s->geom_uploaded) return DNSMC_OK;
-    s->faces_packed.clear();
+    // the traversal recognises a ray that left the domain by the word before or
+    // after the axis's faces
+    s->faces_packed.assign(1, kFaceEnd);
     for (size_t l = 0; l < s->lev.size(); ++l)
         for (int a = 0; a < 3; ++a) {
             s->foff[l][a] = (int)s->faces_packed.size();
             s->faces_packed.insert(s->faces_packed.end(), s->lev[l].faces[a].begin(), s->lev[l].faces[a].end());
+            s->faces_packed.push_back(kFaceEnd);
         }
     s->centres_packed.clear();
     for (int a = 0; a < 3; ++a) {
@@ -370,7 +373,7 @@ static int upload_geometry(dnsmc_solver* s)
             s->ooff[l][a] = (int)s->offs_packed.size();
             for (int c = 0; c < n[a]; ++c) {
                 const int x = a == 0 ? c : 0, y = a == 1 ? c : 0, z = a == 2 ? c : 0;
-                s->offs_packed.push_back(brick_index(x, y, z, s->nbx[l], s->nby[l]));
+                s->offs_packed.push_back((int)(4u * (uint32_t)brick_index(x, y, z, s->nbx[l], s->nby[l])));
             }
         }
     }
@@ -990,7 +993,9 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
         const size_t sliced = lds_trace + sizeof(float) * (size_t)d.nB * (d.nQ + 1) * nw;
         const char* force = getenv("DNSMC_TABLES");   // "global": keep the tables out of LDS
         const bool allow = !(force && !strcmp(force, "global"));
-        if (allow && sliced <= s->lds_max) {
+        // (the sliced lookup takes coordinates below the table's last node)
+        const bool below_top = fmaf(thi, d.inv_dT, d.mT0) < (float)(d.nT - 1);
+        if (allow && below_top && sliced <= s->lds_max) {
             tab = kTabSliced;
             P.tab_lo = lo;
             P.tab_nw = nw;
