@@ -36,6 +36,8 @@ __host__ __device__ inline MlpLayout mlp_layout(int nbin)
     return L;
 }
 
+constexpr int kMlpSmall = (kMlpIn + 1) * kMlpHid + (kMlpHid + 1) * kMlpHid;   // parameters before W3 (a multiple of 64)
+
 struct MlpWeights {
     const uint16_t* W1;   // [6][64] bf16
     const float* b1;      // [64]
@@ -68,8 +70,15 @@ struct MlpTrainArgs {
     int n;
     const float* wsum;    // device scalar: sum of wt over the n samples
     MlpWeights w;
-    float* part;          // [gridDim.x][P] per-block gradient partials
-    float* loss_part;     // [gridDim.x]
+    const uint16_t* W3T;  // [noutp][64] bf16 (mlp_train_prep)
+    // per 64-row block b of the minibatch (rows past n are zero)
+    uint16_t* H2;         // [64 b + row][64] bf16
+    uint16_t* H2T;        // [b][64 h][64 row] bf16
+    float* lse;           // [64 b + row][2] log-sum-exp of the direction and (band, g) logits
+    float* sw;            // [64 b + row] wt / wsum
+    float* part;          // [b][kMlpSmall] gradient of the parameters below W3
+    float* loss_part;     // [b]
+    float* part3;         // [split][64 noutp + noutp] gradient of W3 and b3
 };
 
 // Per-cell features of the proposal (shared by ray generation and training).

@@ -83,9 +83,8 @@ __device__ __forceinline__ void acc_each(const f4v acc[2][2], F f)
             for (int i = 0; i < 4; ++i) f(qr + 16 * ti + 4 * (lane >> 4) + i, qc + 16 * tj + (lane & 15), acc[ti][tj][i]);
 }
 
-// H1 = tanh(X W1 + b1) for rows < nrow (zero rows after), as FP32 and BF16.
-__device__ __forceinline__ void layer1(const float* sX, const MlpWeights& w, int nrow, float* H1f, uint16_t* H1b,
-                                       int hs = kMlpHid)
+// H1 = tanh(X W1 + b1) for rows < nrow (zero rows after), BF16.
+__device__ __forceinline__ void layer1(const float* sX, const MlpWeights& w, int nrow, uint16_t* H1b, int hs = kMlpHid)
 {
     for (int e = threadIdx.x; e < 64 * kMlpHid; e += blockDim.x) {
         const int s = e / kMlpHid, j = e - s * kMlpHid;
@@ -95,20 +94,7 @@ __device__ __forceinline__ void layer1(const float* sX, const MlpWeights& w, int
             for (int i = 0; i < kMlpIn; ++i) acc = fmaf(sX[s * kMlpIn + i], bf2f(w.W1[i * kMlpHid + j]), acc);
             h = tanhf(acc);
         }
-        if (H1f) H1f[e] = h;
         H1b[s * hs + j] = f2bf(h);
-    }
-}
-
-// Stage column tile jt of W3 ([64][noutp] BF16, row-major) into dst[64][64]:
-// 64 rows of 128 contiguous bytes, 16 B per load.
-__device__ __forceinline__ void stage_w3_tile(const uint16_t* W3, int noutp, int jt, uint16_t* dst)
-{
-    const uint4* src = (const uint4*)W3;
-    uint4* d = (uint4*)dst;
-    for (int e = threadIdx.x; e < 512; e += blockDim.x) {
-        const int h = e >> 3, c8 = e & 7;
-        d[e] = src[((size_t)h * noutp + jt * 64) / 8 + c8];
     }
 }
 
@@ -145,223 +131,562 @@ __device__ __forceinline__ void put_w3_tile(const uint4& r0, const uint4& r1, ui
 }
 
 // ------------------------------------------------------------- training ----
-// One block per 64 samples: forward, weighted cross-entropy of both heads,
-// backward; the block's gradient of (sum_s wt_s CE_s) / sum wt goes to its row
-// of `part`.  LDS (dynamic): see the carve-up below (about 91 KB).
-__global__ __launch_bounds__(256) void mlp_train_tile(MlpTrainArgs a)
-{
-    extern __shared__ float lds[];
-    float* sX = lds;                                  // 64*6
-    float* sH1f = sX + 64 * kMlpIn;                   // 64*64
-    float* sH2f = sH1f + 4096;                        // 64*64 (later dA1)
-    float* sZ = sH2f + 4096;                          // 64*64 logits / dZ / dA2
-    float* sw = sZ + 4096;                            // 64 sample scale
-    float* sm_d = sw + 64;                            // log-sum-exp per row, direction head
-    float* sm_b = sm_d + 64;                          // log-sum-exp per row, (band, g) head
-    float* sloss = sm_b + 64;                         // 64
-    int* std_ = (int*)(sloss + 64);                   // 64
-    int* stb_ = std_ + 64;                            // 64
-    uint16_t* sH1b = (uint16_t*)(stb_ + 64);          // 64*64
-    uint16_t* sH2b = sH1b + 4096;
-    uint16_t* sW2b = sH2b + 4096;
-    uint16_t* sW3b = sW2b + 4096;
-    uint16_t* sdZb = sW3b + 4096;
+// One gradient evaluation, four launches over 64-row blocks of the minibatch:
+//   mlp_train_prep  the sum of the sample weights; W3 with the input index
+//                   contiguous (the logits' operand layout),
+//   mlp_train_rows  per 64 rows (16 per wave): forward, log-sum-exp of both
+//                   heads, dH2 and the gradients below W3; H2 and the rows'
+//                   log-sum-exps to memory,
+//   mlp_train_w3    per 64 columns of W3 and split of the rows: the logits and
+//                   dZ again, dW3 and db3 summed over the split in registers,
+//   mlp_reduce      the partial sums.
+// The first form wrote every 64-row block's whole gradient (451 KB) and summed
+// 256 of them: 115 MB each way, 0.42 ms per step of 16384 rows (320 us of tile
+// kernel at one block per CU, 79 us of reduction, 19 us of weight sum).  Here
+// W3's part (96 % of the parameters) is kept in registers over the rows of a
+// split: 0.14 ms for the same step (462 -> 142 us with the update; kernels 75 us
+// for the rows, two blocks per CU, bound by the exponentials and LDS reads of
+// the two passes over W3's columns, 27 us for dW3, 11 us for the sums).  Every
+// sum over rows, columns and blocks below W3 keeps the first form's order, so
+// those gradients are bit for bit what they were.  dZ leaves the logits' accumulators in the layout of the
+// next product's second operand (rows 4 (l / 16) + i, column l % 16), so
+// dW3 = H2^T dZ takes it from registers.
 
-    const MlpLayout L = mlp_layout(a.w.nbin);
-    const int noutp = a.w.noutp, nbin = a.w.nbin;
+// Four BF16 of consecutive k as an MFMA operand, from an 8-byte aligned address.
+__device__ __forceinline__ s4v frag8(const uint16_t* p)
+{
+    const uint2 u = *(const uint2*)p;
+    s4v v;
+    v.x = (short)(u.x & 0xFFFFu);
+    v.y = (short)(u.x >> 16);
+    v.z = (short)(u.y & 0xFFFFu);
+    v.w = (short)(u.y >> 16);
+    return v;
+}
+// Four FP32 as BF16, round to nearest even (v_cvt_pk_bf16_f32).
+typedef float f2v __attribute__((ext_vector_type(2)));
+typedef __bf16 b2v __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ s4v pack4(float a, float b, float c, float d)
+{
+    const uint32_t lo = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2v{a, b}, b2v));
+    const uint32_t hi = __builtin_bit_cast(uint32_t, __builtin_convertvector(f2v{c, d}, b2v));
+    s4v v;
+    v.x = (short)(lo & 0xFFFFu);
+    v.y = (short)(lo >> 16);
+    v.z = (short)(hi & 0xFFFFu);
+    v.w = (short)(hi >> 16);
+    return v;
+}
+__device__ __forceinline__ void put8(uint16_t* p, s4v v)
+{
+    *(uint2*)p = make_uint2((uint32_t)(uint16_t)v.x | ((uint32_t)(uint16_t)v.y << 16),
+                            (uint32_t)(uint16_t)v.z | ((uint32_t)(uint16_t)v.w << 16));
+}
+#define DN_MFMA(a, b, c) __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0)
+
+// dZ = w (softmax - onehot) of a logit z, its head's log-sum-exp and whether
+// its column is the sample's bin.
+__device__ __forceinline__ float mlp_dz(float z, float w, float lse, bool hot)
+{
+    return w * (__expf(z - lse) - (hot ? 1.f : 0.f));
+}
+
+// Block 0: wsum = sum of wt (per thread in steps of 256, eight loads in flight,
+// then a tree).  Block 1 + jt: rows 64 jt .. 64 jt + 63 of W3T[noutp][64].
+__global__ __launch_bounds__(256) void mlp_train_prep(const float* wt, long long n, float* wsum, const uint16_t* W3,
+                                                      int noutp, uint16_t* W3T)
+{
+    __shared__ float s[256];
+    __shared__ uint16_t t[64 * kPropStride];
     const int tid = threadIdx.x;
+    if (blockIdx.x == 0) {
+        float v = 0.f;
+        long long i = tid;
+        for (; i + 7 * 256 < n; i += 8 * 256) {
+            float x[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) x[u] = wt[i + u * 256];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v += x[u];
+        }
+        for (; i < n; i += 256) v += wt[i];
+        s[tid] = v;
+        __syncthreads();
+        for (int o = 128; o > 0; o >>= 1) {
+            if (tid < o) s[tid] += s[tid + o];
+            __syncthreads();
+        }
+        if (tid == 0) *wsum = s[0] > 0.f ? s[0] : 1.f;
+        return;
+    }
+    const int jt = blockIdx.x - 1;
+    for (int e = tid; e < 512; e += 256) {
+        const int h = e >> 3, c8 = e & 7;
+        const uint4 r = ((const uint4*)W3)[((size_t)h * noutp + jt * 64) / 8 + c8];
+        uint2* d = (uint2*)(t + h * kPropStride + c8 * 8);
+        d[0] = make_uint2(r.x, r.y);
+        d[1] = make_uint2(r.z, r.w);
+    }
+    __syncthreads();
+    for (int e = tid; e < 1024; e += 256) {
+        const int c = e >> 4, h = (e & 15) * 4;
+        s4v v;
+        v.x = (short)t[h * kPropStride + c];
+        v.y = (short)t[(h + 1) * kPropStride + c];
+        v.z = (short)t[(h + 2) * kPropStride + c];
+        v.w = (short)t[(h + 3) * kPropStride + c];
+        put8(W3T + ((size_t)jt * 64 + c) * 64 + h, v);
+    }
+}
+
+// Tile jt of row-major W3 (64 rows h, columns 64 jt .. + 63) in two steps, as
+// load_w3_tile / put_w3_tile take W3T's.
+__device__ __forceinline__ void load_w3_cols(const uint16_t* W3, int noutp, int jt, uint4& r0, uint4& r1)
+{
+    const uint4* src = (const uint4*)W3;
+    const int e = threadIdx.x;
+    r0 = src[((size_t)(e >> 3) * noutp + jt * 64) / 8 + (e & 7)];
+    r1 = src[((size_t)((e >> 3) + 32) * noutp + jt * 64) / 8 + (e & 7)];
+}
+
+// One wave per 16 rows.  The logits are formed transposed, Z^T = W3^T H2^T: lane
+// l holds sample l % 16 and columns 4 (l / 16) + i of a 16-column tile, which is
+// the layout of dH2 = dZ W3^T's first operand, so dZ stays in registers.  Sums
+// over the rows and the log-sum-exps (four chains of 16 columns per tile and
+// row, merged at the end) run in a fixed order.
+__global__ __launch_bounds__(256) void mlp_train_rows(MlpTrainArgs a)
+{
+    constexpr int PS = kPropStride;
+    __shared__ __align__(16) uint16_t sA[2 * 64 * PS];   // W3^T tiles (two); H1 before; dA2 [row][col], H1^T [h][row] after
+    __shared__ __align__(16) uint16_t sB[2 * 64 * PS];   // W3 tiles (two); W2 before; W2, dA2^T [col][row] after
+    __shared__ __align__(16) float sZ[64 * PS];          // logits [row][col]; dA2, dA1 after
+    __shared__ float sX[64 * kMlpIn];
+    __shared__ float sl[64];
+    __shared__ __align__(16) float slse[128];
+    const int noutp = a.w.noutp, nbin = a.w.nbin, ntile = noutp / 64;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lc = lane & 15, lr = 4 * (lane >> 4);    // this lane's column and first row of a 16 x 16 tile
+    const int wr = 16 * wv;                            // the wave's first row
     const long long r0 = (long long)blockIdx.x * 64;
     const int nrow = (int)((a.n - r0) < 64 ? (a.n - r0) : 64);
-    float* part = a.part + (size_t)blockIdx.x * L.P;
     const float inv_w = 1.0f / *a.wsum;
 
-    for (int e = tid; e < 64 * kMlpIn; e += blockDim.x) {
+    for (int e = tid; e < 64 * kMlpIn; e += 256) {
         const int s = e / kMlpIn;
         sX[e] = s < nrow ? a.X[(r0 + s) * kMlpIn + (e - s * kMlpIn)] : 0.f;
     }
-    if (tid < 64) {
-        const bool v = tid < nrow;
-        sw[tid] = v ? a.wt[r0 + tid] * inv_w : 0.f;
-        std_[tid] = v ? a.td[r0 + tid] : 0;
-        stb_[tid] = v ? a.tb[r0 + tid] : 0;
+    for (int e = tid; e < 4096; e += 256) sB[(e >> 6) * PS + (e & 63)] = a.w.W2[e];
+    // this lane's sample (row wr + lc)
+    const bool have = wr + lc < nrow;
+    const float sw = have ? a.wt[r0 + wr + lc] * inv_w : 0.f;
+    const int td = have ? a.td[r0 + wr + lc] : 0;
+    const int tb = kMlpDir + (have ? a.tb[r0 + wr + lc] : 0);
+    if (lr == 0) a.sw[r0 + wr + lc] = sw;
+    __syncthreads();
+    // H1 in the accumulators' layout: h1[4 tj + i] = H1(row lr + i, col 16 tj + lc)
+    float h1[16], h2[16];
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {
+        const int j = 16 * tj + lc;
+        float wj[kMlpIn];
+#pragma unroll
+        for (int i = 0; i < kMlpIn; ++i) wj[i] = bf2f(a.w.W1[i * kMlpHid + j]);
+        const float bj = a.w.b1[j];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float acc = bj;
+#pragma unroll
+            for (int i = 0; i < kMlpIn; ++i) acc = fmaf(sX[(wr + lr + r) * kMlpIn + i], wj[i], acc);
+            h1[4 * tj + r] = wr + lr + r < nrow ? tanhf(acc) : 0.f;
+            sA[(wr + lr + r) * PS + j] = f2bf(h1[4 * tj + r]);
+        }
     }
-    for (int e = tid; e < 4096; e += blockDim.x) sW2b[e] = a.w.W2[e];
     __syncthreads();
-    layer1(sX, a.w, nrow, sH1f, sH1b);
-    __syncthreads();
-    {
-        f4v acc[2][2];
-        acc_zero(acc);
-        gemm64(sH1b, 64, 1, sW2b, 64, 1, 64, acc);
-        acc_each(acc, [&](int r, int c, float v) {
-            const float h = r < nrow ? tanhf(v + a.w.b2[c]) : 0.f;
-            sH2f[r * 64 + c] = h;
-            sH2b[r * 64 + c] = f2bf(h);
-        });
-    }
-    __syncthreads();
-
-    const int ntile = noutp / 64;
-    // pass 1: row-wise log-sum-exp of both heads, online over the column
-    // tiles; four threads per row, 16 columns each, merged at the end
-    {
-        const int row = tid >> 2, part = tid & 3;
-        const int td = std_[row], tb = stb_[row];
-        float md = -3.0e38f, sd = 0.f, mb = -3.0e38f, sb = 0.f, ztd = 0.f, ztb = 0.f;
-        for (int jt = 0; jt < ntile; ++jt) {
-            stage_w3_tile(a.w.W3, noutp, jt, sW3b);
-            __syncthreads();
-            f4v acc[2][2];
-            acc_zero(acc);
-            gemm64(sH2b, 64, 1, sW3b, 64, 1, 64, acc);
-            acc_each(acc, [&](int r, int c, float v) { sZ[r * 64 + c] = v + a.w.b3[jt * 64 + c]; });
-            __syncthreads();
-            for (int c = part * 16; c < part * 16 + 16; ++c) {
-                const int gc = jt * 64 + c;
-                const float z = sZ[row * 64 + c];
-                if (gc < kMlpDir) {
-                    if (z > md) { sd = sd * __expf(md - z) + 1.f; md = z; }
-                    else sd += __expf(z - md);
-                    if (gc == td) ztd = z;
-                } else if (gc < kMlpDir + nbin) {
-                    if (z > mb) { sb = sb * __expf(mb - z) + 1.f; mb = z; }
-                    else sb += __expf(z - mb);
-                    if (gc - kMlpDir == tb) ztb = z;
-                }
+    uint16_t* sH = sA + 64 * PS;   // H2 [row][h] (each wave its own rows)
+    {   // H2 = tanh(H1 W2 + b2)
+        f4v acc[4];
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) acc[tj] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < 64; k0 += 16) {
+            const s4v av = frag8(sA + (wr + lc) * PS + k0 + lr);
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) {
+                const uint16_t* q = sB + (k0 + lr) * PS + 16 * tj + lc;
+                s4v bv;
+                bv.x = (short)q[0];
+                bv.y = (short)q[PS];
+                bv.z = (short)q[2 * PS];
+                bv.w = (short)q[3 * PS];
+                acc[tj] = DN_MFMA(av, bv, acc[tj]);
             }
-            __syncthreads();
+        }
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) {
+            const float bj = a.w.b2[16 * tj + lc];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float h = wr + lr + r < nrow ? tanhf(acc[tj][r] + bj) : 0.f;
+                h2[4 * tj + r] = h;
+                sH[(wr + lr + r) * PS + 16 * tj + lc] = f2bf(h);
+            }
+            // H2^T of the block, [h][row], for mlp_train_w3
+            put8(a.H2T + ((size_t)blockIdx.x * 64 + 16 * tj + lc) * 64 + wr + lr,
+                 pack4(h2[4 * tj], h2[4 * tj + 1], h2[4 * tj + 2], h2[4 * tj + 3]));
+        }
+    }
+    lds_sync();
+    s4v ha[4];   // H2 as an operand: row lc of the wave, h = 16 k + lr + i
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        ha[k] = frag8(sH + (wr + lc) * PS + 16 * k + lr);
+        put8(a.H2 + (r0 + wr + lc) * 64 + 16 * k + lr, ha[k]);
+    }
+    lds_sync();  // (H1, W2 and H2 read: the tiles take their place)
+    // b3 of this lane's columns of tile jt
+    auto bias = [&](int jt, f4v* b) {
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) b[tj][i] = a.w.b3[jt * 64 + 16 * tj + lr + i];
+    };
+    // pass 1: log-sum-exp of both heads, online over the column tiles: thread
+    // (row, part) over columns 16 part .. 16 part + 15, the four merged at the end
+    float lse_d, lse_b;
+    {
+        const int row = tid >> 2, part = tid & 3;      // a row of this wave
+        float m = -3.0e38f, sum = 0.f, zt = 0.f, md = 0.f, sd = 0.f, ztd = 0.f;
+        const int rtd = __shfl(td, row & 15), rtb = __shfl(tb, row & 15);
+        uint4 t0, t1;
+        f4v b3[4];
+        load_w3_tile(a.W3T, 0, t0, t1);
+        bias(0, b3);
+        put_w3_tile(t0, t1, sA);
+        for (int jt = 0; jt < ntile; ++jt) {
+            const uint16_t* sW = sA + (jt & 1) * 64 * PS;
+            const int jn = min(jt + 1, ntile - 1);
+            load_w3_tile(a.W3T, jn, t0, t1);
+            lds_sync();
+            f4v acc[4];
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) acc[tj] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int tj = 0; tj < 4; ++tj)
+                    acc[tj] = DN_MFMA(frag8(sW + (16 * tj + lc) * PS + 16 * k + lr), ha[k], acc[tj]);
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) *(f4v*)(sZ + (wr + lc) * PS + 16 * tj + lr) = acc[tj] + b3[tj];
+            bias(jn, b3);
+            put_w3_tile(t0, t1, sA + ((jt + 1) & 1) * 64 * PS);
+            if (jt == 1) {   // the (band, g) head starts
+                md = m;
+                sd = sum;
+                ztd = zt;
+                m = -3.0e38f;
+                sum = zt = 0.f;
+            }
+            // (this wave's rows of sZ only)
+            const int hot = (jt == 0 ? rtd : rtb) - jt * 64 - part * 16;
+            const int nc = min(16, kMlpDir + nbin - jt * 64 - part * 16);   // columns of a head
+            const float* zr = sZ + row * PS + part * 16;
+            float z[16], mm[17], t[16];
+            mm[0] = m;
+#pragma unroll
+            for (int c = 0; c < 16; ++c) z[c] = zr[c];
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                mm[c + 1] = c < nc ? fmaxf(mm[c], z[c]) : mm[c];
+                if (c == hot) zt = z[c];
+            }
+#pragma unroll
+            for (int c = 0; c < 16; ++c) t[c] = __expf(-fabsf(z[c] - mm[c]));
+#pragma unroll
+            for (int c = 0; c < 16; ++c) {
+                const float sn = z[c] > mm[c] ? sum * t[c] + 1.f : sum + t[c];
+                sum = c < nc ? sn : sum;
+            }
+            m = mm[16];
         }
         for (int o = 1; o < 4; o <<= 1) {   // merge the four partial (max, sum) pairs of the row
             const float md2 = __shfl_xor(md, o, 4), sd2 = __shfl_xor(sd, o, 4);
-            const float mb2 = __shfl_xor(mb, o, 4), sb2 = __shfl_xor(sb, o, 4);
-            const float mdn = fmaxf(md, md2), mbn = fmaxf(mb, mb2);
+            const float mb2 = __shfl_xor(m, o, 4), sb2 = __shfl_xor(sum, o, 4);
+            const float mdn = fmaxf(md, md2), mbn = fmaxf(m, mb2);
             sd = sd * __expf(md - mdn) + sd2 * __expf(md2 - mdn);
-            sb = sb * __expf(mb - mbn) + sb2 * __expf(mb2 - mbn);
+            sum = sum * __expf(m - mbn) + sb2 * __expf(mb2 - mbn);
             md = mdn;
-            mb = mbn;
+            m = mbn;
             ztd += __shfl_xor(ztd, o, 4);
-            ztb += __shfl_xor(ztb, o, 4);
+            zt += __shfl_xor(zt, o, 4);
         }
+        const float swr = __shfl(sw, row & 15);
         if (part == 0) {   // log-sum-exp per head; the sample's loss
-            sm_d[row] = md + __logf(sd);
-            sm_b[row] = mb + __logf(sb);
-            sloss[row] = sw[row] * ((sm_d[row] - ztd) + (sm_b[row] - ztb));
+            const float ld = md + __logf(sd), lb = m + __logf(sum);
+            slse[2 * row] = ld;
+            slse[2 * row + 1] = lb;
+            a.lse[2 * (r0 + row)] = ld;
+            a.lse[2 * (r0 + row) + 1] = lb;
+            sl[row] = swr * ((ld - ztd) + (lb - zt));
+        }
+        lds_sync();
+        lse_d = slse[2 * (wr + lc)];
+        lse_b = slse[2 * (wr + lc) + 1];
+    }
+    // pass 2: dZ = w (softmax - onehot), dH2 = dZ W3^T
+    f4v dh[4];
+#pragma unroll
+    for (int th = 0; th < 4; ++th) dh[th] = f4v{0.f, 0.f, 0.f, 0.f};
+    {
+        uint4 t0, t1, c0, c1;
+        f4v b3[4];
+        load_w3_tile(a.W3T, 0, t0, t1);
+        load_w3_cols(a.w.W3, noutp, 0, c0, c1);
+        bias(0, b3);
+        put_w3_tile(t0, t1, sA);
+        put_w3_tile(c0, c1, sB);
+        for (int jt = 0; jt < ntile; ++jt) {
+            const uint16_t* sW = sA + (jt & 1) * 64 * PS;
+            const uint16_t* sC = sB + (jt & 1) * 64 * PS;
+            const int jn = min(jt + 1, ntile - 1);
+            load_w3_tile(a.W3T, jn, t0, t1);
+            load_w3_cols(a.w.W3, noutp, jn, c0, c1);
+            lds_sync();
+            f4v acc[4];
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) acc[tj] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 4; ++k)
+#pragma unroll
+                for (int tj = 0; tj < 4; ++tj)
+                    acc[tj] = DN_MFMA(frag8(sW + (16 * tj + lc) * PS + 16 * k + lr), ha[k], acc[tj]);
+            const float lse = jt == 0 ? lse_d : lse_b;
+            const int hot = (jt == 0 ? td : tb) - jt * 64 - lr, nc = kMlpDir + nbin - jt * 64 - lr;
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) {
+                float dz[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const float v = mlp_dz(acc[tj][i] + b3[tj][i], sw, lse, hot == 16 * tj + i);
+                    dz[i] = 16 * tj + i < nc ? v : 0.f;
+                }
+                const s4v dv = pack4(dz[0], dz[1], dz[2], dz[3]);
+#pragma unroll
+                for (int th = 0; th < 4; ++th)
+                    dh[th] = DN_MFMA(dv, frag8(sC + (16 * th + lc) * PS + 16 * tj + lr), dh[th]);
+            }
+            bias(jn, b3);
+            put_w3_tile(t0, t1, sA + ((jt + 1) & 1) * 64 * PS);
+            put_w3_tile(c0, c1, sB + ((jt + 1) & 1) * 64 * PS);
         }
     }
     __syncthreads();
-
-    // pass 2: dZ = w (softmax - onehot), gradients of W3, b3 and dH2
-    f4v accH[2][2];
-    acc_zero(accH);
-    for (int jt = 0; jt < ntile; ++jt) {
-        stage_w3_tile(a.w.W3, noutp, jt, sW3b);
-        __syncthreads();
-        {
-            f4v acc[2][2];
-            acc_zero(acc);
-            gemm64(sH2b, 64, 1, sW3b, 64, 1, 64, acc);
-            acc_each(acc, [&](int r, int c, float v) {
-                const int gc = jt * 64 + c;
-                const float z = v + a.w.b3[gc];
-                float dz = 0.f;
-                if (gc < kMlpDir) dz = sw[r] * (__expf(z - sm_d[r]) - (gc == std_[r] ? 1.f : 0.f));
-                else if (gc < kMlpDir + nbin) dz = sw[r] * (__expf(z - sm_b[r]) - (gc - kMlpDir == stb_[r] ? 1.f : 0.f));
-                sZ[r * 64 + c] = dz;
-                sdZb[r * 64 + c] = f2bf(dz);
-            });
+    // layer 2 backward: dA2 = dH2 (1 - H2^2); W2 again
+    uint16_t *sD = sA, *sHT = sA + 64 * PS, *sW2 = sB, *sDT = sB + 64 * PS;   // dA2, H1^T, W2, dA2^T
+    for (int e = tid; e < 4096; e += 256) sW2[(e >> 6) * PS + (e & 63)] = a.w.W2[e];
+    float* part = a.part + (size_t)blockIdx.x * kMlpSmall;
+    const MlpLayout L = mlp_layout(nbin);
+#pragma unroll
+    for (int tj = 0; tj < 4; ++tj) {
+        float d[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float h = h2[4 * tj + i];
+            d[i] = dh[tj][i] * (1.f - h * h);
+            sZ[(wr + lr + i) * PS + 16 * tj + lc] = d[i];
+            sD[(wr + lr + i) * PS + 16 * tj + lc] = f2bf(d[i]);
         }
-        __syncthreads();
-        if (tid < 64) {   // db3 (column sums, FP32)
-            float s = 0.f;
-            for (int r = 0; r < 64; ++r) s += sZ[r * 64 + tid];
-            part[L.ob3 + jt * 64 + tid] = s;
-        }
-        {   // dW3 tile = H2^T dZ
-            f4v acc[2][2];
-            acc_zero(acc);
-            gemm64(sH2b, 1, 64, sdZb, 64, 1, 64, acc);
-            acc_each(acc, [&](int h, int c, float v) { part[L.oW3 + (size_t)h * noutp + jt * 64 + c] = v; });
-        }
-        // dH2 += dZ W3_tile^T
-        gemm64(sdZb, 64, 1, sW3b, 1, 64, 64, accH);
-        __syncthreads();
+        put8(sDT + (16 * tj + lc) * PS + wr + lr, pack4(d[0], d[1], d[2], d[3]));
+        put8(sHT + (16 * tj + lc) * PS + wr + lr, pack4(h1[4 * tj], h1[4 * tj + 1], h1[4 * tj + 2], h1[4 * tj + 3]));
     }
-    // layer 2 backward: dA2 = dH2 (1 - H2^2)
-    acc_each(accH, [&](int r, int c, float v) {
-        const float h = sH2f[r * 64 + c];
-        const float d = v * (1.f - h * h);
-        sZ[r * 64 + c] = d;
-        sdZb[r * 64 + c] = f2bf(d);
-    });
     __syncthreads();
     if (tid < 64) {
         float s = 0.f;
-        for (int r = 0; r < 64; ++r) s += sZ[r * 64 + tid];
+        for (int r = 0; r < 64; ++r) s += sZ[r * PS + tid];
         part[L.ob2 + tid] = s;
     }
-    {   // dW2 = H1^T dA2
-        f4v acc[2][2];
-        acc_zero(acc);
-        gemm64(sH1b, 1, 64, sdZb, 64, 1, 64, acc);
-        acc_each(acc, [&](int h, int c, float v) { part[L.oW2 + h * 64 + c] = v; });
+    {   // dW2 = H1^T dA2: this wave's 16 rows h
+        f4v acc[4];
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) acc[tj] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < 64; k0 += 16) {
+            const s4v av = frag8(sHT + (wr + lc) * PS + k0 + lr);
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) acc[tj] = DN_MFMA(av, frag8(sDT + (16 * tj + lc) * PS + k0 + lr), acc[tj]);
+        }
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) part[L.oW2 + (wr + lr + i) * 64 + 16 * tj + lc] = acc[tj][i];
     }
-    {   // dA1 = (dA2 W2^T)(1 - H1^2), kept in sH2f
-        f4v acc[2][2];
-        acc_zero(acc);
-        gemm64(sdZb, 64, 1, sW2b, 1, 64, 64, acc);
-        __syncthreads();   // every wave has read sH2f (dA2 epilogue) before it is overwritten
-        acc_each(acc, [&](int r, int c, float v) {
-            const float h = sH1f[r * 64 + c];
-            sH2f[r * 64 + c] = v * (1.f - h * h);
-        });
+    {   // dA1 = (dA2 W2^T)(1 - H1^2)
+        f4v acc[4];
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj) acc[tj] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k0 = 0; k0 < 64; k0 += 16) {
+            const s4v av = frag8(sD + (wr + lc) * PS + k0 + lr);
+#pragma unroll
+            for (int tj = 0; tj < 4; ++tj) acc[tj] = DN_MFMA(av, frag8(sW2 + (16 * tj + lc) * PS + k0 + lr), acc[tj]);
+        }
+        __syncthreads();   // db2's sums have read sZ
+#pragma unroll
+        for (int tj = 0; tj < 4; ++tj)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float h = h1[4 * tj + i];
+                sZ[(wr + lr + i) * PS + 16 * tj + lc] = acc[tj][i] * (1.f - h * h);
+            }
     }
     __syncthreads();
-    if (tid < 64) {
+    for (int e = tid; e < (kMlpIn + 1) * kMlpHid; e += 256) {   // dW1 = X^T dA1 (FP32), db1
+        const int i = e >> 6, j = e & 63;
         float s = 0.f;
-        for (int r = 0; r < 64; ++r) s += sH2f[r * 64 + tid];
-        part[L.ob1 + tid] = s;
+        if (i < kMlpIn) {
+            for (int r = 0; r < 64; ++r) s = fmaf(sX[r * kMlpIn + i], sZ[r * PS + j], s);
+        } else {
+            for (int r = 0; r < 64; ++r) s += sZ[r * PS + j];
+        }
+        part[(i < kMlpIn ? L.oW1 + i * kMlpHid : L.ob1) + j] = s;
     }
-    for (int e = tid; e < kMlpIn * kMlpHid; e += blockDim.x) {   // dW1 = X^T dA1 (FP32)
-        const int i = e / kMlpHid, j = e - i * kMlpHid;
+    if (tid == 192) {
         float s = 0.f;
-        for (int r = 0; r < 64; ++r) s = fmaf(sX[r * kMlpIn + i], sH2f[r * 64 + j], s);
-        part[L.oW1 + e] = s;
-    }
-    if (tid == 0) {
-        float s = 0.f;
-        for (int r = 0; r < 64; ++r) s += sloss[r];
+        for (int r = 0; r < 64; ++r) s += sl[r];
         a.loss_part[blockIdx.x] = s;
     }
 }
 
-// grad[p] = sum over blocks of part[b][p]; loss = sum of loss_part.
-__global__ void mlp_reduce(const float* part, const float* loss_part, int nblk, int P, float* grad, float* loss)
+// dW3 and db3 of column tile jt = blockIdx.x over the 64-row blocks of split
+// blockIdx.y; wave w holds columns 16 w .. 16 w + 15.
+__global__ __launch_bounds__(256) void mlp_train_w3(MlpTrainArgs a, int per)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p < P) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; ++b) s += part[(size_t)b * P + p];
-        grad[p] = s;
+    constexpr int PS = kPropStride;
+    __shared__ __align__(16) uint16_t sH[2][64 * PS], sHT[2][64 * PS];   // H2 [row][h], H2^T [h][row]
+    __shared__ __align__(16) float slse[2][64], ssw[2][64];
+    __shared__ __align__(16) int shot[2][64];
+    const int noutp = a.w.noutp, jt = blockIdx.x;
+    const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+    const int lc = lane & 15, lr = 4 * (lane >> 4);
+    const int col = jt * 64 + 16 * wv + lc;
+    const bool used = col < kMlpDir + a.w.nbin;
+    const long long nblk = (a.n + 63) / 64;
+    const long long b0 = (long long)blockIdx.y * per, b1 = b0 + per < nblk ? b0 + per : nblk;
+    s4v wf[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) wf[k] = frag8(a.W3T + (size_t)col * 64 + 16 * k + lr);
+    const float bj = a.w.b3[col];
+    f4v dw[4];   // dW3(h = 16 th + lr + i, col)
+#pragma unroll
+    for (int th = 0; th < 4; ++th) dw[th] = f4v{0.f, 0.f, 0.f, 0.f};
+    float db = 0.f;
+    uint4 h0, h1, t0, t1;
+    float xl = 0.f;   // this thread's of: 64 log-sum-exps of the tile's head, 64 weights, 64 bins' columns
+    int xt = 0;
+    auto load = [&](long long b) {
+        h0 = ((const uint4*)(a.H2 + b * 4096))[tid];
+        h1 = ((const uint4*)(a.H2 + b * 4096))[tid + 256];
+        t0 = ((const uint4*)(a.H2T + b * 4096))[tid];
+        t1 = ((const uint4*)(a.H2T + b * 4096))[tid + 256];
+        const long long r = b * 64 + (tid & 63);
+        if (tid < 64) xl = a.lse[2 * r + (jt > 0 ? 1 : 0)];
+        else if (tid < 128) xl = a.sw[r];
+        else if (tid < 192) xt = r < a.n ? (jt > 0 ? kMlpDir + a.tb[r] : a.td[r]) : -1;
+    };
+    auto put = [&](int p) {
+        put_w3_tile(h0, h1, sH[p]);
+        put_w3_tile(t0, t1, sHT[p]);
+        if (tid < 64) slse[p][tid] = xl;
+        else if (tid < 128) ssw[p][tid - 64] = xl;
+        else if (tid < 192) shot[p][tid - 128] = xt;
+    };
+    if (b0 < b1) {
+        load(b0);
+        put(0);
     }
-    if (p == 0) {
-        float s = 0.f;
-        for (int b = 0; b < nblk; ++b) s += loss_part[b];
-        *loss = s;
+    for (long long b = b0; b < b1; ++b) {
+        const int p = (int)(b - b0) & 1;
+        load(b + 1 < b1 ? b + 1 : b);
+        lds_sync();
+        s4v dv[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {   // 16 rows
+            f4v acc = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) acc = DN_MFMA(frag8(sH[p] + (16 * q + lc) * PS + 16 * k + lr), wf[k], acc);
+            const f4v lse = *(const f4v*)(slse[p] + 16 * q + lr), w = *(const f4v*)(ssw[p] + 16 * q + lr);
+            const int4 hot = *(const int4*)(shot[p] + 16 * q + lr);
+            const float d0 = mlp_dz(acc[0] + bj, w[0], lse[0], hot.x == col), d1 = mlp_dz(acc[1] + bj, w[1], lse[1], hot.y == col);
+            const float d2 = mlp_dz(acc[2] + bj, w[2], lse[2], hot.z == col), d3 = mlp_dz(acc[3] + bj, w[3], lse[3], hot.w == col);
+            db += used ? (d0 + d1) + (d2 + d3) : 0.f;
+            dv[q] = used ? pack4(d0, d1, d2, d3) : s4v{0, 0, 0, 0};
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+#pragma unroll
+            for (int th = 0; th < 4; ++th) dw[th] = DN_MFMA(frag8(sHT[p] + (16 * th + lc) * PS + 16 * q + lr), dv[q], dw[th]);
+        put(p ^ 1);
     }
+    float* part = a.part3 + (size_t)blockIdx.y * (64 + 1) * noutp;
+#pragma unroll
+    for (int th = 0; th < 4; ++th)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) part[(size_t)(16 * th + lr + i) * noutp + col] = dw[th][i];
+    db += __shfl_xor(db, 16);
+    db += __shfl_xor(db, 32);
+    if (lane < 16) part[(size_t)64 * noutp + col] = db;
 }
 
-__global__ void mlp_wsum(const float* wt, long long n, float* out)
+// grad: the parameters below W3 summed over the row blocks in order (64 per
+// block here: a wave with 32 loads in flight), W3 and b3 over the splits; loss.
+__global__ __launch_bounds__(256) void mlp_reduce(const float* part, const float* loss_part, int nblk, const float* part3,
+                                                  int nsplit, int P, float* grad, float* loss)
 {
     __shared__ float s[256];
-    float v = 0.f;
-    for (long long i = threadIdx.x; i < n; i += blockDim.x) v += wt[i];
-    s[threadIdx.x] = v;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if (threadIdx.x < o) s[threadIdx.x] += s[threadIdx.x + o];
-        __syncthreads();
+    const int tid = threadIdx.x;
+    constexpr int nsb = kMlpSmall / 64;
+    if ((int)blockIdx.x < nsb) {
+        if (tid < 64) {
+            const float* q = part + blockIdx.x * 64 + tid;
+            float v = 0.f;
+            int b = 0;
+            for (; b + 32 <= nblk; b += 32) {
+                float x[32];
+#pragma unroll
+                for (int u = 0; u < 32; ++u) x[u] = q[(size_t)(b + u) * kMlpSmall];
+#pragma unroll
+                for (int u = 0; u < 32; ++u) v += x[u];
+            }
+            for (; b < nblk; ++b) v += q[(size_t)b * kMlpSmall];
+            grad[blockIdx.x * 64 + tid] = v;
+        }
+        if (blockIdx.x == 0) {
+            float l = 0.f;
+            for (int i = tid; i < nblk; i += 256) l += loss_part[i];
+            s[tid] = l;
+            __syncthreads();
+            for (int o = 128; o > 0; o >>= 1) {
+                if (tid < o) s[tid] += s[tid + o];
+                __syncthreads();
+            }
+            if (tid == 0) *loss = s[0];
+        }
+        return;
     }
-    if (threadIdx.x == 0) *out = s[0] > 0.f ? s[0] : 1.f;
+    const int p = kMlpSmall + (blockIdx.x - nsb) * 256 + tid;
+    if (p >= P) return;
+    const size_t st = (size_t)(P - kMlpSmall);
+    const float* q = part3 + (p - kMlpSmall);
+    float v = 0.f;
+    int k = 0;
+    for (; k + 8 <= nsplit; k += 8) {
+        float x[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) x[u] = q[(size_t)(k + u) * st];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) v += x[u];
+    }
+    for (; k < nsplit; ++k) v += q[(size_t)k * st];
+    grad[p] = v;
 }
 
 // Adam on the FP32 master parameters; BF16 copies of the weight matrices.
@@ -410,7 +735,7 @@ __global__ __launch_bounds__(256) void mlp_forward_rows(const float* X, long lon
     }
     for (int e = threadIdx.x; e < 4096; e += blockDim.x) sW2b[e] = w.W2[e];
     __syncthreads();
-    layer1(sX, w, nrow, nullptr, sH1b);
+    layer1(sX, w, nrow, sH1b);
     __syncthreads();
     {
         f4v acc[2][2];
@@ -517,7 +842,7 @@ __global__ __launch_bounds__(256) void mlp_proposal(GenArgs a, float* U)
             cell_features(f, si.w & 1023, (si.w >> 10) & 1023, (si.w >> 20) & 1023, sX + tid * kMlpIn);
         }
         __syncthreads();
-        layer1(sX, a.mlpw, ns, nullptr, sH1b, PS);
+        layer1(sX, a.mlpw, ns, sH1b, PS);
         __syncthreads();
         {
             f4v acc[2][2];

@@ -45,9 +45,11 @@ __global__ void cand_scan(TraceArgs P, uint32_t nfin, uint32_t* list);
 __global__ void mlp_proposal(GenArgs a, float* cdf);
 __global__ void raygen_learned(GenArgs a, const float* U, const float* pcdf);
 __global__ void raygen_learned_lds(GenArgs a, const float* U, const float* pcdf, int G);
-__global__ void mlp_train_tile(MlpTrainArgs a);
-__global__ void mlp_reduce(const float* part, const float* loss_part, int nblk, int P, float* grad, float* loss);
-__global__ void mlp_wsum(const float* wt, long long n, float* out);
+__global__ void mlp_train_prep(const float* wt, long long n, float* wsum, const uint16_t* W3, int noutp, uint16_t* W3T);
+__global__ void mlp_train_rows(MlpTrainArgs a);
+__global__ void mlp_train_w3(MlpTrainArgs a, int per);
+__global__ void mlp_reduce(const float* part, const float* loss_part, int nblk, const float* part3, int nsplit, int P,
+                           float* grad, float* loss);
 __global__ void mlp_adam(float* theta, float* m, float* v, const float* grad, int P, MlpLayout L, float lr, float b1,
                          float b2, float eps, float c1, float c2, uint16_t* W1b, uint16_t* W2b, uint16_t* W3b);
 __global__ void mlp_forward_rows(const float* X, long long n, MlpWeights w, float* Z);
@@ -2257,20 +2259,47 @@ int dnsmc_mlp_grad(int nbin, const float* theta, const unsigned short* W1b, cons
     const MlpLayout L = mlp_layout(nbin);
     const long long nblk = (n + 63) / 64;
     if (nblk > 0x7FFFFFFF || nwork < nblk * (L.P + 1) + L.P + 2) return fail(DNSMC_EINVAL, "work buffer too small");
-    float* part = work;
-    float* lpart = part + nblk * L.P;
-    float* wsum = lpart + nblk;
-    float* dloss = wsum + 1;
+    // the work buffer, in 16-byte units from its first aligned address: the
+    // rows' H2 (twice), log-sum-exps, weights and small partials, W3^T, then as
+    // many splits of W3's gradient as fit (at least one, by the check above:
+    // the rest of a block's P + 1 floats, and P + 2 more, exceed W3^T and one
+    // split for every nbin)
+    float* w0 = (float*)(((uintptr_t)work + 15) & ~(uintptr_t)15);
+    float* end = work + nwork;
+    auto take = [&](long long floats) {
+        float* p = w0;
+        w0 += (floats + 3) / 4 * 4;
+        return p;
+    };
     MlpTrainArgs a;
     a.X = X; a.td = td; a.tb = tb; a.wt = wt; a.n = (int)std::min<long long>(n, 0x7FFFFFFF);
+    float* wsum = take(4);
+    float* dloss = wsum + 1;
     a.wsum = wsum;
     a.w = mlp_weights_of(nbin, W1b, W2b, W3b, theta);
-    a.part = part;
-    a.loss_part = lpart;
-    hipLaunchKernelGGL(mlp_wsum, dim3(1), dim3(256), 0, 0, wt, n, wsum);
-    const size_t lds = sizeof(float) * (64 * kMlpIn + 3 * 4096 + 8 * 64 + 2 * 64) + 5 * 4096 * sizeof(uint16_t);
-    hipLaunchKernelGGL(mlp_train_tile, dim3((unsigned)nblk), dim3(256), lds, 0, a);
-    hipLaunchKernelGGL(mlp_reduce, dim3((L.P + 255) / 256), dim3(256), 0, 0, part, lpart, (int)nblk, L.P, grad, dloss);
+    a.H2 = (uint16_t*)take(nblk * 2048);
+    a.H2T = (uint16_t*)take(nblk * 2048);
+    a.lse = take(nblk * 128);
+    a.sw = take(nblk * 64);
+    a.part = take(nblk * kMlpSmall);
+    a.loss_part = take(nblk);
+    uint16_t* W3T = (uint16_t*)take(32ll * L.noutp);
+    a.W3T = W3T;
+    a.part3 = w0;
+    const long long st3 = (long long)L.P - kMlpSmall;
+    // splits of the rows: about four blocks of mlp_train_w3 per CU, at least two
+    // row blocks each
+    const int ntile = L.noutp / 64;
+    long long nsplit = std::min<long long>((nblk + 1) / 2, std::max<long long>(1, 1024 / ntile));
+    nsplit = std::max<long long>(1, std::min<long long>(nsplit, (end - w0) / st3));
+    if (end - w0 < st3) return fail(DNSMC_EINVAL, "work buffer too small");
+    const int per = (int)((nblk + nsplit - 1) / nsplit);
+    nsplit = (nblk + per - 1) / per;
+    hipLaunchKernelGGL(mlp_train_prep, dim3(1 + ntile), dim3(256), 0, 0, wt, n, wsum, W3b, L.noutp, W3T);
+    hipLaunchKernelGGL(mlp_train_rows, dim3((unsigned)nblk), dim3(256), 0, 0, a);
+    hipLaunchKernelGGL(mlp_train_w3, dim3((unsigned)ntile, (unsigned)nsplit), dim3(256), 0, 0, a, per);
+    hipLaunchKernelGGL(mlp_reduce, dim3((unsigned)(kMlpSmall / 64 + (st3 + 255) / 256)), dim3(256), 0, 0, a.part,
+                       a.loss_part, (int)nblk, a.part3, (int)nsplit, L.P, grad, dloss);
     HIPCHK(hipGetLastError());
     if (loss) HIPCHK(hipMemcpy(loss, dloss, sizeof(float), hipMemcpyDeviceToHost));
     else HIPCHK(hipDeviceSynchronize());
