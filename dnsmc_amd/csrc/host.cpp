@@ -677,4 +677,82 @@ void xorwow_jump_tables(std::vector<uint32_t>& out)
     delete t;
 }
 
+namespace {
+struct P160 { uint32_t c[5]; };
+
+// a b modulo x^160 + low
+P160 p_mul(const P160& a, const P160& b, const P160& low)
+{
+    P160 r{{0, 0, 0, 0, 0}};
+    for (int i = 159; i >= 0; --i) {
+        const uint32_t top = r.c[4] >> 31;
+        for (int w = 4; w > 0; --w) r.c[w] = (r.c[w] << 1) | (r.c[w - 1] >> 31);
+        r.c[0] <<= 1;
+        if (top)
+            for (int w = 0; w < 5; ++w) r.c[w] ^= low.c[w];
+        if ((b.c[i >> 5] >> (i & 31)) & 1u)
+            for (int w = 0; w < 5; ++w) r.c[w] ^= a.c[w];
+    }
+    return r;
+}
+
+P160 p_pow(uint64_t n, const P160& low)
+{
+    P160 r{{1u, 0, 0, 0, 0}}, x{{2u, 0, 0, 0, 0}};
+    for (; n; n >>= 1) {
+        if (n & 1u) r = p_mul(r, x, low);
+        x = p_mul(x, x, low);
+    }
+    return r;
+}
+
+// The coefficients below x^160 of the step matrix's characteristic polynomial
+// (irreducible: the recurrence has period 2^160 - 1), as the shortest linear
+// recurrence of one bit of the sequence (Berlekamp-Massey; Massey 1969).
+P160 xorwow_char_poly()
+{
+    const int N = 352;
+    std::vector<uint8_t> b(N), C(N + 1, 0), B(N + 1, 0), T;
+    Xorwow s{1u, 0, 0, 0, 0, 0};
+    for (int i = 0; i < N; ++i) {
+        b[i] = (uint8_t)(s.x0 & 1u);
+        (void)xorwow_next(s);
+    }
+    C[0] = B[0] = 1;
+    int Ln = 0, m = 1;
+    for (int n = 0; n < N; ++n) {
+        int d = b[n];
+        for (int i = 1; i <= Ln; ++i) d ^= C[i] & b[n - i];
+        if (!d) {
+            ++m;
+            continue;
+        }
+        T = C;
+        for (int i = 0; i + m <= N; ++i) C[i + m] ^= B[i];
+        if (2 * Ln <= n) {
+            Ln = n + 1 - Ln;
+            B = T;
+            m = 1;
+        } else {
+            ++m;
+        }
+    }
+    P160 low{{0, 0, 0, 0, 0}};   // sum of C_i s_{n-i} = 0: x^160 + sum of C_i x^(160-i)
+    for (int i = 1; i <= 160; ++i)
+        if (C[i]) low.c[(160 - i) >> 5] |= 1u << ((160 - i) & 31);
+    return low;
+}
+}  // namespace
+
+void xorwow_jump_polys(uint64_t base, uint64_t step, int count, std::vector<uint32_t>& out)
+{
+    const P160 low = xorwow_char_poly();
+    P160 p = p_pow(base, low);
+    const P160 d = p_pow(step, low);
+    for (int i = 0; i < count; ++i) {
+        out.insert(out.end(), p.c, p.c + 5);
+        p = p_mul(p, d, low);
+    }
+}
+
 }  // namespace dn

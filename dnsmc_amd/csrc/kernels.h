@@ -150,6 +150,9 @@ struct TraceArgs {
     float* log_w;
 };
 
+// Words of a slot's XORWOW sequence a jump reads (160 + 4, in uint4).
+constexpr int kXwSeq = 168;
+
 struct GenArgs {
     // geometry of level 0 (emitter temperature)
     const float* T0;
@@ -176,11 +179,15 @@ struct GenArgs {
     // compat
     uint32_t xw_seed[6];
     const uint32_t* xw_jump_sub;   // 60 matrices (2^(67+j))
-    const uint32_t* xw_jump_off;   // 64 matrices (2^j)
+    const uint32_t* xw_poly;       // 5 words per run: the jump to its first draw (xorwow_jump_polys); sorted
+                                   // without Sobol: 256 more to its first direction draw, from entry 256
     const uint32_t* sobol_v;       // 2 x 32
     int use_sobol;
     int draws_per_bundle;
-    int sub_len;                   // bundles per generator thread
+    int run_len;                   // bundles per generator thread
+    int bin_weights;               // raygen_compat: a slot's weights once per bin
+    int cdf_lds;                   // raygen_compat: the g CDFs in LDS
+    FastDiv fd_nQ;
     int n0, n1, n2;                // level-0 sizes (reference stream decomposition)
     int num_streams, num_gpu, gpu, p_row, ystart;
     const int* band_order;         // sorted mode: band at each position of the kavg order

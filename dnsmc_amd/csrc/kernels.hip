@@ -25,7 +25,7 @@ typedef __attribute__((address_space(1))) const float gfloat;
 // Emitter weights shared by the generators: Ibmax kappa_i Ib_i / (kappa_max Ib_max)
 // (code/mc_gpu.cu:63,:163-169).
 __device__ __forceinline__ void bundle_weight(const GenArgs& a, const float* ib_tab, float Ti, int band, int g,
-                                              float* w, float* winv)
+                                              float* w, float* winv, float* inv_ib)
 {
     float kap, ib;
     int bg = band * a.nQ + g;
@@ -48,7 +48,8 @@ __device__ __forceinline__ void bundle_weight(const GenArgs& a, const float* ib_
     }
     float ww = a.Ibmax * (kap * ib) * a.inv_emax[bg];
     *w = ww;
-    *winv = ww * (1.0f / ib);
+    *inv_ib = 1.0f / ib;
+    *winv = ww * *inv_ib;
 }
 
 // ------------------------------------------------------- raygen_plain ----
@@ -79,8 +80,8 @@ __global__ __launch_bounds__(256) void raygen_plain(GenArgs a)
         int g = a.g_search ? cdf_search(s_cdfg + band * a.nQ, a.nQ, u01_open(x.y)) : 0;
         g = g > a.nQ - 1 ? a.nQ - 1 : g;
         float Ti = a.T0[(size_t)a.snap * a.tstride0 + si.z];
-        float w, winv;
-        bundle_weight(a, ibt, Ti, band, g, &w, &winv);
+        float w, winv, iib;
+        bundle_weight(a, ibt, Ti, band, g, &w, &winv, &iib);
         uint32_t w0, w1;
         desc_pack(x.z >> 8, x.w >> 8, band, g, &w0, &w1);
         a.w0[q] = w0;
@@ -91,31 +92,24 @@ __global__ __launch_bounds__(256) void raygen_plain(GenArgs a)
 }
 
 // ------------------------------------------------------ raygen_compat ----
-// 160-bit GF(2) matrix (160 columns x 5 words) applied to an XORWOW state.
-__device__ __forceinline__ void gf2_apply(const uint32_t* __restrict__ M, Xorwow& s)
-{
-    uint32_t in[5] = {s.x0, s.x1, s.x2, s.x3, s.x4};
-    uint32_t r0 = 0, r1 = 0, r2 = 0, r3 = 0, r4 = 0;
-#pragma unroll
-    for (int w = 0; w < 5; ++w) {
-        uint32_t v = in[w];
-        for (int bit = 0; bit < 32; ++bit) {
-            if ((v >> bit) & 1u) {
-                const uint32_t* c = M + (size_t)(w * 32 + bit) * 5;
-                r0 ^= c[0]; r1 ^= c[1]; r2 ^= c[2]; r3 ^= c[3]; r4 ^= c[4];
-            }
-        }
-    }
-    s.x0 = r0; s.x1 = r1; s.x2 = r2; s.x3 = r3; s.x4 = r4;
-}
-
 __device__ __forceinline__ uint32_t sobol_at(const uint32_t* v, uint64_t n)
 {
-    uint64_t gc = n ^ (n >> 1);
+    const uint32_t gc = (uint32_t)(n ^ (n >> 1));
     uint32_t x = 0;
-    for (int k = 0; k < 32; ++k)
-        if ((gc >> k) & 1ull) x ^= v[k];
+#pragma unroll 8
+    for (int k = 0; k < 32; ++k) x ^= v[k] & (uint32_t)((int32_t)(gc << (31 - k)) >> 31);
     return x;
+}
+
+// Exclusive or over the wave, in every lane.
+__device__ __forceinline__ uint32_t wave_xor(uint32_t v)
+{
+    v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0xB1, 0xF, 0xF, false);    // quad: lane ^ 1
+    v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x4E, 0xF, 0xF, false);    // quad: lane ^ 2
+    v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x141, 0xF, 0xF, false);   // row_half_mirror
+    v ^= (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x140, 0xF, 0xF, false);   // row_mirror
+    const uint32_t a = (uint32_t)__builtin_amdgcn_readlane((int)v, 0) ^ (uint32_t)__builtin_amdgcn_readlane((int)v, 16);
+    return a ^ (uint32_t)__builtin_amdgcn_readlane((int)v, 32) ^ (uint32_t)__builtin_amdgcn_readlane((int)v, 48);
 }
 
 // XORWOW stream of a compat slot (cell, block v), seeded as
@@ -123,7 +117,14 @@ __device__ __forceinline__ uint32_t sobol_at(const uint32_t* v, uint64_t n)
 // scramble, subsequence = the reference's product
 // (idx+1)(stream+1)(v+1)(1+gpu)ystart over its stream decomposition of the
 // cell (code/mc_gpu.cu:84-87), jump 2^67 per subsequence.
-__device__ Xorwow compat_stream(const GenArgs& a, int cell, int v)
+//
+// The generator's recurrence is linear over GF(2) with step matrix A, and its
+// state after i steps is y_i .. y_{i+4} of one word sequence.  Called by one
+// wave: the subsequence's 160 x 160 bit matrices are applied to the seed with
+// 64 columns at a time across the lanes, and the first kXwSeq words of the
+// slot's sequence are written to y.  Threads then start anywhere in the stream
+// with one product, xorwow_jump.
+__device__ __forceinline__ void compat_sequence(const GenArgs& a, int cell, int v, int lane, uint32_t* y)
 {
     int ci = cell % a.n0, cj = (cell / a.n0) % a.n1, ck = cell / (a.n0 * a.n1);
     int per_stream = a.n0 / a.num_streams;
@@ -133,190 +134,129 @@ __device__ Xorwow compat_stream(const GenArgs& a, int cell, int v)
     int idx = (ci - stream * per_stream) * (a.n2 / a.num_gpu * (a.n1 / a.p_row)) + jloc * (a.n2 / a.num_gpu) + kloc;
     int32_t prod = (int32_t)((uint32_t)(idx + 1) * (uint32_t)(stream + 1) * (uint32_t)(v + 1) *
                              (uint32_t)(1 + a.gpu) * (uint32_t)a.ystart);
-    uint64_t subseq = (uint64_t)(int64_t)prod;
-    Xorwow s{a.xw_seed[0], a.xw_seed[1], a.xw_seed[2], a.xw_seed[3], a.xw_seed[4], a.xw_seed[5]};
-    for (int j = 0; j < 60; ++j)
-        if ((subseq >> j) & 1ull) gf2_apply(a.xw_jump_sub + (size_t)j * 800, s);
-    return s;
-}
-
-// Advance an XORWOW state by `off` draws (the Weyl counter d by 362437 per draw).
-__device__ void xorwow_skip(const GenArgs& a, Xorwow& s, uint64_t off)
-{
-    for (int j = 0; j < 64; ++j)
-        if ((off >> j) & 1ull) {
-            gf2_apply(a.xw_jump_off + (size_t)j * 800, s);
-            if (j < 32) s.d += 362437u * (1u << j);
+    prod = __builtin_amdgcn_readfirstlane(prod);
+    uint64_t m = (uint64_t)(int64_t)prod & ((1ull << 60) - 1ull);
+    uint32_t x[5];
+    for (int w = 0; w < 5; ++w) x[w] = a.xw_seed[w];
+    const uint32_t* col = a.xw_jump_sub + lane * 5;
+    const int l5 = lane & 31;
+    uint32_t c[15], d[15];
+    auto load = [&](int j, uint32_t* o) {   // columns lane, lane + 64 and (lanes 0..31) lane + 128
+        const uint32_t* q = col + (size_t)j * 800;
+#pragma unroll
+        for (int w = 0; w < 5; ++w) {
+            o[w] = q[w];
+            o[5 + w] = q[320 + w];
+            o[10 + w] = q[lane < 32 ? 640 + w : w];
         }
+    };
+    if (m) load(__builtin_ctzll(m), c);
+    while (m) {
+        m &= m - 1;
+        if (m) load(__builtin_ctzll(m), d);
+        const uint32_t m0 = 0u - (((lane < 32 ? x[0] : x[1]) >> l5) & 1u);
+        const uint32_t m1 = 0u - (((lane < 32 ? x[2] : x[3]) >> l5) & 1u);
+        const uint32_t m2 = lane < 32 ? 0u - ((x[4] >> l5) & 1u) : 0u;
+#pragma unroll
+        for (int w = 0; w < 5; ++w) x[w] = wave_xor((c[w] & m0) ^ (c[5 + w] & m1) ^ (c[10 + w] & m2));
+#pragma unroll
+        for (int w = 0; w < 15; ++w) c[w] = d[w];
+    }
+    Xorwow s{x[0], x[1], x[2], x[3], x[4], 0u};
+    if (lane < 5) y[lane] = lane == 0 ? x[0] : lane == 1 ? x[1] : lane == 2 ? x[2] : lane == 3 ? x[3] : x[4];
+#pragma unroll 5
+    for (int i = 5; i < kXwSeq; ++i) {
+        (void)xorwow_next(s);
+        if (lane == 0) y[i] = s.x4;
+    }
 }
 
-// One thread per (slot, run of sub_len bundles).  The stream of a slot (cell c,
-// block v) is XORWOW seeded as curand_init(1234, subsequence, 0) is in
-// code/mc_gpu.cu:99 (own seed scramble, subsequence = the reference's product
-// (idx+1)(stream+1)(v+1)(1+gpu)ystart, jump 2^67 per subsequence); the run
-// starting at bundle h0 jumps h0*draws_per_bundle further.  Sobol points are
-// v*photmax + h (the Sobol states restart per cell, :79-82).
+// State n steps into the stream: A^n = sum of c_i A^i, i < 160, with
+// c = x^n modulo A's characteristic polynomial (the host's table), so the
+// state is the sum of the c_i = 1 states of the sequence y.
+__device__ __forceinline__ Xorwow xorwow_jump(const uint32_t* y, const uint32_t* poly, uint32_t d0, uint32_t n)
+{
+    uint32_t r[5] = {0, 0, 0, 0, 0}, c[5];
+#pragma unroll
+    for (int w = 0; w < 5; ++w) c[w] = poly[w];
+    uint4 lo = *(const uint4*)y;
+#pragma unroll 1
+    for (int j = 0; j < 5; ++j) {
+#pragma unroll
+        for (int i = 0; i < 32; i += 4) {
+            const uint4 hi = *(const uint4*)(y + 32 * j + i + 4);
+            const uint32_t q[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const uint32_t m = (uint32_t)((int32_t)(c[0] << (31 - (i + b))) >> 31);
+#pragma unroll
+                for (int w = 0; w < 5; ++w) r[w] = __builtin_amdgcn_bitop3_b32(m, q[b + w], r[w], 0x6A);   // r ^ (m & q)
+            }
+            lo = hi;
+        }
+        c[0] = c[1]; c[1] = c[2]; c[2] = c[3]; c[3] = c[4];
+    }
+    return Xorwow{r[0], r[1], r[2], r[3], r[4], d0 + 362437u * n};
+}
+
+// One block per slot, the bundles in runs of run_len consecutive ones per
+// thread (at most one run each).  The Sobol points are v*photmax + h (the Sobol
+// states restart per cell, :79-82).  Descriptors are staged in LDS, kStage
+// bundles of every run at a time, and leave in pieces of 64 (32) bytes; the
+// weights of the slot's (band, g) bins are computed once where a slot has at
+// least as many bundles as bins.
+//
+// Before, each thread of 256 bundles multiplied the seed by its subsequence's
+// and offset's matrices alone, 160 columns of five words at a time.  A solve of
+// 9216 slots of 1019 bundles went from 1.76 to 1.06 ms with this kernel.
 __global__ __launch_bounds__(256) void raygen_compat(GenArgs a)
 {
-    extern __shared__ float lds[];
-    float* s_cdfb = lds;
-    float* s_cdfg = s_cdfb + a.nB;
-    float* s_ib = s_cdfg + a.nB * a.nQ;
-    uint32_t* s_sob = (uint32_t*)(s_ib + ((a.spec == kSpecTable && a.nB * a.nT <= 16384) ? a.nB * a.nT : 0));
-    const bool ib_lds = a.spec == kSpecTable && a.nB * a.nT <= 16384;
-    for (int i = threadIdx.x; i < a.nB; i += blockDim.x) s_cdfb[i] = a.cdf_band[i];
-    for (int i = threadIdx.x; i < a.nB * a.nQ; i += blockDim.x) s_cdfg[i] = a.cdf_g[i];
-    if (ib_lds)
-        for (int i = threadIdx.x; i < a.nB * a.nT; i += blockDim.x) s_ib[i] = a.Ib[i];
-    for (int i = threadIdx.x; i < 64; i += blockDim.x) s_sob[i] = a.sobol_v[i];
-    __syncthreads();
-    const float* ibt = ib_lds ? s_ib : a.Ib;
-    const int runs = (a.rays_per_slot + a.sub_len - 1) / a.sub_len;
-    const long long nthreads = a.nslots * runs;
-    for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < nthreads; t += (long long)gridDim.x * blockDim.x) {
-        long long sl = t / runs;
-        int run = (int)(t - sl * runs);
-        const int4 si = a.slotinfo[a.slot0 + sl];
-        const int cell = si.y;
-        const int v = si.x % a.slots_per_emitter;
-        Xorwow s = compat_stream(a, cell, v);
-        int h0 = run * a.sub_len;
-        xorwow_skip(a, s, (uint64_t)h0 * (uint64_t)a.draws_per_bundle);
-        int h1 = h0 + a.sub_len < a.rays_per_slot ? h0 + a.sub_len : a.rays_per_slot;
-        uint64_t n = (uint64_t)v * (uint64_t)a.rays_per_slot + (uint64_t)h0;
-        uint32_t sx0 = sobol_at(s_sob, n), sx1 = sobol_at(s_sob + 32, n);
-        float Ti = a.T0[(size_t)a.snap * a.tstride0 + si.z];
-        for (int h = h0; h < h1; ++h) {
-            uint32_t mp, mt;
-            if (a.use_sobol) {
-                mp = sx0 >> 8;
-                mt = sx1 >> 8;
-                int c = __builtin_ctzll(~n);
-                sx0 ^= s_sob[c];
-                sx1 ^= s_sob[32 + c];
-                ++n;
-            } else {
-                mp = xorwow_next(s) >> 8;
-                mt = xorwow_next(s) >> 8;
-            }
-            int band = cdf_search(s_cdfb, a.nB, u01_incl(xorwow_next(s)));
-            int g = 0;
-            if (a.g_search) g = cdf_search(s_cdfg + band * a.nQ, a.nQ, u01_incl(xorwow_next(s)));
-            g = g > a.nQ - 1 ? a.nQ - 1 : g;
-            float w, winv;
-            bundle_weight(a, ibt, Ti, band, g, &w, &winv);
-            uint32_t w0, w1;
-            desc_pack(mt, mp, band, g, &w0, &w1);
-            long long q = sl * a.rays_per_slot + h;
-            a.w0[q] = w0;
-            a.w1[q] = w1;
-            a.w[q] = w;
-            a.winv[q] = winv;
-        }
-    }
-}
-
-// Sorted compat generation (srt == 1: code/mc_gpu.cu:100-102, :138-139).  The
-// reference draws all photmax (band, g) pairs of the slot's stream first and
-// counts them (kernel_find, :786-812), then replays the counts position by
-// position of the kavg band order, g ascending inside a band (wave_find,
-// :897-930), drawing each bundle's direction in the photon loop.  Bundles with
-// the same (band, g) are interchangeable until a direction is attached, so
-// the replay is a histogram and a scan: one block per slot,
-//  (1) each thread jumps to its run of (band, g) draws and counts them in LDS,
-//  (2) the histogram is scanned in replay order (position p, then g),
-//  (3) bundle h takes the bin where the running count first exceeds h, and its
-//      direction is Sobol point v*photmax + h, or XORWOW uniforms
-//      draws_find*photmax + 2h (phi) and + 2h + 1 (theta) of the stream.
-// The reference permutes its tables into the sorted order, so position p
-// carries band band_order[p]; the descriptor holds that band.
-__global__ __launch_bounds__(256) void raygen_compat_sorted(GenArgs a)
-{
-    extern __shared__ float lds[];
-    __shared__ uint32_t s_part[256];
-    const int nbin = a.nB * a.nQ;
-    float* s_cdfb = lds;
-    float* s_cdfg = s_cdfb + a.nB;
-    uint32_t* s_sob = (uint32_t*)(s_cdfg + nbin);
-    int* s_ord = (int*)(s_sob + 64);
-    uint32_t* s_hist = (uint32_t*)(s_ord + a.nB);
-    uint32_t* s_cum = s_hist + nbin;
-    const int tid = threadIdx.x, nth = blockDim.x;
-    for (int i = tid; i < a.nB; i += nth) {
-        s_cdfb[i] = a.cdf_band[i];
-        s_ord[i] = a.band_order[i];
-    }
-    for (int i = tid; i < nbin; i += nth) {
-        s_cdfg[i] = a.cdf_g[i];
-        s_hist[i] = 0u;
-    }
+    extern __shared__ __align__(16) float lds[];
+    const int nbin = a.nB * a.nQ, tid = threadIdx.x, nth = blockDim.x;
+    const int R = a.rays_per_slot, L = a.run_len;
+    const int st = L < 16 ? 8 : 16, sh = L < 16 ? 3 : 4;   // staged bundles per run (divides L)
+    uint32_t* s_y = (uint32_t*)lds;
+    uint32_t* s_sob = s_y + kXwSeq;
+    uint32_t* s_w0 = s_sob + 64;
+    uint32_t* s_w1 = s_w0 + nth * (st + 1);
+    float* s_cdfb = (float*)(s_w1 + nth * (st + 1));
+    float* s_iib = s_cdfb + a.nB;
+    float* s_bw = s_iib + a.nB;                            // weight of each bin (bin_weights)
+    float* s_cdfg = s_bw + (a.bin_weights ? nbin : 0);
+    const float* cdfg = a.cdf_lds ? s_cdfg : a.cdf_g;
+    for (int i = tid; i < a.nB; i += nth) s_cdfb[i] = a.cdf_band[i];
+    if (a.cdf_lds)
+        for (int i = tid; i < nbin; i += nth) s_cdfg[i] = a.cdf_g[i];
     for (int i = tid; i < 64; i += nth) s_sob[i] = a.sobol_v[i];
-    __syncthreads();
-    const int R = a.rays_per_slot;
-    const int L = (R + nth - 1) / nth;
-    const int h0 = tid * L < R ? tid * L : R;
-    const int h1 = h0 + L < R ? h0 + L : R;
+    const int h0 = tid * L;
     for (long long sl = blockIdx.x; sl < a.nslots; sl += gridDim.x) {
         const int4 si = a.slotinfo[a.slot0 + sl];
         const int cell = si.y;
         const int v = si.x % a.slots_per_emitter;
-        const Xorwow s0 = compat_stream(a, cell, v);
-        // (1) histogram of the (band, g) draws h0..h1-1
-        if (h0 < h1) {
-            Xorwow s = s0;
-            xorwow_skip(a, s, (uint64_t)h0 * (uint64_t)a.draws_find);
-            for (int h = h0; h < h1; ++h) {
-                int band = cdf_search(s_cdfb, a.nB, u01_incl(xorwow_next(s)));
-                int g = 0;
-                if (a.g_search) g = cdf_search(s_cdfg + band * a.nQ, a.nQ, u01_incl(xorwow_next(s)));
-                g = g > a.nQ - 1 ? a.nQ - 1 : g;
-                atomicAdd(&s_hist[band * a.nQ + g], 1u);
+        const float Ti = a.T0[(size_t)a.snap * a.tstride0 + si.z];
+        if (tid < 64) compat_sequence(a, cell, v, tid, s_y);
+        if (a.bin_weights)
+            for (int k = tid; k < nbin; k += nth) {
+                const int band = (int)fdiv((uint32_t)k, a.fd_nQ), g = k - band * a.nQ;
+                float w, winv, iib;
+                bundle_weight(a, a.Ib, Ti, band, g, &w, &winv, &iib);
+                s_bw[k] = w;
+                if (g == 0) s_iib[band] = iib;
             }
-        }
         __syncthreads();
-        // (2) inclusive scan in replay order: entry k = p*nQ + g counts bin order[p]*nQ + g
-        const int per = (nbin + nth - 1) / nth;
-        const int k0 = tid * per < nbin ? tid * per : nbin;
-        const int k1 = k0 + per < nbin ? k0 + per : nbin;
-        uint32_t run = 0;
-        for (int k = k0; k < k1; ++k) {
-            const int p = k / a.nQ, g = k - p * a.nQ;
-            run += s_hist[s_ord[p] * a.nQ + g];
-        }
-        s_part[tid] = run;
-        __syncthreads();
-        for (int o = 1; o < nth; o <<= 1) {
-            uint32_t add = tid >= o ? s_part[tid - o] : 0u;
-            __syncthreads();
-            s_part[tid] += add;
-            __syncthreads();
-        }
-        run = tid > 0 ? s_part[tid - 1] : 0u;
-        for (int k = k0; k < k1; ++k) {
-            const int p = k / a.nQ, g = k - p * a.nQ;
-            run += s_hist[s_ord[p] * a.nQ + g];
-            s_cum[k] = run;
-        }
-        __syncthreads();
-        // (3) bundles h0..h1-1
-        if (h0 < h1) {
-            int lo = 0, hi = nbin - 1;             // first k with s_cum[k] > h0 (s_cum[nbin-1] == R)
-            while (lo < hi) {
-                const int mid = (lo + hi) >> 1;
-                if (s_cum[mid] > (uint32_t)h0) hi = mid; else lo = mid + 1;
-            }
-            int k = lo;
-            Xorwow s = s0;
-            uint64_t n = (uint64_t)v * (uint64_t)R + (uint64_t)h0;
-            uint32_t sx0 = 0, sx1 = 0;
+        Xorwow s{0, 0, 0, 0, 0, 0};
+        uint32_t sx0 = 0, sx1 = 0;
+        uint64_t n = (uint64_t)v * (uint64_t)R + (uint64_t)h0;
+        if (h0 < R) {
+            s = xorwow_jump(s_y, a.xw_poly + 5 * tid, a.xw_seed[5], (uint32_t)h0 * (uint32_t)a.draws_per_bundle);
             if (a.use_sobol) {
                 sx0 = sobol_at(s_sob, n);
                 sx1 = sobol_at(s_sob + 32, n);
-            } else {
-                xorwow_skip(a, s, (uint64_t)R * (uint64_t)a.draws_find + 2ull * (uint64_t)h0);
             }
-            const float Ti = a.T0[(size_t)a.snap * a.tstride0 + si.z];
-            for (int h = h0; h < h1; ++h) {
+        }
+        for (int b0 = 0; b0 < L; b0 += st) {
+            if (b0 > 0) __syncthreads();
+            for (int i = 0; i < st && h0 + b0 + i < R; ++i) {
                 uint32_t mp, mt;
                 if (a.use_sobol) {
                     mp = sx0 >> 8;
@@ -329,24 +269,207 @@ __global__ __launch_bounds__(256) void raygen_compat_sorted(GenArgs a)
                     mp = xorwow_next(s) >> 8;
                     mt = xorwow_next(s) >> 8;
                 }
-                while (s_cum[k] <= (uint32_t)h) ++k;
-                const int p = k / a.nQ, g = k - p * a.nQ;
-                const int band = s_ord[p];
-                float w, winv;
-                bundle_weight(a, a.Ib, Ti, band, g, &w, &winv);
-                uint32_t w0, w1;
-                desc_pack(mt, mp, band, g, &w0, &w1);
-                const long long q = sl * R + h;
-                a.w0[q] = w0;
-                a.w1[q] = w1;
-                a.w[q] = w;
-                a.winv[q] = winv;
+                int band = cdf_search(s_cdfb, a.nB, u01_incl(xorwow_next(s)));
+                int g = 0;
+                if (a.g_search) g = cdf_search(cdfg + band * a.nQ, a.nQ, u01_incl(xorwow_next(s)));
+                g = g > a.nQ - 1 ? a.nQ - 1 : g;
+                desc_pack(mt, mp, band, g, &s_w0[tid * (st + 1) + i], &s_w1[tid * (st + 1) + i]);
+            }
+            __syncthreads();
+            for (int e = tid; e < nth << sh; e += nth) {
+                const int t = e >> sh, i = e & (st - 1), h = t * L + b0 + i;
+                if (h < R) {
+                    const uint32_t w0 = s_w0[t * (st + 1) + i], w1 = s_w1[t * (st + 1) + i];
+                    const int band = desc_band(w0, w1), g = desc_g(w1);
+                    float w, winv, iib;
+                    if (a.bin_weights) {
+                        w = s_bw[band * a.nQ + g];
+                        winv = w * s_iib[band];
+                    } else {
+                        bundle_weight(a, a.Ib, Ti, band, g, &w, &winv, &iib);
+                    }
+                    const long long q = sl * R + h;
+                    a.w0[q] = w0;
+                    a.w1[q] = w1;
+                    a.w[q] = w;
+                    a.winv[q] = winv;
+                }
             }
         }
-        // the next slot reuses the histogram
+        __syncthreads();   // the next slot's sequence and weights
+    }
+}
+
+// Sorted compat generation (srt == 1: code/mc_gpu.cu:100-102, :138-139).  The
+// reference draws all photmax (band, g) pairs of the slot's stream first and
+// counts them (kernel_find, :786-812), then replays the counts position by
+// position of the kavg band order, g ascending inside a band (wave_find,
+// :897-930), drawing each bundle's direction in the photon loop.  Bundles with
+// the same (band, g) are interchangeable until a direction is attached, so
+// the replay is a histogram and a scan: one block per slot,
+//  (1) each thread jumps to its run of (band, g) draws and counts them in LDS,
+//  (2) the histogram is scanned in replay order (position p, then g), and each
+//      drawn bin's weights take the place of its count and CDF entry,
+//  (3) bundle h takes the bin where the running count first exceeds h, and its
+//      direction is Sobol point v*photmax + h, or XORWOW uniforms
+//      draws_find*photmax + 2h (phi) and + 2h + 1 (theta) of the stream.
+// The reference permutes its tables into the sorted order, so position p
+// carries band band_order[p]; the descriptor holds that band.
+//
+// (3) gives each wave 64 consecutive bundles at a time, so the four arrays are
+// written in whole lines, and finds the bins by walking the running counts, a
+// lane each, once for the 64.  With Sobol directions the 64 start at a multiple
+// of 64 of the sequence: a point is then the exclusive or of the wave's (one
+// step per 64) and the lane's (constant) part.
+//
+// 3.7e8 bundles of 18432 slots (100 bands x 16 g): 20.9 -> 3.2 ms (the 16 B per
+// bundle alone 1 ms; instruction issue and the two CDF searches' LDS reads bound
+// it).  Before, every thread multiplied its slot's seed by the subsequence's and
+// its offset's bit matrices alone, weights were computed and tables gathered per
+// bundle, and the lanes of a wave wrote 64 different lines.  Seven blocks per CU
+// (LDS) against five and six with more registers: 3.2, 4.1 and 4.1 ms.
+__global__ __launch_bounds__(256, 7) void raygen_compat_sorted(GenArgs a)
+{
+    extern __shared__ __align__(16) float lds[];
+    __shared__ __align__(16) uint32_t s_part[256];   // the slot's sequence; the scan's wave sums after
+    const int nbin = a.nB * a.nQ;
+    float* s_cdfb = lds;
+    float* s_cdfg = s_cdfb + a.nB;                   // w / Ib of the drawn bins in (3)
+    uint32_t* s_sob = (uint32_t*)(s_cdfg + nbin);
+    int* s_ord = (int*)(s_sob + 64);
+    uint32_t* s_hist = (uint32_t*)(s_ord + a.nB);    // w of the drawn bins in (3)
+    uint32_t* s_cum = s_hist + nbin;
+    const int tid = threadIdx.x, nth = blockDim.x, lane = tid & 63, wv = tid >> 6;
+    for (int i = tid; i < a.nB; i += nth) {
+        s_cdfb[i] = a.cdf_band[i];
+        s_ord[i] = a.band_order[i];
+    }
+    for (int i = tid; i < nbin; i += nth) {
+        s_cdfg[i] = a.cdf_g[i];
+        s_hist[i] = 0u;
+    }
+    for (int i = tid; i < 64; i += nth) s_sob[i] = a.sobol_v[i];
+    __syncthreads();
+    const int R = a.rays_per_slot, L = a.run_len;
+    const int h0 = tid * L < R ? tid * L : R;
+    const int h1 = h0 + L < R ? h0 + L : R;
+    const uint32_t xr0 = sobol_at(s_sob, lane), xr1 = sobol_at(s_sob + 32, lane);
+    for (long long sl = blockIdx.x; sl < a.nslots; sl += gridDim.x) {
+        const int4 si = a.slotinfo[a.slot0 + sl];
+        const int cell = si.y;
+        const int v = si.x % a.slots_per_emitter;
+        const float Ti = a.T0[(size_t)a.snap * a.tstride0 + si.z];
+        const long long q0 = sl * R;
+        if (wv == 0) compat_sequence(a, cell, v, lane, s_part);
         __syncthreads();
-        for (int i = tid; i < nbin; i += nth) s_hist[i] = 0u;
+        // (1) histogram of the (band, g) draws h0..h1-1
+        if (h0 < h1) {
+            Xorwow s = xorwow_jump(s_part, a.xw_poly + 5 * tid, a.xw_seed[5], (uint32_t)h0 * (uint32_t)a.draws_find);
+            for (int h = h0; h < h1; ++h) {
+                int band = cdf_search(s_cdfb, a.nB, u01_incl(xorwow_next(s)));
+                int g = 0;
+                if (a.g_search) g = cdf_search(s_cdfg + band * a.nQ, a.nQ, u01_incl(xorwow_next(s)));
+                g = g > a.nQ - 1 ? a.nQ - 1 : g;
+                atomicAdd(&s_hist[band * a.nQ + g], 1u);
+            }
+            if (!a.use_sobol) {   // the directions' 24-bit uniforms, taken up again in (3)
+                s = xorwow_jump(s_part, a.xw_poly + 5 * (256 + tid), a.xw_seed[5],
+                                (uint32_t)R * (uint32_t)a.draws_find + 2u * (uint32_t)h0);
+                for (int h = h0; h < h1; ++h) {
+                    a.w1[q0 + h] = xorwow_next(s) >> 8;
+                    a.w0[q0 + h] = xorwow_next(s) >> 8;
+                }
+            }
+        }
         __syncthreads();
+        // (2) inclusive scan in replay order: entry k = p*nQ + g counts bin order[p]*nQ + g
+        const int per = (nbin + nth - 1) / nth;
+        const int k0 = tid * per < nbin ? tid * per : nbin;
+        const int k1 = k0 + per < nbin ? k0 + per : nbin;
+        const int p0 = (int)fdiv((uint32_t)k0, a.fd_nQ), g0 = k0 - p0 * a.nQ;
+        uint32_t run = 0;
+        for (int k = k0, p = p0, g = g0; k < k1; ++k) {
+            run += s_hist[s_ord[p] * a.nQ + g];
+            if (++g == a.nQ) { g = 0; ++p; }
+        }
+        uint32_t inc = run;
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t t = __shfl_up(inc, o);
+            inc += lane >= o ? t : 0u;
+        }
+        if (lane == 63) s_part[wv] = inc;
+        __syncthreads();
+        inc -= run;
+        for (int w = 0; w < wv; ++w) inc += s_part[w];
+        for (int k = k0, p = p0, g = g0; k < k1; ++k) {
+            const int band = s_ord[p], bin = band * a.nQ + g;
+            const uint32_t cnt = s_hist[bin];
+            inc += cnt;
+            s_cum[k] = inc;
+            if (cnt) {
+                float w, winv, iib;
+                bundle_weight(a, a.Ib, Ti, band, g, &w, &winv, &iib);
+                s_hist[bin] = __float_as_uint(w);
+                s_cdfg[bin] = winv;
+            }
+            if (++g == a.nQ) { g = 0; ++p; }
+        }
+        __syncthreads();
+        // (3) bundles in chunks of 64 from n0 rounded down to a multiple of 64
+        {
+            const uint64_t n0 = (uint64_t)v * (uint64_t)R;
+            const int lead = a.use_sobol ? (int)(n0 & 63ull) : 0;
+            const int nch = (int)(((long long)lead + R + 63) / 64);
+            const int c0 = (int)((long long)wv * nch / 4), c1 = (int)((long long)(wv + 1) * nch / 4);
+            const int hf = max(64 * c0 - lead, 0);
+            int lo = 0, hi = nbin - 1;             // first k with s_cum[k] > hf (s_cum[nbin-1] == R)
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (s_cum[mid] > (uint32_t)hf) hi = mid; else lo = mid + 1;
+            }
+            int kc = __builtin_amdgcn_readfirstlane(lo);
+            uint64_t nb = n0 - (uint64_t)lead + 64ull * (uint64_t)c0;
+            uint32_t x0 = sobol_at(s_sob, nb), x1 = sobol_at(s_sob + 32, nb);
+            for (int c = c0; c < c1; ++c) {
+                const int h = 64 * c - lead + lane, hl = min(64 * c - lead + 63, R - 1);
+                int k = kc;                        // the first k with s_cum[k] > h
+                for (bool more = true; more;) {
+                    const int cl = (int)s_cum[min(kc + lane, nbin - 1)];
+                    int i = 0;
+                    for (; i < 64; ++i) {
+                        const int ci = __builtin_amdgcn_readlane(cl, i);
+                        if (ci > hl) break;
+                        k += h >= ci ? 1 : 0;
+                    }
+                    more = i == 64;
+                    kc += i;
+                }
+                const uint32_t mp = (x0 ^ xr0) >> 8, mt = (x1 ^ xr1) >> 8;
+                if (h >= 0 && h < R) {
+                    const long long q = q0 + h;
+                    const int p = (int)fdiv((uint32_t)k, a.fd_nQ), g = k - p * a.nQ;
+                    const int band = s_ord[p], bin = band * a.nQ + g;
+                    uint32_t w0, w1;
+                    if (a.use_sobol) desc_pack(mt, mp, band, g, &w0, &w1);
+                    else desc_pack(a.w0[q], a.w1[q], band, g, &w0, &w1);
+                    a.w0[q] = w0;
+                    a.w1[q] = w1;
+                    a.w[q] = __uint_as_float(s_hist[bin]);
+                    a.winv[q] = s_cdfg[bin];
+                }
+                // Gray code of nb -> nb + 64: bits 5 and 6 + (trailing ones of nb / 64) change
+                const int t = 6 + __builtin_ctzll(~(nb >> 6));
+                x0 ^= s_sob[5] ^ (t < 32 ? s_sob[t] : 0u);
+                x1 ^= s_sob[37] ^ (t < 32 ? s_sob[32 + t] : 0u);
+                nb += 64;
+            }
+        }
+        // the next slot's histogram and CDFs
+        __syncthreads();
+        for (int i = tid; i < nbin; i += nth) {
+            s_hist[i] = 0u;
+            s_cdfg[i] = a.cdf_g[i];
+        }
     }
 }
 

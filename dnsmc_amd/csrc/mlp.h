@@ -48,7 +48,7 @@ struct MlpWeights {
     int nbin, noutp;
     // the same W2 and W3 with the input index contiguous ([64][64] and
     // [noutp][64]), for the proposal kernel's MFMA operand tiles (set by the
-    // solver; the training kernels do not use them)
+    // solver; training transposes W3 itself)
     const uint16_t* W2T;
     const uint16_t* W3T;
 };

@@ -148,9 +148,9 @@ __device__ __forceinline__ void put_w3_tile(const uint4& r0, const uint4& r1, ui
 // for the rows, two blocks per CU, bound by the exponentials and LDS reads of
 // the two passes over W3's columns, 27 us for dW3, 11 us for the sums).  Every
 // sum over rows, columns and blocks below W3 keeps the first form's order, so
-// those gradients are bit for bit what they were.  dZ leaves the logits' accumulators in the layout of the
-// next product's second operand (rows 4 (l / 16) + i, column l % 16), so
-// dW3 = H2^T dZ takes it from registers.
+// those gradients are bit for bit what they were.  dZ leaves the logits'
+// accumulators in the layout of the next product's operand (rows
+// 4 (l / 16) + i, column l % 16), so dW3 = H2^T dZ takes it from registers.
 
 // Four BF16 of consecutive k as an MFMA operand, from an 8-byte aligned address.
 __device__ __forceinline__ s4v frag8(const uint16_t* p)

@@ -209,8 +209,9 @@ struct dnsmc_solver {
     DevBuf<int> d_band_order;   // sorted compat mode
     DevBuf<double> d_inv_emax_d;
     // compat
-    DevBuf<uint32_t> d_xw_sub, d_xw_off, d_sobol;
+    DevBuf<uint32_t> d_xw_sub, d_xw_poly, d_sobol;
     bool compat_ready = false;
+    int compat_key = 0;   // what d_xw_poly was made for
     // emitters
     std::vector<int> emit;
     std::vector<int> order;     // processing position -> emitter, 3-D brick order
@@ -520,34 +521,33 @@ static int ensure_derived(dnsmc_solver* s, float Tmax, const NoAlloc* na)
     return DNSMC_OK;
 }
 
+// Bundles per generator thread of the compat generators: one run per thread of
+// a block of at most 256, a multiple of 8 (16 from 2048 bundles) where they are
+// staged.
+static int compat_run_len(bool sorted, int R)
+{
+    if (sorted) return std::max(4, (int)(((long long)R + 255) / 256));
+    return R <= 2048 ? 8 : 16 * (int)(((long long)R + 4095) / 4096);
+}
+
 static int ensure_compat(dnsmc_solver* s)
 {
-    if (s->compat_ready) return DNSMC_OK;
-    std::vector<uint32_t> sub, off;
-    xorwow_jump_tables(sub);
-    // offsets: M^(2^j), j < 64
-    {
-        std::vector<uint32_t> m(160 * 5), t(160 * 5);
-        for (int b = 0; b < 160; ++b) {
-            Xorwow x{0, 0, 0, 0, 0, 0};
-            uint32_t* w = &x.x0;
-            w[b >> 5] = 1u << (b & 31);
-            (void)xorwow_next(x);
-            m[b * 5 + 0] = x.x0; m[b * 5 + 1] = x.x1; m[b * 5 + 2] = x.x2; m[b * 5 + 3] = x.x3; m[b * 5 + 4] = x.x4;
-        }
-        off.assign((size_t)64 * 800, 0u);
-        for (int j = 0; j < 64; ++j) {
-            std::copy(m.begin(), m.end(), off.begin() + (size_t)j * 800);
-            for (int b = 0; b < 160; ++b) {   // square
-                uint32_t r[5] = {0, 0, 0, 0, 0};
-                for (int c = 0; c < 160; ++c)
-                    if ((m[b * 5 + (c >> 5)] >> (c & 31)) & 1u)
-                        for (int w = 0; w < 5; ++w) r[w] ^= m[c * 5 + w];
-                for (int w = 0; w < 5; ++w) t[b * 5 + w] = r[w];
-            }
-            m.swap(t);
-        }
+    const dnsmc_config& c = s->cfg;
+    const uint64_t R = (uint64_t)c.photmax, find = 1u + (s->der.g_search ? 1u : 0u);
+    const uint64_t L = (uint64_t)compat_run_len(s->der.sorted, c.photmax);
+    const int key = (int)find | (s->der.sorted ? 4 : 0);   // (photmax and sobol are the solver's own)
+    if (s->compat_ready && s->compat_key == key) return DNSMC_OK;
+    std::vector<uint32_t> sub, poly;
+    if (s->der.sorted) {
+        xorwow_jump_polys(0, L * find, 256, poly);
+        if (!c.sobol) xorwow_jump_polys(R * find, 2 * L, 256, poly);
+    } else {
+        xorwow_jump_polys(0, L * (find + (c.sobol ? 0u : 2u)), 256, poly);
     }
+    HIPCHK(s->d_xw_poly.upload(poly, s->stream));
+    s->compat_key = key;
+    if (s->compat_ready) return DNSMC_OK;
+    xorwow_jump_tables(sub);
     std::vector<uint32_t> sob(64);
     for (int k = 1; k <= 32; ++k) sob[k - 1] = 1u << (32 - k);   // dimension 0 (van der Corput)
     uint32_t mk = 1u;                                           // dimension 1: s=1, a=0, m1=1
@@ -556,7 +556,6 @@ static int ensure_compat(dnsmc_solver* s)
         sob[32 + k - 1] = mk << (32 - k);
     }
     HIPCHK(s->d_xw_sub.upload(sub, s->stream));
-    HIPCHK(s->d_xw_off.upload(off, s->stream));
     HIPCHK(s->d_sobol.upload(sob, s->stream));
     s->compat_ready = true;
     return DNSMC_OK;
@@ -1096,11 +1095,12 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     if (c.mode == DNSMC_MODE_COMPAT) {
         xorwow_seed_state(c.seed, G.xw_seed);
         G.xw_jump_sub = s->d_xw_sub.p;
-        G.xw_jump_off = s->d_xw_off.p;
+        G.xw_poly = s->d_xw_poly.p;
         G.sobol_v = s->d_sobol.p;
         G.use_sobol = c.sobol;
         G.draws_per_bundle = (c.sobol ? 0 : 2) + 1 + (d.g_search ? 1 : 0);
-        G.sub_len = 256;
+        G.run_len = compat_run_len(d.sorted, c.photmax);
+        G.fd_nQ = make_fastdiv((uint32_t)d.nQ);
         G.n0 = c.n[0]; G.n1 = c.n[1]; G.n2 = c.n[2];
         G.num_streams = c.num_streams; G.num_gpu = c.num_gpu; G.gpu = c.gpu; G.p_row = c.p_row;
         G.ystart = s->ystart;
@@ -1111,6 +1111,20 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     const size_t lds_gen = sizeof(float) * ((size_t)d.nB + (size_t)d.nB * d.nQ + (gib ? (size_t)d.nB * d.nT : 0) + 64);
     const bool sorted = c.mode == DNSMC_MODE_COMPAT && d.sorted;
     const size_t lds_sorted = sizeof(float) * (2 * (size_t)d.nB + 3 * (size_t)d.nB * d.nQ + 64);
+    if (c.mode == DNSMC_MODE_COMPAT && !sorted && lds_gen > s->lds_max)
+        return fail(DNSMC_EDEVICE, "reference sampling: too many (band, g) bins for the proposal's CDFs in LDS");
+    const int compat_threads = std::min(256, (c.photmax + 64 * std::max(1, G.run_len) - 1) / (64 * std::max(1, G.run_len)) * 64);
+    size_t lds_compat = 0;
+    if (c.mode == DNSMC_MODE_COMPAT && !sorted) {
+        // the slot's weights per bin while three blocks of 256 threads stay on a
+        // CU; the CDFs from memory only where the staging leaves them no room
+        const size_t nbin = (size_t)d.nB * d.nQ;
+        lds_compat = sizeof(float) * (kXwSeq + 64 + 2 * (size_t)compat_threads * (G.run_len < 16 ? 9 : 17) + 2 * (size_t)d.nB);
+        G.cdf_lds = lds_compat + sizeof(float) * nbin <= s->lds_max;
+        if (G.cdf_lds) lds_compat += sizeof(float) * nbin;
+        G.bin_weights = G.cdf_lds && (size_t)R >= nbin && lds_compat + sizeof(float) * nbin <= s->lds_max / 3;
+        if (G.bin_weights) lds_compat += sizeof(float) * nbin;
+    }
     if (sorted && lds_sorted + 1024 > s->lds_max)
         return fail(DNSMC_EINVAL, "sorted mode: too many (band, g) bins for the per-block histogram");
     size_t lds_learn = 0;
@@ -1331,12 +1345,13 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
                 HIPCHK(hipGetLastError());
                 HIPCHK(launch_raygen_learned(s, G, nsl, R, st, (const float*)pp.d_qcdf.p, (const float*)s->d_pcdf.p));
             } else if (sorted) {
-                int nb = (int)std::min<long long>(nsl, (long long)s->ncu * 8);
+                const long long per = std::max<long long>(1, std::min<long long>(8, (long long)(s->lds_max / (lds_sorted + 1024))));
+                int nb = (int)std::min<long long>(nsl, s->ncu * per);
                 hipLaunchKernelGGL(raygen_compat_sorted, dim3(nb), dim3(256), lds_sorted, st, G);
             } else if (c.mode == DNSMC_MODE_COMPAT) {
-                long long nth = nsl * ((R + G.sub_len - 1) / G.sub_len);
-                int nb = (int)std::min<long long>((nth + 255) / 256, 1 << 20);
-                hipLaunchKernelGGL(raygen_compat, dim3(nb), dim3(256), lds_gen, st, G);
+                const long long per = std::max<long long>(1, std::min<long long>(2048 / compat_threads, (long long)(s->lds_max / lds_compat)));
+                int nb = (int)std::min<long long>(nsl, s->ncu * per);
+                hipLaunchKernelGGL(raygen_compat, dim3(nb), dim3(compat_threads), lds_compat, st, G);
             } else {
                 int nb = (int)std::min<long long>((nr + 255) / 256, (long long)s->ncu * 64);
                 hipLaunchKernelGGL(raygen_plain, dim3(nb), dim3(256), lds_gen, st, G);

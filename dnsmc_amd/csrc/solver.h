@@ -71,6 +71,10 @@ void spline_axis_coeffs(const std::vector<float>& xf_centres, int nf, const std:
 
 // XORWOW jump matrices: M^(2^(67+j)) for j in [0, 60), each 160 columns x 5 words.
 void xorwow_jump_tables(std::vector<uint32_t>& out);
+// Jumps by base + i*step draws, i < count, as x^n modulo the characteristic
+// polynomial of the XORWOW step matrix, appended to out: 5 words each, bit j of
+// the 160 the coefficient of x^j.
+void xorwow_jump_polys(uint64_t base, uint64_t step, int count, std::vector<uint32_t>& out);
 void xorwow_seed_state(uint64_t seed, uint32_t st[6]);
 
 }  // namespace dn
