@@ -1899,8 +1899,8 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
 // FP64 oracle computes it.  Direction from the descriptor's 24-bit uniforms,
 // table lookups interpolated in FP64 from the FP32 tables, FP64 optical depth,
 // transmissivity and gathered emission, bundle weights recomputed in FP64:
-// w = Ibmax (k_i Ib_i) / (k_max Ib_max), E = w D, A = w G / Ib_i.  One thread
-// per ray (grid-stride); each ray's (E, A) goes to pray64 for reduce_rays64.
+// w = Ibmax (k_i Ib_i) / (k_max Ib_max), E = w D, A = w G / Ib_i; each ray's
+// (E, A) goes to pray64 for reduce_rays64.
 __device__ __forceinline__ void lookup_f64(const TraceArgs& P, double Tj, int bg, int band, double* kap, double* ib)
 {
     double pos = Tj * (double)P.inv_dT + (double)P.mT0;
@@ -1915,8 +1915,37 @@ __device__ __forceinline__ void lookup_f64(const TraceArgs& P, double Tj, int bg
     *ib = (double)ir[t0] + fr * ((double)ir[t0 + 1] - (double)ir[t0]);
 }
 
+template <int CTRL>
+__device__ __forceinline__ double quad_d(double v)
+{
+    const int2 u = __builtin_bit_cast(int2, v);
+    return __builtin_bit_cast(double, make_int2(quad_i<CTRL>(u.x), quad_i<CTRL>(u.y)));
+}
+__device__ __forceinline__ double min_f64(double x, double y)   // (no NaN)
+{
+    double r;
+    asm("v_min_f64 %0, %1, %2" : "=v"(r) : "v"(x), "v"(y));
+    return r;
+}
+__device__ __forceinline__ double quad_min_d(double v)
+{
+    v = min_f64(v, quad_d<kQuadXor1>(v));
+    return min_f64(v, quad_d<kQuadXor2>(v));
+}
+
+// Work: waves claim `super` consecutive rays at a time and start new ones when
+// 16 lanes are idle.  The drain below is the FP32 traversal's: when nothing is
+// left to hand out and at most 16 of a wave's rays run on, all on the last
+// level, four lanes follow a ray, kDrain crossings ahead, with the loop's
+// arithmetic and order (a crossing past the ray's end has length 0).
+//
+// Such a launch waits for its longest ray: one crossing after another takes
+// about 700 ns here (faces, field, table and exponential one behind the other).
+// 1024 cells x 8192 rays of a 64x96x64 channel, 9.1e7 crossings, longest ray
+// 16000: 12.1 ms with a thread per ray, 4.0 ms with the drain (the bulk about
+// 1 ms of it).
 template <int SPEC, bool REC>
-__global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
+__global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64, int super)
 {
     extern __shared__ float lds[];
     int* s_lev = (int*)lds;
@@ -1929,6 +1958,8 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
         L[0] = P.lev[i].n[0]; L[1] = P.lev[i].n[1]; L[2] = P.lev[i].n[2];
         L[3] = P.lev[i].foff[0]; L[4] = P.lev[i].foff[1]; L[5] = P.lev[i].foff[2];
         L[6] = P.lev[i].maxs;
+        const unsigned long long t = (unsigned long long)(P.T[i] + (size_t)P.snap * P.lev[i].tstride);
+        L[7] = (int)(uint32_t)t; L[8] = (int)(uint32_t)(t >> 32);
         L[11] = P.lev[i].ooff[0]; L[12] = P.lev[i].ooff[1]; L[13] = P.lev[i].ooff[2];
     }
     for (int i = threadIdx.x; i < P.nfaces; i += blockDim.x) s_face[i] = P.faces[i];
@@ -1936,17 +1967,69 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
     for (int i = threadIdx.x; i < P.ncent; i += blockDim.x) s_cent[i] = P.centres[i];
     for (int i = threadIdx.x; i < 6 * P.nB; i += blockDim.x) s_ibw[i] = P.Ibw[i];
     __syncthreads();
-    const double Tm = (double)P.Tmax;
+    const int lane = threadIdx.x & 63;
+    const double Tm = (double)P.Tmax, tau_cut = (double)P.tau_cut;
     unsigned long long steps_t = 0;
-    for (long long q = blockIdx.x * (long long)blockDim.x + threadIdx.x; q < P.nrays;
-         q += (long long)gridDim.x * blockDim.x) {
+    // the lane's ray
+    bool alive = false;
+    uint32_t q = 0;
+    int f[3], c[3], band = 0, bg = 0, lev = 0, cnt = 0, steps = 0;
+    double s[3], inv[3], p[3], w = 0.0, ii = 1.0, tau = 0.0, tra = 1.0, G = 0.0;
+    uint32_t hash = 0;
+    // of its level
+    int n[3], fo[3], oo[3], maxs = 0;
+    gfloat* T = nullptr;
+    for (int a = 0; a < 3; ++a) {
+        f[a] = 0; c[a] = 1; n[a] = fo[a] = oo[a] = 0;
+        s[a] = inv[a] = 1.0; p[a] = 0.0;
+    }
+    auto set_level = [&]() {
+        const int* L = s_lev + lev * kLevWords;
+        for (int a = 0; a < 3; ++a) {
+            n[a] = L[a];
+            fo[a] = L[3 + a];
+            oo[a] = L[11 + a];
+        }
+        maxs = L[6];
+        T = lev_T(L);
+        cnt = 0;
+    };
+    auto finish = [&](double D, int endt) {
+        pray64[q] = make_double2(w * D, w * G / ii);
+        steps_t += (unsigned long long)steps;
+        if (REC && q < P.nrec) {
+            P.rec_steps[q] = steps;
+            P.rec_end[q] = endt;
+            P.rec_hash[q] = hash;
+            P.rec_D[q] = (float)D;
+            P.rec_G[q] = (float)G;
+        }
+        alive = false;
+    };
+    // the step cap: the next coarser level, or the end on the last
+    auto capped = [&]() {
+        while (alive && cnt >= maxs) {
+            if (lev + 1 < P.nlev) {
+                const int m[3] = {n[0], n[1], n[2]};
+                ++lev;
+                set_level();
+                for (int a = 0; a < 3; ++a) {
+                    const int r = m[a] / n[a];
+                    c[a] = (c[a] + r - 1) / r;
+                }
+            } else {
+                finish(1.0 - tra, 2);
+            }
+        }
+    };
+    auto start = [&]() {
         const uint32_t a0 = P.w0[q], a1 = P.w1[q];
-        const int4 si = P.slotinfo[P.slot0 + fdiv((uint32_t)q, P.fd_R)];
-        const int band = desc_band(a0, a1), g = desc_g(a1);
-        const int bg = band * P.nQ + g;
+        const int4 si = P.slotinfo[P.slot0 + fdiv(q, P.fd_R)];
+        const int g = desc_g(a1);
+        band = desc_band(a0, a1);
+        bg = band * P.nQ + g;
         const double ut = ((double)(a0 & 0xFFFFFFu) + (double)P.u_off) * 5.9604644775390625e-08;
         const double up = ((double)(a1 & 0xFFFFFFu) + (double)P.u_off) * 5.9604644775390625e-08;
-        double s[3], inv[3], p[3];
         {
             const int a = P.polar;
             const double cth = 1.0 - 2.0 * ut, st = 2.0 * sqrt(ut * (1.0 - ut));
@@ -1956,7 +2039,6 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
             s[1] = a == 0 ? c1 : (a == 1 ? cth : c2);
             s[2] = a == 0 ? c2 : (a == 1 ? c1 : cth);
         }
-        int f[3], c[3];
         for (int a = 0; a < 3; ++a) {
             if (s[a] == 0.0) s[a] = 1e-10;
             f[a] = s[a] < 0.0;
@@ -1967,7 +2049,7 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
         c[2] = ((si.w >> 20) & 1023) + 1;
         for (int a = 0; a < 3; ++a) p[a] = (double)s_cent[P.coff[a] + c[a]];
         const double Ti = (double)P.T[0][(size_t)P.snap * P.lev[0].tstride + si.z];
-        double ki, ii, kmx, imx;
+        double ki, kmx, imx;
         if (SPEC == kSpecGreyT4) {
             ki = kmx = (double)P.kappa_grey;
             ii = Ti * Ti * Ti * Ti;
@@ -1976,97 +2058,322 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64)
             lookup_f64(P, Ti, bg, band, &ki, &ii);
             lookup_f64(P, Tm, bg, band, &kmx, &imx);
         }
-        const double w = P.Ibmax_d * (ki * ii) / (kmx * imx);
-        double tau = 0.0, tra = 1.0, G = 0.0, D = 1.0;
-        const double tau_cut = (double)P.tau_cut;
-        int steps = 0, endt = 2;
-        uint32_t hash = 2166136261u;
-        bool done = false;
-        for (int lev = 0; lev < P.nlev && !done; ++lev) {
-            const int* L = s_lev + lev * kLevWords;
-            const int n[3] = {L[0], L[1], L[2]};
-            const int fo[3] = {L[3], L[4], L[5]};
-            const int oo[3] = {L[11], L[12], L[13]};
-            const float* T = P.T[lev] + (size_t)P.snap * P.lev[lev].tstride;
-            if (lev > 0) {
-                const int* Lp = s_lev + (lev - 1) * kLevWords;
-                for (int a = 0; a < 3; ++a) {
-                    const int r = Lp[a] / n[a];
-                    c[a] = (c[a] + r - 1) / r;
+        w = P.Ibmax_d * (ki * ii) / (kmx * imx);
+        tau = 0.0;
+        tra = 1.0;
+        G = 0.0;
+        steps = 0;
+        hash = 2166136261u;
+        lev = 0;
+        alive = true;
+        set_level();
+        capped();
+    };
+    auto cross = [&]() {
+        double fx[3], d[3];
+        for (int a = 0; a < 3; ++a) {
+            fx[a] = (double)s_face[fo[a] + c[a] - f[a]];
+            d[a] = (fx[a] - p[a]) * inv[a];
+        }
+        double ds = d[0];
+        ds = ds > d[1] ? d[1] : ds;
+        ds = ds > d[2] ? d[2] : ds;
+        for (int a = 0; a < 3; ++a) p[a] = (ds == d[a]) ? fx[a] : p[a] + ds * s[a];
+        if (REC) {
+            const int lin = (c[0] - 1) + n[0] * ((c[1] - 1) + n[1] * (c[2] - 1));
+            hash = (hash ^ (((uint32_t)lev << 28) ^ (uint32_t)lin)) * 16777619u;
+        }
+        const double Tj = (double)load_T(T, s_off[oo[0] + c[0] - 1] + s_off[oo[1] + c[1] - 1] + s_off[oo[2] + c[2] - 1]);
+        double kap, ibj;
+        if (SPEC == kSpecGreyT4) {
+            kap = (double)P.kappa_grey;
+            ibj = Tj * Tj * Tj * Tj;
+        } else {
+            lookup_f64(P, Tj, bg, band, &kap, &ibj);
+        }
+        ++steps;
+        ++cnt;
+        const double tau1 = tau + kap * ds;
+        if (tau1 >= tau_cut) {
+            G += tra * ibj;
+            finish(1.0, 0);
+            return;
+        }
+        const double tra1 = exp(-tau1);
+        G += (tra - tra1) * ibj;
+        tau = tau1;
+        tra = tra1;
+        const int ax = (d[0] < d[1]) ? ((d[0] < d[2]) ? 0 : 2) : ((d[1] < d[2]) ? 1 : 2);
+        for (int a = 0; a < 3; ++a) {
+            if (ax != a) continue;
+            c[a] += f[a] ? -1 : 1;
+            if (c[a] == 0 || c[a] == n[a] + 1) {
+                const int side = c[a] != 0;
+                if ((P.bc_periodic >> (a * 2 + side)) & 1) {
+                    c[a] = side ? 1 : n[a];
+                    p[a] = (double)s_face[fo[a] + (side ? 0 : n[a])];
+                } else {
+                    G += tra * (double)s_ibw[(a * 2 + side) * P.nB + band];
+                    finish(1.0, 1);
                 }
             }
-            int cnt = 0;
-            while (cnt < L[6]) {
-                double fx[3], d[3];
-                for (int a = 0; a < 3; ++a) {
-                    fx[a] = (double)s_face[fo[a] + c[a] - f[a]];
-                    d[a] = (fx[a] - p[a]) * inv[a];
-                }
-                double ds = d[0];
-                ds = ds > d[1] ? d[1] : ds;
-                ds = ds > d[2] ? d[2] : ds;
-                for (int a = 0; a < 3; ++a) p[a] = (ds == d[a]) ? fx[a] : p[a] + ds * s[a];
-                if (REC) {
-                    const int lin = (c[0] - 1) + n[0] * ((c[1] - 1) + n[1] * (c[2] - 1));
-                    hash = (hash ^ (((uint32_t)lev << 28) ^ (uint32_t)lin)) * 16777619u;
-                }
-                const uint32_t off = (uint32_t)(s_off[oo[0] + c[0] - 1] + s_off[oo[1] + c[1] - 1] + s_off[oo[2] + c[2] - 1]);
-                const double Tj = (double)*(const float*)((const char*)T + off);
-                double kap, ibj;
-                if (SPEC == kSpecGreyT4) {
-                    kap = (double)P.kappa_grey;
-                    ibj = Tj * Tj * Tj * Tj;
-                } else {
-                    lookup_f64(P, Tj, bg, band, &kap, &ibj);
-                }
-                ++steps;
-                ++cnt;
-                const double tau1 = tau + kap * ds;
-                if (tau1 >= tau_cut) {
-                    G += tra * ibj;
-                    endt = 0;
-                    done = true;
-                    break;
-                }
-                const double tra1 = exp(-tau1);
-                G += (tra - tra1) * ibj;
-                tau = tau1;
-                tra = tra1;
-                const int ax = (d[0] < d[1]) ? ((d[0] < d[2]) ? 0 : 2) : ((d[1] < d[2]) ? 1 : 2);
-                c[ax] += f[ax] ? -1 : 1;
-                if (c[ax] == 0 || c[ax] == n[ax] + 1) {
-                    const int side = c[ax] != 0;
-                    if ((P.bc_periodic >> (ax * 2 + side)) & 1) {
-                        c[ax] = side ? 1 : n[ax];
-                        p[ax] = (double)s_face[fo[ax] + (side ? 0 : n[ax])];
-                    } else {
-                        c[ax] -= f[ax] ? -1 : 1;
-                        G += tra * (double)s_ibw[(ax * 2 + side) * P.nB + band];
-                        endt = 1;
-                        done = true;
+        }
+        capped();
+    };
+    unsigned long long cb = 0, ce = 0;   // the wave's claimed rays
+    bool more = true;
+    for (;;) {
+        unsigned long long idle = __ballot(!alive);
+        if (more && __popcll(idle) >= 16) {
+            while (idle) {
+                if (cb >= ce) {
+                    unsigned long long r = 0;
+                    if (lane == 0) r = atomicAdd((unsigned long long*)P.claim, (unsigned long long)super);
+                    r = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(r >> 32)) << 32) |
+                        (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
+                    if (r >= (unsigned long long)P.nrays) {
+                        more = false;
                         break;
                     }
+                    cb = r;
+                    ce = min(r + (unsigned long long)super, (unsigned long long)P.nrays);
                 }
+                const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
+                                                                __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+                const int take = (int)min((unsigned long long)__popcll(idle), ce - cb);
+                if (!alive && rank < take) {
+                    q = (uint32_t)(cb + (unsigned long long)rank);
+                    start();
+                }
+                cb += (unsigned long long)take;
+                idle = __ballot(!alive);
             }
         }
-        if (!done) D = 1.0 - tra;
-        pray64[q] = make_double2(w * D, w * G / ii);
-        steps_t += (unsigned long long)steps;
-        if (REC && q < P.nrec) {
-            P.rec_steps[q] = steps;
-            P.rec_end[q] = endt;
-            P.rec_hash[q] = hash;
-            P.rec_D[q] = (float)D;
-            P.rec_G[q] = (float)G;
+        const unsigned long long am = __ballot(alive);
+        if (!am) break;   // (nothing is left to hand out either)
+        if (!more && __popcll(am) <= kQuads && !__ballot(alive && lev + 1 < P.nlev)) break;
+        if (alive) cross();
+    }
+    // ---- drain: lane a of a quad holds axis a of its ray (lane 3 none)
+    if (__ballot(alive)) {
+        __builtin_amdgcn_s_setprio(3);
+        const unsigned long long am = __ballot(alive);
+        const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(am >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)am, 0u));
+        // the lane of the ray that this quad follows: its rank-th alive lane
+        // (each alive lane sends its number to lane 4 rank, the others to 63)
+        int src = quad_i<0>(__builtin_amdgcn_ds_permute(alive ? 16 * rank : 4 * 63, lane));
+        const int a = lane & 3;
+        const bool ax3 = a == 3;
+        bool run = (lane >> 2) < __popcll(am);
+        src = run ? src : 0;
+        auto axis_d = [&](const double* v, double w3) -> double {
+            const double vx = __shfl(v[0], src), vy = __shfl(v[1], src), vz = __shfl(v[2], src);
+            return a == 0 ? vx : (a == 1 ? vy : (a == 2 ? vz : w3));
+        };
+        const int* L = s_lev + (P.nlev - 1) * kLevWords;   // the last level
+        double qp = axis_d(p, 0.0), qs = axis_d(s, 0.0), qi = axis_d(inv, 1.0);
+        int qc;                                            // 0-based cell (0 where the quad has no ray)
+        bool neg;
+        {
+            const int c0 = __shfl(c[0], src), c1 = __shfl(c[1], src), c2 = __shfl(c[2], src);
+            const int f0 = __shfl(f[0], src), f1 = __shfl(f[1], src), f2 = __shfl(f[2], src);
+            qc = !run || ax3 ? 0 : (a == 0 ? c0 : (a == 1 ? c1 : c2)) - 1;
+            neg = a == 0 ? f0 != 0 : (a == 1 ? f1 != 0 : (a == 2 ? f2 != 0 : false));
         }
+        const int st = neg ? -1 : 1;
+        double qtau = __shfl(tau, src), qtra = __shfl(tra, src), qG = __shfl(G, src);
+        const int qbg = __shfl(bg, src), qband = __shfl(band, src);
+        int qcnt = __shfl(cnt, src), qtot = 0, qend = 0;
+        double qD = 1.0;
+        uint32_t qhash = REC ? (uint32_t)__shfl((int)hash, src) : 0u;
+        const int bcbit = 2 * a + (neg ? 0 : 1);           // the boundary this axis runs into
+        const bool per = (P.bc_periodic >> bcbit) & 1;
+        const int qn = ax3 ? 0x7FFFFFFF : L[a], qmaxs = L[6];
+        const int fb = L[3 + (ax3 ? 0 : a)] + (neg ? 0 : 1), ob = L[11 + (ax3 ? 0 : a)];   // exit face, offset of cell 0
+        const int qstride = a == 0 ? 1 : (a == 1 ? L[0] : (a == 2 ? L[0] * L[1] : 0));
+        gfloat* qT = lev_T(L);
+        // (lane 3 is never the nearest face: distance 3e38)
+        double qf = ax3 ? 3.0e38 : (double)s_face[fb + qc];
+        while (__ballot(run)) {
+            int lim = run ? min(kDrain, qmaxs - qcnt) : 0;
+            int wall = -1;
+            // a frozen quad (no ray, or its ray hit a wall inside the batch) has
+            // length-0 crossings and does not move
+            unsigned long long live = __ballot(run);
+            int nlive = __popcll(live) >> 2;
+            qs = run ? qs : 0.0;
+            qi = run ? qi : 0.0;
+            double dso[kDrain / 4];                        // crossing 4 k + a on lane a
+            int oid[kDrain / 4], lin[kDrain / 4];
+            // the two faces behind the exit face (a word past the axis's faces is
+            // one of its LDS neighbours and is not used)
+            double g = (double)s_face[fb + qc + st];
+            float h = s_face[fb + qc + 2 * st];
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                int ov[4];
+                oid[k] = lin[k] = 0;
+                dso[k] = 0.0;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int u = 4 * k + j;
+                    ov[j] = s_off[ob + qc];
+                    const double d = (qf - qp) * qi;
+                    const double ds = quad_min_d(d);
+                    dso[k] = a == j ? ds : dso[k];
+                    unsigned long long em = __ballot(d == ds) & live;
+                    qp = __builtin_amdgcn_inverse_ballot_w64(em) ? qf : qp + ds * qs;
+                    // of several axes at the same distance the last one moves
+                    if (__builtin_expect(__popcll(em) != nlive, 0))
+                        em &= ~((em >> 1) | ((em >> 2) & 0x1111111111111111ull));
+                    const bool mv = __builtin_amdgcn_inverse_ballot_w64(em);
+                    if (REC) {
+                        const int l = quad_sum(qc * qstride);
+                        lin[k] = a == j ? l : lin[k];
+                    }
+                    qc += mv ? st : 0;
+                    qf = mv ? g : qf;
+                    g = mv ? (double)h : g;
+                    const bool out = (uint32_t)qc >= (uint32_t)qn;
+                    if (__builtin_expect(__ballot(out) != 0ull, 0)) {
+                        int wl = -1;
+                        if (out) {
+                            if (per) {
+                                qc = neg ? qn - 1 : 0;
+                                qp = (double)s_face[fb + qc - st];
+                            } else {
+                                wl = bcbit;
+                                qc -= st;
+                            }
+                            qf = (double)s_face[fb + qc];
+                            g = (double)s_face[fb + qc + st];
+                        }
+                        wl = quad_max(wl);
+                        const bool hit = wl >= 0;
+                        wall = hit && u < lim ? wl : wall;
+                        lim = hit ? min(lim, u + 1) : lim;
+                        qs = hit ? 0.0 : qs;
+                        qi = hit ? 0.0 : qi;
+                        live &= ~__ballot(hit);
+                        nlive = __popcll(live) >> 2;
+                    }
+                    h = s_face[fb + qc + 2 * st];
+                }
+                // the cells' field offsets: crossing 4 k + j to lane j
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int ou = quad_sum(ax3 ? 0 : ov[j]);
+                    oid[k] = a == j ? ou : oid[k];
+                }
+            }
+            if (__ballot(run && lim < kDrain)) {           // a wall or the step cap inside the batch
+#pragma unroll
+                for (int k = 0; k < kDrain / 4; ++k) dso[k] = 4 * k + a < lim ? dso[k] : 0.0;
+            }
+            // the cells' temperatures and lookups; each crossing's optical depth
+            double Tv[kDrain / 4], dt[kDrain / 4], ibv[kDrain / 4], tk[kDrain / 4], dg[kDrain / 4];
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) Tv[k] = (double)load_T(qT, oid[k]);
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                double kap;
+                if (SPEC == kSpecGreyT4) {
+                    kap = (double)P.kappa_grey;
+                    ibv[k] = Tv[k] * Tv[k] * Tv[k] * Tv[k];
+                } else {
+                    lookup_f64(P, Tv[k], qbg, qband, &kap, &ibv[k]);
+                }
+                dt[k] = kap * dso[k];
+            }
+            // summed in crossing order (every lane of the quad), kept by the
+            // crossing's lane
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                const double t0 = qtau + quad_d<0x00>(dt[k]), t1 = t0 + quad_d<0x55>(dt[k]);
+                const double t2 = t1 + quad_d<0xAA>(dt[k]);
+                qtau = t2 + quad_d<0xFF>(dt[k]);
+                tk[k] = a == 0 ? t0 : (a == 1 ? t1 : (a == 2 ? t2 : qtau));
+            }
+            // transmissivities; the first crossing past the cut-off
+            int first = kDrain;
+            double before = qtra;   // transmissivity before this group of four
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                const bool cut = tk[k] >= tau_cut;
+                const double e1 = exp(-tk[k]);
+                const double e0 = quad_d<kQuadPrev>(e1);   // (every lane of the quad takes part)
+                const double ep = a == 0 ? before : e0;
+                dg[k] = cut ? ep : ep - e1;
+                first = min(first, cut ? 4 * k + a : kDrain);
+                before = quad_d<0xFF>(e1);
+            }
+            bool cutq = false;
+            int taken = lim;
+            if (__ballot(first < lim)) {
+                first = quad_min_i(first);
+                cutq = first < lim;
+                taken = cutq ? first + 1 : lim;
+#pragma unroll
+                for (int k = 0; k < kDrain / 4; ++k) dg[k] = 4 * k + a < taken ? dg[k] : 0.0;
+            }
+#pragma unroll
+            for (int k = 0; k < kDrain / 4; ++k) {
+                const double x = dg[k] * ibv[k];
+                qG += quad_d<0x00>(x);
+                qG += quad_d<0x55>(x);
+                qG += quad_d<0xAA>(x);
+                qG += quad_d<0xFF>(x);
+            }
+            if (REC) {
+                const uint32_t lb = (uint32_t)(P.nlev - 1) << 28;
+#pragma unroll
+                for (int k = 0; k < kDrain / 4; ++k) {
+                    const uint32_t l0 = (uint32_t)quad_i<0x00>(lin[k]), l1 = (uint32_t)quad_i<0x55>(lin[k]);
+                    const uint32_t l2 = (uint32_t)quad_i<0xAA>(lin[k]), l3 = (uint32_t)quad_i<0xFF>(lin[k]);
+                    if (4 * k < taken) qhash = (qhash ^ (lb ^ l0)) * 16777619u;
+                    if (4 * k + 1 < taken) qhash = (qhash ^ (lb ^ l1)) * 16777619u;
+                    if (4 * k + 2 < taken) qhash = (qhash ^ (lb ^ l2)) * 16777619u;
+                    if (4 * k + 3 < taken) qhash = (qhash ^ (lb ^ l3)) * 16777619u;
+                }
+            }
+            qtra = before;   // (not used after a cut-off)
+            qcnt += taken;
+            qtot += taken;
+            const bool hitw = run && !cutq && wall >= 0;
+            if (hitw) qG += qtra * (double)s_ibw[wall * P.nB + qband];
+            if (run && (cutq || hitw)) {
+                run = false;
+                qend = cutq ? 0 : 1;
+                qtau = 0.0;   // (the quad idles below the cut-off: it adds 0)
+                qtra = 1.0;
+            } else if (run && qcnt >= qmaxs) {
+                run = false;
+                qend = 2;
+                qD = 1.0 - qtra;
+                qtau = 0.0;
+                qtra = 1.0;
+            }
+        }
+        // back to the lanes that held the rays
+        const int from = alive ? 4 * rank : lane;
+        const double rG = __shfl(qG, from), rD = __shfl(qD, from);
+        const int rtot = __shfl(qtot, from), ren = __shfl(qend, from);
+        const uint32_t rh = REC ? (uint32_t)__shfl((int)qhash, from) : 0u;
+        if (alive) {
+            G = rG;
+            steps += rtot;
+            if (REC) hash = rh;
+            finish(rD, ren);
+        }
+        __builtin_amdgcn_s_setprio(0);
     }
     for (int off = 32; off > 0; off >>= 1) steps_t += __shfl_xor(steps_t, off);
-    if ((threadIdx.x & 63) == 0) atomicAdd(P.nsteps, steps_t);
+    if (lane == 0) atomicAdd(P.nsteps, steps_t);
 }
-template __global__ void trace_f64<kSpecTable, false>(TraceArgs, double2*);
-template __global__ void trace_f64<kSpecTable, true>(TraceArgs, double2*);
-template __global__ void trace_f64<kSpecGreyT4, false>(TraceArgs, double2*);
-template __global__ void trace_f64<kSpecGreyT4, true>(TraceArgs, double2*);
+template __global__ void trace_f64<kSpecTable, false>(TraceArgs, double2*, int);
+template __global__ void trace_f64<kSpecTable, true>(TraceArgs, double2*, int);
+template __global__ void trace_f64<kSpecGreyT4, false>(TraceArgs, double2*, int);
+template __global__ void trace_f64<kSpecGreyT4, true>(TraceArgs, double2*, int);
 
 // Per-slot sums of the FP64 traversal's per-ray (E, A), in ray order, in the
 // configured tally arithmetic (FP64, Kahan-compensated FP32 or plain FP32).

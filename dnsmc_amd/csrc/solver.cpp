@@ -31,7 +31,7 @@ __global__ void raygen_plain(GenArgs a);
 __global__ void raygen_compat(GenArgs a);
 __global__ void raygen_compat_sorted(GenArgs a);
 template <int SPEC, bool REC>
-__global__ void trace_f64(TraceArgs P, double2* pray64);
+__global__ void trace_f64(TraceArgs P, double2* pray64, int super);
 __global__ void reduce_rays64(const double2* pray, int tally, long long nslots, int R, long long slot0,
                               const int4* slotinfo, double* E, double* A, double* Q2);
 __global__ void finalize(const double* E, const double* A, const double* Q2, long long nemit, int spe, int R,
@@ -1377,11 +1377,13 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             HIPCHK(hipEventRecord(et.a, st));
             if (f64) {
                 const size_t lds64 = sizeof(float) * (6 * kLevWords + P.nfaces + P.noffs + P.ncent + 6 * (size_t)d.nB);
-                const int nb = (int)std::min<long long>((nr + 255) / 256, (long long)s->ncu * 16);
-                void (*k)(TraceArgs, double2*) =
+                // three waves per SIMD (registers); about four claims per wave
+                const int nb = (int)std::min<long long>((nr + 255) / 256, (long long)s->ncu * 3);
+                const int super = (int)std::max(64ll, std::min<long long>(512, nr / (16ll * nb) / 64 * 64));
+                void (*k)(TraceArgs, double2*, int) =
                     spec == kSpecGreyT4 ? (rec ? trace_f64<kSpecGreyT4, true> : trace_f64<kSpecGreyT4, false>)
                                         : (rec ? trace_f64<kSpecTable, true> : trace_f64<kSpecTable, false>);
-                hipLaunchKernelGGL(k, dim3(nb), dim3(256), lds64, st, P, pp.d_pray64.p);
+                hipLaunchKernelGGL(k, dim3(nb), dim3(256), lds64, st, P, pp.d_pray64.p, super);
             } else {
                 HIPCHK(launch_trace(spec, tab, false, det, rec, amc, s->ncu, tb_cap, lds_trace, st, P));
             }
