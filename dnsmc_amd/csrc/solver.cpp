@@ -32,13 +32,12 @@ __global__ void raygen_compat(GenArgs a);
 __global__ void raygen_compat_sorted(GenArgs a);
 template <int SPEC, bool REC>
 __global__ void trace_f64(TraceArgs P, double2* pray64, int super);
-__global__ void reduce_rays64(const double2* pray, int tally, long long nslots, int R, long long slot0,
-                              const int4* slotinfo, double* E, double* A, double* Q2);
 __global__ void finalize(const double* E, const double* A, const double* Q2, long long nemit, int spe, int R,
                          int compat, double* Q, double* Eo, double* Ao, double* sd);
 __global__ void spline_pass(SplineArgs s);
-__global__ void reduce_rays(const float2* pray, int tally, long long nslots, int R, long long slot0,
-                            const int4* slotinfo, double* E, double* A, double* Q2);
+template <typename V, int NS>
+__global__ void reduce_rays(const V* pray, int tally, long long nslots, int R, long long slot0, const int4* slotinfo,
+                            double* E, double* A, double* Q2);
 __global__ void fill_f64(double* p, long long n, double v);
 __global__ void cand_scan(TraceArgs P, uint32_t nfin, uint32_t* list);
 // mlp.hip
@@ -1389,15 +1388,18 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             }
             HIPCHK(hipEventRecord(et.b, st));
             s->st.n_trace_launches++;
-            if (f64) {
-                int nb = (int)((nsl + 255) / 256);
-                hipLaunchKernelGGL(reduce_rays64, dim3(nb), dim3(256), 0, st, (const double2*)pp.d_pray64.p, c.tally,
-                                   nsl, R, b0, (const int4*)s->d_slotinfo.p, P.E, P.A, P.Q2);
-                HIPCHK(hipGetLastError());
-            } else if (det && !rec) {   // record launches tally with FP64 atomics
-                int nb = (int)((nsl + 255) / 256);
-                hipLaunchKernelGGL(reduce_rays, dim3(nb), dim3(256), 0, st, (const float2*)pp.d_pray.p, c.tally, nsl, R,
-                                   b0, (const int4*)s->d_slotinfo.p, P.E, P.A, P.Q2);
+            if (f64 || (det && !rec)) {   // FP32 record launches tally with FP64 atomics
+                // 64 slots per block while that gives every CU one, else 16
+                const bool wide = nsl >= 64ll * s->ncu;
+                const int nb = (int)((nsl + (wide ? 63 : 15)) / (wide ? 64 : 16));
+                if (f64)
+                    hipLaunchKernelGGL(HIP_KERNEL_NAME(wide ? reduce_rays<double2, 64> : reduce_rays<double2, 16>), dim3(nb),
+                                       dim3(256), 0, st, (const double2*)pp.d_pray64.p, c.tally, nsl, R, b0,
+                                       (const int4*)s->d_slotinfo.p, P.E, P.A, P.Q2);
+                else
+                    hipLaunchKernelGGL(HIP_KERNEL_NAME(wide ? reduce_rays<float2, 64> : reduce_rays<float2, 16>), dim3(nb),
+                                       dim3(256), 0, st, (const float2*)pp.d_pray.p, c.tally, nsl, R, b0,
+                                       (const int4*)s->d_slotinfo.p, P.E, P.A, P.Q2);
                 HIPCHK(hipGetLastError());
             }
         }
