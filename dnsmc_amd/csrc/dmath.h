@@ -13,6 +13,8 @@
 
 namespace dn {
 
+constexpr int kMaxLev = 6;   // grid levels
+
 // 2^-24: descriptor direction fields hold 24-bit integers m, u = (m + off) 2^-24.
 constexpr float kTwoM24 = 5.9604644775390625e-08f;
 

@@ -204,27 +204,46 @@ struct GenArgs {
     float* winv;
 };
 
-struct SplineArgs {
-    const float* in;
+// One axis of the coarse levels' spline (spline_pass), all levels in one launch.
+struct SplineLevel {
+    const float* in;         // (x: SplinePass::fine)
     float* out;
-    double* work;
-    int nlines;
-    int nf, nc;
-    long long A, sa_in, sb_in, st_in, sa_out, sb_out, st_out;
-    const double* sig;
+    const int* klo;          // per coarse centre: the fine interval and its weights
+    const double* ca;
+    const double* cb;
+    const double* cA;
+    const double* cB;
+    size_t work0;            // the level's part of SplinePass::work (x: shared)
+    int nc, nlines;
+    int m0, m1;              // the level's cells along x and y
+    int nbx, nby;            // its bricks (z)
+};
+struct SplinePass {
+    const double* sig;       // [nf], the fine grid's alone
     const double* invp;
     const double* y2f;
     const double* c6;
     const double* ihl;
     const double* ihh;
-    const int* klo;
-    const double* ca;
-    const double* cb;
-    const double* cA;
-    const double* cB;
-    long long snap_in, snap_out;   // per-snapshot strides
-    int brick_out, m0, nbx, nby;   // z pass: write the bricked layout of the coarse level
-    int in_bricked, fn1, fnbx, fnby;   // x pass: read the bricked fine field (line = j + n1 k)
+    double* work;            // second derivatives, [i][line]
+    int nf, nlev;
+    int fn1;                 // fine cells along y
+    const float* fine;       // bricked fine field (x)
+    int fnbx, fnby;
+    SplineLevel lv[kMaxLev - 1];
+};
+
+// Temperature range of the levels (t_range).
+struct RangeLevel {
+    const float* T;
+    int n[3];
+    int nbricks;
+    FastDiv fd_nbx, fd_nby;
+};
+struct RangeArgs {
+    RangeLevel lv[kMaxLev];
+    int nlev;
+    unsigned* keys;          // per level: smallest key, complement of the largest (both start at ~0u)
 };
 
 // ------------------------------------------------ shared device helpers ----

@@ -2384,27 +2384,56 @@ DN_TRACE_INST3(kSpecTable, kTabIbLds)
 DN_TRACE_INST3(kSpecTable, kTabGlobal)
 DN_TRACE_INST3(kSpecGreyT4, kTabGlobal)
 
-// Range of a bricked level field as order-preserving keys of its FP32 values
-// (lohi = {min key, max key}; the host starts them at {~0u, 0}).
-__global__ void t_range(const float* T, int n0, int n1, int n2, int nbx, int nby, unsigned* lohi)
+// Range of the bricked level fields as order-preserving keys of their FP32
+// values.  A wave takes a brick (64 cells) per load; one pair of atomics per
+// block and level that has bricks for it (a wave's pair each, on the two words
+// of a level, serialised at 11 ns: 376 us per level of 4.2e6 cells, now
+// 27 us for that level and four coarser ones, 37 us for 25e6 cells).
+__global__ __launch_bounds__(1024) void t_range(RangeArgs a)
 {
-    const long long n = (long long)n0 * n1 * n2;
-    unsigned lo = 0xFFFFFFFFu, hi = 0u;
-    for (long long c = blockIdx.x * (long long)blockDim.x + threadIdx.x; c < n; c += (long long)gridDim.x * blockDim.x) {
-        const int i = (int)(c % n0), j = (int)((c / n0) % n1), k = (int)(c / ((long long)n0 * n1));
-        const unsigned u = __float_as_uint(T[brick_index(i, j, k, nbx, nby)]);
-        const unsigned key = (u & 0x80000000u) ? ~u : (u | 0x80000000u);
-        lo = key < lo ? key : lo;
-        hi = key > hi ? key : hi;
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned a = __shfl_xor(lo, off), b = __shfl_xor(hi, off);
-        lo = a < lo ? a : lo;
-        hi = b > hi ? b : hi;
-    }
-    if ((threadIdx.x & 63) == 0) {
-        atomicMin(&lohi[0], lo);
-        atomicMax(&lohi[1], hi);
+    __shared__ unsigned s_lo[16], s_hi[16];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int w = blockIdx.x * 16 + wv, nw = gridDim.x * 16;
+    const int x = ((lane >> 5) << 1) | (lane & 1), y = (lane >> 1) & 3, z = (lane >> 3) & 3;   // brick_index
+    for (int l = 0; l < a.nlev; ++l) {
+        const RangeLevel& L = a.lv[l];
+        if ((int)blockIdx.x * 16 >= L.nbricks) continue;
+        unsigned lo = 0xFFFFFFFFu, hi = 0u;
+        for (int b0 = w; b0 < L.nbricks; b0 += 8 * nw) {
+            float v[8];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) v[u] = L.T[(size_t)min(b0 + u * nw, L.nbricks - 1) * 64 + lane];
+#pragma unroll
+            for (int u = 0; u < 8; ++u) {
+                const uint32_t b = (uint32_t)min(b0 + u * nw, L.nbricks - 1);
+                const uint32_t r = fdiv(b, L.fd_nbx), bx = b - r * L.fd_nbx.d;
+                const uint32_t bz = fdiv(r, L.fd_nby), by = r - bz * L.fd_nby.d;
+                const unsigned k = __float_as_uint(v[u]);
+                const unsigned key = (k & 0x80000000u) ? ~k : (k | 0x80000000u);
+                if ((int)bx * 4 + x < L.n[0] && (int)by * 4 + y < L.n[1] && (int)bz * 4 + z < L.n[2]) {
+                    lo = key < lo ? key : lo;
+                    hi = key > hi ? key : hi;
+                }
+            }
+        }
+        for (int off = 32; off > 0; off >>= 1) {
+            lo = min(lo, (unsigned)__shfl_xor((int)lo, off));
+            hi = max(hi, (unsigned)__shfl_xor((int)hi, off));
+        }
+        if (lane == 0) {
+            s_lo[wv] = lo;
+            s_hi[wv] = hi;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            for (int i = 1; i < 16; ++i) {
+                lo = min(lo, s_lo[i]);
+                hi = max(hi, s_hi[i]);
+            }
+            atomicMin(&a.keys[2 * l], lo);
+            atomicMin(&a.keys[2 * l + 1], ~hi);
+        }
+        __syncthreads();
     }
 }
 
@@ -2532,44 +2561,149 @@ __global__ void finalize(const double* E, const double* A, const double* Q2, lon
 }
 
 // --------------------------------------------------------- spline pass ----
-// One thread per grid line: natural-spline second derivatives through the
-// fine values (forward sweep + back substitution, FP64), then evaluation at
-// the coarse centres.  The grid-only factors come precomputed from the host.
-// The x pass reads the bricked fine field; the z pass writes the bricked
-// layout of the coarse level.
-__global__ void spline_pass(SplineArgs s)
+// One lane per grid line: natural-spline second derivatives through the fine
+// values (forward sweep + back substitution, FP64), then evaluation at the
+// coarse centres.  The grid-only factors come precomputed from the host.  The x
+// pass sweeps the bricked fine field's lines once and evaluates every level on
+// them (line j + n1 k); the y and z passes hold every level's lines (i + m0 k,
+// i + m0 j) in one launch, and z writes the bricked layout of the levels.
+//
+// A sweep is one dependent chain per line, and the lines are few (a wave per CU
+// on 256x128x128 cells), so what counts is that no load stands in the chain: the
+// next kSpl values are in flight while a group is computed, the second
+// derivatives lie [i][line] (whole lines per wave), the factors in LDS, and the
+// x pass's rows leave through LDS in pieces of 16.  Five levels of 256x128x128
+// cells: 12 launches of 128 us each (a load, a line-strided store and a
+// coefficient load behind each other in the chain) -> 190 + 52 + 52 us.
+constexpr int kSpl = 16;
+template <int AXIS>
+__global__ __launch_bounds__(64) void spline_pass(SplinePass s)
 {
-    int l = blockIdx.x * blockDim.x + threadIdx.x;
-    if (l >= s.nlines) return;
-    double* u = s.work + (size_t)l * s.nf;
-    const int nf = s.nf;
-    const float* in = s.in + (l % s.A) * s.sa_in + (l / s.A) * s.sb_in;
-    const int bj = s.in_bricked ? l % s.fn1 : 0, bk = s.in_bricked ? l / s.fn1 : 0;
-    auto rd = [&](int i) -> double {
-        if (s.in_bricked) return (double)s.in[brick_index(i, bj, bk, s.fnbx, s.fnby)];
-        return (double)in[(long long)i * s.st_in];
-    };
-    u[0] = 0.0;
-    double ym = rd(0), y0 = rd(1);
-    for (int i = 1; i < nf - 1; ++i) {
-        double yp = rd(i + 1);
-        double dd = (yp - y0) * s.ihh[i] - (y0 - ym) * s.ihl[i];
-        u[i] = (s.c6[i] * dd - s.sig[i] * u[i - 1]) * s.invp[i];
-        ym = y0;
-        y0 = yp;
+    extern __shared__ __align__(16) double s_f[];   // [6][nf] factors; x: 64 x 17 floats
+    const int nf = s.nf, lane = threadIdx.x;
+    double *f_ihh = s_f, *f_ihl = s_f + nf, *f_c6 = s_f + 2 * nf, *f_sig = s_f + 3 * nf, *f_invp = s_f + 4 * nf, *f_y2f = s_f + 5 * nf;
+    float* s_t = (float*)(s_f + 6 * nf);
+    for (int i = lane; i < nf; i += 64) {
+        f_ihh[i] = s.ihh[i];
+        f_ihl[i] = s.ihl[i];
+        f_c6[i] = s.c6[i];
+        f_sig[i] = s.sig[i];
+        f_invp[i] = s.invp[i];
+        f_y2f[i] = s.y2f[i];
     }
-    u[nf - 1] = 0.0;
-    for (int k = nf - 2; k >= 1; --k) u[k] = s.y2f[k] * u[k + 1] + u[k];
-    u[0] = 0.0;
-    for (int q = 0; q < s.nc; ++q) {
-        int k = s.klo[q];
-        double v = s.ca[q] * rd(k) + s.cb[q] * rd(k + 1) + s.cA[q] * u[k] + s.cB[q] * u[k + 1];
-        long long o;
-        if (s.brick_out) o = brick_index(l % s.m0, l / s.m0, q, s.nbx, s.nby);   // line l = i + m0 j
-        else o = (l % s.A) * s.sa_out + (l / s.A) * s.sb_out + (long long)q * s.st_out;
-        s.out[o] = (float)v;
+    int lv = 0, blk = blockIdx.x;
+    if (AXIS != 0)
+        for (int nb = (s.lv[0].nlines + 63) / 64; blk >= nb; nb = (s.lv[lv].nlines + 63) / 64) {
+            blk -= nb;
+            ++lv;
+        }
+    const SplineLevel& L0 = s.lv[lv];
+    const int nl = L0.nlines, l = blk * 64 + lane, lc = min(l, nl - 1);   // (lanes past the last line repeat it)
+    const bool live = l < nl;
+    const float* in;
+    long long st_in = 0;
+    if (AXIS == 0) {
+        in = s.fine + brick_index(0, lc % s.fn1, lc / s.fn1, s.fnbx, s.fnby);
+    } else if (AXIS == 1) {
+        in = L0.in + (lc % L0.m0) + (long long)(lc / L0.m0) * L0.m0 * s.fn1;
+        st_in = L0.m0;
+    } else {
+        in = L0.in + lc;
+        st_in = (long long)L0.m0 * L0.m1;
+    }
+    auto rd = [&](int i) -> float {
+        return AXIS == 0 ? in[(size_t)(((i >> 2) << 6) | (((i >> 1) & 1) << 5) | (i & 1))] : in[(long long)i * st_in];
+    };
+    double* __restrict__ u = s.work + L0.work0 + lc;
+    __syncthreads();
+    float yn[kSpl];
+    {   // forward
+        double ym = (double)rd(0), y0 = (double)rd(min(1, nf - 1)), up = 0.0;
+#pragma unroll
+        for (int b = 0; b < kSpl; ++b) yn[b] = rd(min(2 + b, nf - 1));
+        if (live) u[0] = 0.0;
+        for (int i = 1; i < nf - 1; i += kSpl) {
+            float yc[kSpl];
+#pragma unroll
+            for (int b = 0; b < kSpl; ++b) {
+                yc[b] = yn[b];
+                yn[b] = rd(min(i + kSpl + 1 + b, nf - 1));
+            }
+#pragma unroll
+            for (int b = 0; b < kSpl; ++b) {
+                if (i + b >= nf - 1) break;
+                const double yp = (double)yc[b];
+                const double dd = (yp - y0) * f_ihh[i + b] - (y0 - ym) * f_ihl[i + b];
+                up = (f_c6[i + b] * dd - f_sig[i + b] * up) * f_invp[i + b];
+                if (live) u[(size_t)(i + b) * nl] = up;
+                ym = y0;
+                y0 = yp;
+            }
+        }
+        if (live) u[(size_t)(nf - 1) * nl] = 0.0;
+    }
+    {   // back
+        double un = 0.0, vn[kSpl];
+#pragma unroll
+        for (int b = 0; b < kSpl; ++b) vn[b] = u[(size_t)max(nf - 2 - b, 0) * nl];
+        for (int k = nf - 2; k >= 1; k -= kSpl) {
+            double vc[kSpl];
+#pragma unroll
+            for (int b = 0; b < kSpl; ++b) {
+                vc[b] = vn[b];
+                vn[b] = u[(size_t)max(k - kSpl - b, 0) * nl];
+            }
+#pragma unroll
+            for (int b = 0; b < kSpl; ++b) {
+                if (k - b < 1) break;
+                un = f_y2f[k - b] * un + vc[b];
+                if (live) u[(size_t)(k - b) * nl] = un;
+            }
+        }
+    }
+    // evaluation
+    constexpr int E = 8;
+    for (int v = lv; v < (AXIS == 0 ? s.nlev : lv + 1); ++v) {
+        const SplineLevel& L = s.lv[v];
+        for (int q0 = 0; q0 < L.nc; q0 += 16) {
+#pragma unroll
+            for (int h = 0; h < 16; h += E) {
+                float ya[E], yb[E];
+                double ua[E], ub[E];
+#pragma unroll
+                for (int b = 0; b < E; ++b) {
+                    const int k = L.klo[min(q0 + h + b, L.nc - 1)];
+                    ya[b] = rd(k);
+                    yb[b] = rd(k + 1);
+                    ua[b] = u[(size_t)k * nl];
+                    ub[b] = u[(size_t)(k + 1) * nl];
+                }
+#pragma unroll
+                for (int b = 0; b < E; ++b) {
+                    const int q = q0 + h + b;
+                    if (q >= L.nc) break;
+                    const double val = L.ca[q] * (double)ya[b] + L.cb[q] * (double)yb[b] + L.cA[q] * ua[b] + L.cB[q] * ub[b];
+                    if (AXIS == 0) s_t[lane * 17 + h + b] = (float)val;
+                    else if (!live) continue;
+                    else if (AXIS == 1) L.out[(l % L.m0) + (long long)(l / L.m0) * L.m0 * L.m1 + (long long)q * L.m0] = (float)val;
+                    else L.out[brick_index(l % L.m0, l / L.m0, q, L.nbx, L.nby)] = (float)val;
+                }
+            }
+            if (AXIS == 0) {   // 64 rows of 16
+                __syncthreads();
+#pragma unroll
+                for (int e = lane; e < 64 * 16; e += 64) {
+                    const int r = e >> 4, q = q0 + (e & 15);
+                    if (q < L.nc && blk * 64 + r < nl) L.out[(size_t)(blk * 64 + r) * L.nc + q] = s_t[r * 17 + (e & 15)];
+                }
+                __syncthreads();
+            }
+        }
     }
 }
+template __global__ void spline_pass<0>(SplinePass);
+template __global__ void spline_pass<1>(SplinePass);
+template __global__ void spline_pass<2>(SplinePass);
 
 // Plain streaming copy (16 B per thread and iteration); the reference point
 // for calibrating HBM byte counters.

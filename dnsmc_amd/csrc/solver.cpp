@@ -26,7 +26,7 @@ namespace dn {
 // kernels.hip
 template <int SPEC, int TAB, int TMODE, bool REC, bool AMC, int GEN>
 __global__ void trace(TraceArgs P);
-__global__ void t_range(const float* T, int n0, int n1, int n2, int nbx, int nby, unsigned* lohi);
+__global__ void t_range(RangeArgs a);
 __global__ void raygen_plain(GenArgs a);
 __global__ void raygen_compat(GenArgs a);
 __global__ void raygen_compat_sorted(GenArgs a);
@@ -34,7 +34,8 @@ template <int SPEC, bool REC>
 __global__ void trace_f64(TraceArgs P, double2* pray64, int super);
 __global__ void finalize(const double* E, const double* A, const double* Q2, long long nemit, int spe, int R,
                          int compat, double* Q, double* Eo, double* Ao, double* sd);
-__global__ void spline_pass(SplineArgs s);
+template <int AXIS>
+__global__ void spline_pass(SplinePass s);
 template <typename V, int NS>
 __global__ void reduce_rays(const V* pray, int tally, long long nslots, int R, long long slot0, const int4* slotinfo,
                             double* E, double* A, double* Q2);
@@ -201,7 +202,8 @@ struct dnsmc_solver {
     DevBuf<double> d_spw;
     std::vector<DevBuf<double>*> sp_dbufs;
     std::vector<DevBuf<int>*> sp_ibufs;
-    SplineArgs spa[kMaxLev][3];
+    SplinePass spa[3];
+    DevBuf<float> d_spx, d_spy;   // the coarse levels after the x and y passes
     bool spline_ready = false;
     // tables
     DevBuf<float> d_kq, d_Ib, d_Ibw, d_cdfb, d_cdfg, d_inv_emax;
@@ -388,47 +390,62 @@ static int prepare_spline(dnsmc_solver* s)
 {
     if (s->spline_ready || s->lev.size() < 2) return DNSMC_OK;
     const Level& L0 = s->lev[0];
-    size_t work = 0;
+    const size_t n1 = L0.n[1], n2 = L0.n[2];
+    memset(s->spa, 0, sizeof s->spa);
+    auto up_d = [&](const std::vector<double>& v) {
+        DevBuf<double>* b = new DevBuf<double>();
+        (void)b->upload(v, s->stream);
+        s->sp_dbufs.push_back(b);
+        return (const double*)b->p;
+    };
+    size_t nx = 0, ny = 0, work[3] = {(size_t)L0.n[0] * n1 * n2, 0, 0};
+    for (size_t l = 1; l < s->lev.size(); ++l) {
+        nx += (size_t)s->lev[l].n[0] * n1 * n2;
+        ny += (size_t)s->lev[l].n[0] * s->lev[l].n[1] * n2;
+    }
+    HIPCHK(s->d_spx.ensure(nx));
+    HIPCHK(s->d_spy.ensure(ny));
+    size_t ox = 0, oy = 0;
     for (size_t l = 1; l < s->lev.size(); ++l) {
         const Level& Lc = s->lev[l];
-        int nf[3] = {L0.n[0], L0.n[1], L0.n[2]}, nc[3] = {Lc.n[0], Lc.n[1], Lc.n[2]};
+        const int m0 = Lc.n[0], m1 = Lc.n[1];
         for (int a = 0; a < 3; ++a) {
             SplineAxis ax;
-            spline_axis_coeffs(L0.centres[a], nf[a], Lc.centres[a], nc[a], ax);
-            SplineArgs& A = s->spa[l][a];
-            memset(&A, 0, sizeof A);
-            auto up_d = [&](const std::vector<double>& v) {
-                DevBuf<double>* b = new DevBuf<double>();
-                (void)b->upload(v, s->stream);
-                s->sp_dbufs.push_back(b);
-                return (const double*)b->p;
-            };
+            spline_axis_coeffs(L0.centres[a], L0.n[a], Lc.centres[a], Lc.n[a], ax);
+            SplinePass& A = s->spa[a];
+            SplineLevel& V = A.lv[l - 1];
             DevBuf<int>* kb = new DevBuf<int>();
             HIPCHK(kb->upload(ax.klo, s->stream));
             s->sp_ibufs.push_back(kb);
-            A.sig = up_d(ax.sig); A.invp = up_d(ax.invp); A.y2f = up_d(ax.y2f);
-            A.c6 = up_d(ax.c6); A.ihl = up_d(ax.ihl); A.ihh = up_d(ax.ihh);
-            A.ca = up_d(ax.a); A.cb = up_d(ax.b); A.cA = up_d(ax.A); A.cB = up_d(ax.B);
-            A.klo = kb->p;
-            A.nf = nf[a];
-            A.nc = nc[a];
-            if (a == 0) {          // (n0,n1,n2) -> (m0,n1,n2): line l = j + n1 k
-                A.nlines = nf[1] * nf[2];
-                A.A = 1ll << 40; A.sa_in = nf[0]; A.sb_in = 0; A.st_in = 1;
-                A.sa_out = nc[0]; A.sb_out = 0; A.st_out = 1;
-            } else if (a == 1) {   // (m0,n1,n2) -> (m0,m1,n2): line l = i + m0 k
-                A.nlines = nc[0] * nf[2];
-                A.A = nc[0]; A.sa_in = 1; A.sb_in = (long long)nc[0] * nf[1]; A.st_in = nc[0];
-                A.sa_out = 1; A.sb_out = (long long)nc[0] * nc[1]; A.st_out = nc[0];
-            } else {               // (m0,m1,n2) -> (m0,m1,m2): line l = i + m0 j
-                A.nlines = nc[0] * nc[1];
-                A.A = 1ll << 40; A.sa_in = 1; A.sb_in = 0; A.st_in = (long long)nc[0] * nc[1];
-                A.sa_out = 1; A.sb_out = 0; A.st_out = (long long)nc[0] * nc[1];
+            if (l == 1) {
+                A.sig = up_d(ax.sig); A.invp = up_d(ax.invp); A.y2f = up_d(ax.y2f);
+                A.c6 = up_d(ax.c6); A.ihl = up_d(ax.ihl); A.ihh = up_d(ax.ihh);
+                A.nf = L0.n[a];
+                A.nlev = (int)s->lev.size() - 1;
+                A.fn1 = (int)n1;
+                A.fnbx = s->nbx[0];
+                A.fnby = s->nby[0];
             }
-            work = std::max(work, (size_t)A.nlines * A.nf);
+            V.ca = up_d(ax.a); V.cb = up_d(ax.b); V.cA = up_d(ax.A); V.cB = up_d(ax.B);
+            V.klo = kb->p;
+            V.nc = Lc.n[a];
+            V.m0 = m0;
+            V.m1 = m1;
+            V.nbx = s->nbx[l];
+            V.nby = s->nby[l];
+            V.nlines = (int)(a == 0 ? n1 * n2 : a == 1 ? m0 * n2 : (size_t)m0 * m1);
+            if (a > 0) {
+                V.work0 = work[a];
+                work[a] += (size_t)V.nlines * A.nf;
+            }
+            V.in = a == 1 ? s->d_spx.p + ox : s->d_spy.p + oy;
+            V.out = a == 0 ? s->d_spx.p + ox : s->d_spy.p + oy;   // (z: the level's field, per snapshot)
         }
+        ox += (size_t)m0 * n1 * n2;
+        oy += (size_t)m0 * m1 * n2;
     }
-    HIPCHK(s->d_spw.ensure(work));
+    HIPCHK(s->d_spw.ensure(std::max(work[0], std::max(work[1], work[2]))));
+    for (SplinePass& A : s->spa) A.work = s->d_spw.p;
     s->spline_ready = true;
     return DNSMC_OK;
 }
@@ -439,39 +456,18 @@ static int run_spline(dnsmc_solver* s, int snap)
     if (s->lev.size() < 2) return DNSMC_OK;
     int rc = prepare_spline(s);
     if (rc) return rc;
-    const Level& L0 = s->lev[0];
-    static DevBuf<float> tmpx, tmpy;   // per-process scratch for the intermediate passes
-    for (size_t l = 1; l < s->lev.size(); ++l) {
-        const Level& Lc = s->lev[l];
-        size_t nx = (size_t)Lc.n[0] * L0.n[1] * L0.n[2], ny = (size_t)Lc.n[0] * Lc.n[1] * L0.n[2];
-        HIPCHK(tmpx.ensure(nx));
-        HIPCHK(tmpy.ensure(ny));
-        for (int a = 0; a < 3; ++a) {
-            SplineArgs A = s->spa[l][a];
-            A.work = s->d_spw.p;
-            if (a == 0) {   // bricked fine field in, line l = j + n1 k
-                A.in = s->d_T[0].p + (size_t)snap * s->tstride[0];
-                A.out = tmpx.p;
-                A.in_bricked = 1;
-                A.fn1 = L0.n[1];
-                A.fnbx = s->nbx[0];
-                A.fnby = s->nby[0];
-            } else if (a == 1) {
-                A.in = tmpx.p;
-                A.out = tmpy.p;
-            } else {        // bricked coarse level out, line l = i + m0 j
-                A.in = tmpy.p;
-                A.out = s->d_T[l].p + (size_t)snap * s->tstride[l];
-                A.brick_out = 1;
-                A.m0 = Lc.n[0];
-                A.nbx = s->nbx[l];
-                A.nby = s->nby[l];
-            }
-            A.snap_in = A.snap_out = 0;
-            int nb = (A.nlines + 127) / 128;
-            hipLaunchKernelGGL(spline_pass, dim3(nb), dim3(128), 0, s->stream, A);
-            HIPCHK(hipGetLastError());
+    for (int a = 0; a < 3; ++a) {
+        SplinePass A = s->spa[a];
+        A.fine = s->d_T[0].p + (size_t)snap * s->tstride[0];
+        int nb = 0;
+        for (int l = 0; l < A.nlev; ++l) {
+            nb = a == 0 ? (A.lv[0].nlines + 63) / 64 : nb + (A.lv[l].nlines + 63) / 64;
+            if (a == 2) A.lv[l].out = s->d_T[l + 1].p + (size_t)snap * s->tstride[l + 1];
         }
+        const size_t lds = 6 * sizeof(double) * (size_t)A.nf + (a == 0 ? 64 * 17 * sizeof(float) : 0);
+        hipLaunchKernelGGL(HIP_KERNEL_NAME(a == 0 ? spline_pass<0> : a == 1 ? spline_pass<1> : spline_pass<2>), dim3(nb),
+                           dim3(64), lds, s->stream, A);
+        HIPCHK(hipGetLastError());
     }
     return DNSMC_OK;
 }
@@ -1489,16 +1485,20 @@ static int commit_field(dnsmc_solver* s, int snap)
     if (rc) return rc;
     // temperature range over every level (the spline can leave the fine range)
     HIPCHK(s->d_lohi.ensure(2 * s->lev.size()));
+    RangeArgs ra;
+    ra.nlev = (int)s->lev.size();
+    ra.keys = s->d_lohi.p;
     for (size_t l = 0; l < s->lev.size(); ++l) {
-        hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s->stream, s->d_lohi.p + 2 * l, 1ll, 0xFFFFFFFFu);
-        hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s->stream, s->d_lohi.p + 2 * l + 1, 1ll, 0u);
-        const int* ln = s->lev[l].n;
-        const long long ncl = (long long)ln[0] * ln[1] * ln[2];
-        const int nb = (int)std::min<long long>((ncl + 255) / 256, (long long)s->ncu * 16);
-        hipLaunchKernelGGL(t_range, dim3(nb), dim3(256), 0, s->stream, s->d_T[l].p + (size_t)snap * s->tstride[l],
-                           ln[0], ln[1], ln[2], s->nbx[l], s->nby[l], s->d_lohi.p + 2 * l);
-        HIPCHK(hipGetLastError());
+        RangeLevel& L = ra.lv[l];
+        L.T = s->d_T[l].p + (size_t)snap * s->tstride[l];
+        for (int a = 0; a < 3; ++a) L.n[a] = s->lev[l].n[a];
+        L.nbricks = s->nbx[l] * s->nby[l] * ((L.n[2] + 3) / 4);
+        L.fd_nbx = make_fastdiv((uint32_t)s->nbx[l]);
+        L.fd_nby = make_fastdiv((uint32_t)s->nby[l]);
     }
+    hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s->stream, s->d_lohi.p, 2ll * ra.nlev, 0xFFFFFFFFu);
+    hipLaunchKernelGGL(t_range, dim3(std::min(s->ncu, (ra.lv[0].nbricks + 15) / 16)), dim3(1024), 0, s->stream, ra);
+    HIPCHK(hipGetLastError());
     std::vector<unsigned> lohi(2 * s->lev.size());
     HIPCHK(hipMemcpyAsync(lohi.data(), s->d_lohi.p, lohi.size() * sizeof(unsigned), hipMemcpyDeviceToHost, s->stream));
     HIPCHK(hipStreamSynchronize(s->stream));
@@ -1510,16 +1510,16 @@ static int commit_field(dnsmc_solver* s, int snap)
     };
     float lo = 0.f, hi = 0.f;
     for (size_t l = 0; l < s->lev.size(); ++l) {
-        const float a = key_float(lohi[2 * l]), b = key_float(lohi[2 * l + 1]);
+        const float a = key_float(lohi[2 * l]), b = key_float(~lohi[2 * l + 1]);
         lo = l == 0 ? a : std::min(lo, a);
         hi = l == 0 ? b : std::max(hi, b);
     }
     s->Tlo_snap[snap] = lo;
     s->Thi_snap[snap] = hi;
-    s->Tmax_snap[snap] = key_float(lohi[1]);   // level-0 maximum
+    s->Tmax_snap[snap] = key_float(~lohi[1]);   // level-0 maximum
     s->slab_open[snap] = 0;
     // fine field: positive and finite everywhere (a NaN shows in the level-0 bounds)
-    if (!(key_float(lohi[0]) > 0.f) || !std::isfinite(key_float(lohi[1]))) {
+    if (!(key_float(lohi[0]) > 0.f) || !std::isfinite(key_float(~lohi[1]))) {
         s->field_set[snap] = 0;
         return fail(DNSMC_ERANGE, "temperature field holds a non-positive or non-finite value");
     }

@@ -10,8 +10,6 @@
 
 namespace dn {
 
-constexpr int kMaxLev = 6;
-
 // Spectral tables as read (reference layouts, code/NarrowBand.h:3-8 and
 // code/read_tables.cpp): kq[b][t][g], prob[t][b] band CDF, probg[t][b][g] g-CDF.
 struct Tables {
