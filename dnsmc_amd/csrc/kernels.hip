@@ -2804,6 +2804,16 @@ __global__ void results_to_fortran(const int* emit, long long nemit, const doubl
     varf[o] = (float)sd[e];
 }
 
+// The same where every interior entry has a result, in row order: [Q | standard
+// error] as FP32, for the host to place.
+__global__ void results_to_f32(const double* Q, const double* sd, long long n, float* out)
+{
+    const long long e = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (e >= n) return;
+    out[e] = (float)Q[e];
+    out[n + e] = (float)sd[e];
+}
+
 // fix_rad (code/fix_var.f:75-121) for one rank's k range, from the device
 // results: divQ(i, jl, k - k0 + 1) = Q / stefan / Tc^4 and vcore likewise from
 // the standard error, for the emitters in the solver's j slab [jlo, jlo + nj)

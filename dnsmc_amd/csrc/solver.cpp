@@ -21,6 +21,7 @@
 
 #include "kernels.h"
 #include "solver.h"
+#include "transfer.h"
 
 namespace dn {
 // kernels.hip
@@ -60,6 +61,7 @@ __global__ void mlp_samples(FeatArgs f, const int4* slotinfo, long long slot0, i
 __global__ void mlp_features(FeatArgs f, const int4* slotinfo, long long n, float* X);
 __global__ void fill_u32(unsigned* p, long long n, unsigned v);
 __global__ void t_to_u(const float* T, float* U, long long n, float inv_dT, float mT0, float top, float lo);
+__global__ void results_to_f32(const double* Q, const double* sd, long long n, float* out);
 __global__ void ghost_to_bricks(const float* Tg, int n0, int n1, int n2, float* T, int nbx, int nby);
 __global__ void results_to_fortran(const int* emit, long long nemit, const double* Q, const double* sd, int n0,
                                    int n1, int jlo, int nj, int n2, float* resf, float* varf);
@@ -186,6 +188,7 @@ struct dnsmc_solver {
     DevBuf<unsigned> d_lohi;
     DevBuf<double> d_slab;         // staging of the DNS coupling slabs
     DevBuf<float> d_stage;         // staging of host temperature fields
+    HostPipe pipe_host;            // copies from and to the caller's arrays
     DevBuf<float> d_T[kMaxLev];
     DevBuf<float> d_U[kMaxLev];    // table coordinates of the sliced-table traversal
     long long ncell[kMaxLev] = {0, 0, 0, 0, 0, 0};     // cells per level
@@ -220,6 +223,8 @@ struct dnsmc_solver {
     DevBuf<int4> d_slotinfo;    // processing slot -> {tally slot, cell, bricked index, packed i|j|k}
     bool emit_dirty = true;
     bool order_yfast = false;      // the slot tables' emitter order (brick_order)
+    bool emit_rows = false;        // emit holds that slab's cells in row order (also the default, every cell of one slab)
+    bool last_rows = false;        // ... at the last run
     bool emit_is_slab = false;     // emit holds the j slab from ystart (dnsmc_set_emitters_slab)
     // ray batches are pipelined over kPipes streams, each with its own buffers,
     // so the tail of one traversal launch overlaps the next batch
@@ -1425,6 +1430,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     s->last_spe = spe;
     s->last_nemit = na ? 0 : nemit;   // an allocation-free run's results are the caller's only
     s->last_ystart = s->ystart;
+    s->last_rows = s->emit_rows;
     s->nsteps_src = nsteps;
     s->running = true;
     return DNSMC_OK;
@@ -1474,6 +1480,33 @@ static int fetch_perm(const T* dev, long long c, const std::vector<long long>& p
     for (long long q = 0; q < c; ++q)
         if (perm[q] < c) out[perm[q]] = tmp[q];
     return DNSMC_OK;
+}
+
+// The caller's array to the device, in stream order; the array is free again on
+// return unless HIP knows its memory (a copy in the stream then).
+static hipError_t upload_host(dnsmc_solver* s, void* dev, const void* host, size_t bytes)
+{
+    if (bytes < HostPipe::kParallel || !HostPipe::pageable(host))
+        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s->stream);
+    const HostRows job = host_block(dev, host, bytes);
+    return s->pipe_host.run(s->dev, s->stream, true, &job, 1);
+}
+
+// Device ranges into the caller's arrays, done on return.
+static hipError_t download_host(dnsmc_solver* s, const HostRows* jobs, int n)
+{
+    HostRows pg[4];
+    int np = 0;
+    for (int i = 0; i < n; ++i) {
+        if (HostPipe::pageable(jobs[i].host)) {
+            pg[np++] = jobs[i];
+            continue;
+        }
+        const hipError_t e = hipMemcpyAsync(jobs[i].host, jobs[i].dev, jobs[i].bytes, hipMemcpyDeviceToHost, s->stream);
+        if (e != hipSuccess) return e;
+    }
+    const hipError_t e = s->pipe_host.run(s->dev, s->stream, false, pg, np);
+    return e != hipSuccess ? e : hipStreamSynchronize(s->stream);
 }
 
 // After the fine field of snapshot `snap` is on the device: coarse levels by
@@ -1590,6 +1623,7 @@ int dnsmc_create(const dnsmc_config* cfg, dnsmc_solver** out)
     long long n = (long long)cfg->n[0] * cfg->n[1] * cfg->n[2];
     s->emit.resize(n);
     for (long long i = 0; i < n; ++i) s->emit[i] = (int)i;
+    s->emit_rows = cfg->p_row == 1;
     *out = s;
     return DNSMC_OK;
 }
@@ -1693,7 +1727,7 @@ int dnsmc_set_field(dnsmc_solver* s, int snap, const float* T, int is_device)
     const float* src = T;
     if (!is_device) {
         HIPCHK(s->d_stage.ensure(gsz));
-        HIPCHK(hipMemcpyAsync(s->d_stage.p, T, gsz * sizeof(float), hipMemcpyHostToDevice, s->stream));
+        HIPCHK(upload_host(s, s->d_stage.p, T, gsz * sizeof(float)));
         src = s->d_stage.p;
     }
     const long long nc = (long long)n0 * n1 * n2;
@@ -1736,7 +1770,7 @@ int dnsmc_fix_temp_slab(dnsmc_solver* s, int snap, const double* cnew, const int
     // cnew(0:n0+1, nj, nk) of the rank, i fastest
     const size_t cnt = (size_t)(n[0] + 2) * len[1] * len[2];
     HIPCHK(s->d_slab.ensure(cnt));
-    HIPCHK(hipMemcpyAsync(s->d_slab.p, cnew, cnt * sizeof(double), hipMemcpyHostToDevice, s->stream));
+    HIPCHK(upload_host(s, s->d_slab.p, cnew, cnt * sizeof(double)));
     const long long nc = (long long)len[0] * len[1] * len[2];
     const int nb = (int)std::min<long long>((nc + 255) / 256, (long long)s->ncu * 16);
     hipLaunchKernelGGL(slab_to_field, dim3(nb), dim3(256), 0, s->stream, (const double*)s->d_slab.p, n[0], n[1], n[2],
@@ -1783,9 +1817,8 @@ int dnsmc_fix_rad_slab(dnsmc_solver* s, int snap, const int* startc, const int* 
                        (const double*)(s->d_sd.p + (size_t)snap * ne), n[0], n[1], s->last_ystart - 1, nj, startc[2] - 1, nk,
                        stefan, tc4, dq, dv);
     HIPCHK(hipGetLastError());
-    HIPCHK(hipMemcpyAsync(divQ, dq, cnt * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipMemcpyAsync(vcore, dv, cnt * sizeof(double), hipMemcpyDeviceToHost, s->stream));
-    HIPCHK(hipStreamSynchronize(s->stream));
+    const HostRows jobs[2] = {host_block(dq, divQ, cnt * sizeof(double)), host_block(dv, vcore, cnt * sizeof(double))};
+    HIPCHK(download_host(s, jobs, 2));
     return DNSMC_OK;
 }
 
@@ -1842,7 +1875,7 @@ int dnsmc_set_emitters_slab(dnsmc_solver* s, int ystart)
         for (int j = ystart - 1; j < ystart - 1 + nj; ++j)
             for (int i = 0; i < n0; ++i) s->emit.push_back(i + n0 * (j + n1 * k));
     s->emit_dirty = true;
-    s->emit_is_slab = true;
+    s->emit_is_slab = s->emit_rows = true;
     s->ystart = ystart;
     return DNSMC_OK;
 }
@@ -1855,7 +1888,7 @@ int dnsmc_set_emitters_list(dnsmc_solver* s, const int* cells, int ncells)
         if (cells[i] < 0 || cells[i] >= ntot) return fail(DNSMC_EINVAL, "emitter cell out of range");
     s->emit.assign(cells, cells + ncells);
     s->emit_dirty = true;
-    s->emit_is_slab = false;
+    s->emit_is_slab = s->emit_rows = false;
     s->ystart = 1;
     return DNSMC_OK;
 }
@@ -1894,10 +1927,13 @@ int dnsmc_get_results(dnsmc_solver* s, int snap, double* Q, double* E, double* A
     if (rc) return rc;
     if (snap < 0 || snap >= s->cfg.nsnap || s->last_nemit == 0) return fail(DNSMC_ESTATE, "no results for snapshot");
     size_t n = (size_t)s->last_nemit, o = (size_t)snap * n;
-    if (Q) HIPCHK(hipMemcpy(Q, s->d_Q.p + o, n * sizeof(double), hipMemcpyDeviceToHost));
-    if (E) HIPCHK(hipMemcpy(E, s->d_Eo.p + o, n * sizeof(double), hipMemcpyDeviceToHost));
-    if (A) HIPCHK(hipMemcpy(A, s->d_Ao.p + o, n * sizeof(double), hipMemcpyDeviceToHost));
-    if (sdev) HIPCHK(hipMemcpy(sdev, s->d_sd.p + o, n * sizeof(double), hipMemcpyDeviceToHost));
+    HostRows jobs[4];
+    int nj = 0;
+    if (Q) jobs[nj++] = host_block(s->d_Q.p + o, Q, n * sizeof(double));
+    if (E) jobs[nj++] = host_block(s->d_Eo.p + o, E, n * sizeof(double));
+    if (A) jobs[nj++] = host_block(s->d_Ao.p + o, A, n * sizeof(double));
+    if (sdev) jobs[nj++] = host_block(s->d_sd.p + o, sdev, n * sizeof(double));
+    HIPCHK(download_host(s, jobs, nj));
     return DNSMC_OK;
 }
 
@@ -1911,15 +1947,34 @@ int dnsmc_get_results_fortran(dnsmc_solver* s, int snap, float* resfort, float* 
     const int n0 = s->cfg.n[0], n1 = s->cfg.n[1], n2 = s->cfg.n[2];
     const int nj = n1 / s->cfg.p_row;
     const size_t fsz = (size_t)(n0 + 2) * (nj + 2) * (n2 + 2);
+    const long long ne = s->last_nemit;
+    if (s->last_rows && HostPipe::pageable(resfort) && HostPipe::pageable(varfort)) {
+        // every interior entry has a result, in row order: the rows as FP32, and
+        // each row to its place (the ghost entries are not touched)
+        HIPCHK(s->d_stage.ensure(2 * (size_t)ne));
+        hipLaunchKernelGGL(results_to_f32, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s->stream,
+                           (const double*)(s->d_Q.p + (size_t)snap * ne), (const double*)(s->d_sd.p + (size_t)snap * ne), ne,
+                           s->d_stage.p);
+        HIPCHK(hipGetLastError());
+        const ptrdiff_t p1 = (ptrdiff_t)(n0 + 2) * sizeof(float), p2 = p1 * (nj + 2);
+        HostRows job = host_block(s->d_stage.p, (const char*)resfort + sizeof(float) + p1 + p2, 2 * (size_t)ne * sizeof(float));
+        job.row = (size_t)n0 * sizeof(float);
+        job.n1 = nj;
+        job.n2 = n2;
+        job.p1 = p1;
+        job.p2 = p2;
+        job.p3 = (const char*)varfort - (const char*)resfort;
+        HIPCHK(s->pipe_host.run(s->dev, s->stream, false, &job, 1));
+        return DNSMC_OK;
+    }
     // the caller's arrays round-trip through the device so that the entries
-    // the results do not cover (ghost layers) keep their values; the interior
-    // is written by a kernel from the FP64 results
+    // the results do not cover (ghost layers, other cells) keep their values;
+    // the rest is written by a kernel from the FP64 results
     HIPCHK(s->d_stage.ensure(2 * fsz));
     float* dq = s->d_stage.p;
     float* dv = s->d_stage.p + fsz;
     HIPCHK(hipMemcpyAsync(dq, resfort, fsz * sizeof(float), hipMemcpyHostToDevice, s->stream));
     HIPCHK(hipMemcpyAsync(dv, varfort, fsz * sizeof(float), hipMemcpyHostToDevice, s->stream));
-    const long long ne = s->last_nemit;
     hipLaunchKernelGGL(results_to_fortran, dim3((unsigned)((ne + 255) / 256)), dim3(256), 0, s->stream,
                        (const int*)s->d_emit.p, ne, (const double*)(s->d_Q.p + (size_t)snap * ne),
                        (const double*)(s->d_sd.p + (size_t)snap * ne), n0, n1, s->last_ystart - 1, nj, n2, dq, dv);
