@@ -788,6 +788,14 @@ __device__ __forceinline__ int quad_sum(int v)
     v += quad_i<kQuadXor1>(v);
     return v + quad_i<kQuadXor2>(v);
 }
+// Lane a of a quad: the quad's sum of v[a].
+__device__ __forceinline__ int quad_spread(const int* v, int a)
+{
+    const bool odd = a & 1, hi = a & 2;
+    const int p = (odd ? v[1] : v[0]) + quad_i<kQuadXor1>(odd ? v[0] : v[1]);
+    const int q = (odd ? v[3] : v[2]) + quad_i<kQuadXor1>(odd ? v[2] : v[3]);
+    return (hi ? q : p) + quad_i<kQuadXor2>(hi ? p : q);
+}
 __device__ __forceinline__ int quad_max(int v)
 {
     v = max(v, quad_i<kQuadXor1>(v));
@@ -1664,8 +1672,11 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     // the exit face read ahead.  Then the batch's field loads and table
     // lookups run in parallel, crossing 4 k + j on lane j, and tau and G
     // follow in crossing order with the main loop's arithmetic (a crossing
-    // past the ray's end has length 0 and adds 0): 122 ns per crossing, the
-    // solve 46 -> 24 ms (18 to 24 with retiring waves, above).
+    // past the ray's end has length 0 and adds 0): 122 ns per crossing with
+    // a branch per crossing for walls, wraps and ties, 105 ns without (below):
+    // a solve bound by one ray of 16000 crossings 2.22 -> 2.05 ms.  Batches of
+    // 8, 16, 24 and 32 crossings: 2.34, 2.03, 2.18 and 2.22 ms there.  The
+    // first solve 46 -> 22 ms (18 with retiring waves, above).
     if (__ballot(alive)) {
         __builtin_amdgcn_s_setprio(3);   // ahead of the waves that still trace the bulk
         const unsigned long long am = __ballot(alive);
@@ -1712,83 +1723,97 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         // the face table from gb - st (a word past the axis's faces is one of its
         // LDS neighbours and is not used)
         auto face_w = [&](int byte, int i) -> float { return lds_f(byte + (i << 2)); };
+        // the walk's per-lane constants (lane 3: one cell, never left): the
+        // cell behind the domain's last (the other end's, or out of range at a
+        // wall) and the coordinate there
+        const uint32_t wn = ax3 ? 1u : (uint32_t)qn;
+        const int wrapc = ax3 ? 0 : (per ? (neg ? qn - 1 : 0) : (neg ? -1 : qn));
+        const float wrapp = per && !ax3 ? face_w(gb - 4 * st - (neg ? 0 : 4), neg ? qn : 0) : 0.0f;
+        const int xb = gb - 4 * st;                      // exit face of cell 0
         while (__ballot(run)) {
             int lim = run ? min(kDrain, qmaxs - qcnt) : 0;
             int wall = -1;
-            // a frozen quad (no ray, or its ray hit a wall inside the batch) has
-            // length-0 crossings and does not move
-            unsigned long long live = __ballot(run);
-            int nlive = __popcll(live) >> 2;
+            // (a quad without a running ray moves within the domain, or not at all,
+            // and its crossings have length 0)
+            qc = run ? qc : 0;
             qs = run ? qs : 0.0f;
             qi = run ? qi : 0.0f;
-            float dsv[kDrain];
-            int oid[kDrain / 4], lin[kDrain / 4];
-            float g = face_w(gb, qc), h = face_w(gb + 4 * st, qc);
+            float dsv[kDrain], Tv[kDrain / 4];
+            int lin[kDrain / 4];
+            // The walk, without a branch and with nothing through scalar registers: a
+            // lane moves when its face is the nearest, wraps and walls follow from
+            // its cell (past a wall the face is at 3e38 and the cell stays out of
+            // range: nout counts the crossings since).  Axes that tie show in the
+            // number of moves; the batch is then walked again, the last of them
+            // moving first.
+            const float qp0 = qp, qf0 = qf;
+            const int qc0 = qc;
+            int nout, nm;
+            for (bool careful = false;; careful = true) {
+                nout = nm = 0;
+                auto behind = [&](int c, bool& out) -> int {
+                    out = (uint32_t)(c + st) >= wn;
+                    return out ? wrapc : c + st;
+                };
+                bool o1, o2;
+                int cn = behind(qc, o1);
+                float qa = o1 ? wrapp : qf;              // the coordinate behind the exit face
+                float g = face_w(xb, cn);
+                float h = face_w(xb, behind(cn, o2));
 #pragma unroll
-            for (int k = 0; k < kDrain / 4; ++k) {
-                int ov[4];
-                oid[k] = lin[k] = 0;
+                for (int k = 0; k < kDrain / 4; ++k) {
+                    int ov[4];
+                    lin[k] = 0;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int u = 4 * k + j;
-                    ov[j] = lds_i(ob + (qc << 2));
-                    const float d = (qf - qp) * qi;
-                    const float ds = quad_min(d);
-                    dsv[u] = ds;
-                    unsigned long long em = __ballot(d == ds) & live;
-                    qp = __builtin_amdgcn_inverse_ballot_w64(em) ? qf : fmaf(ds, qs, qp);
-                    // of several axes at the same distance the last one moves
-                    if (__builtin_expect(__popcll(em) != nlive, 0))
-                        em &= ~((em >> 1) | ((em >> 2) & 0x1111111111111111ull));
-                    const bool mv = __builtin_amdgcn_inverse_ballot_w64(em);
-                    if (REC) {
-                        const int l = quad_sum(qc * qstride);
-                        lin[k] = a == j ? l : lin[k];
-                    }
-                    qc += mv ? st : 0;
-                    qf = mv ? g : qf;
-                    g = mv ? h : g;
-                    const bool out = (uint32_t)qc >= (uint32_t)qn;
-                    if (__builtin_expect(__ballot(out) != 0ull, 0)) {
-                        int w = -1;
-                        if (out) {
-                            if (per) {
-                                qc = neg ? qn - 1 : 0;
-                                qp = face_w(gb - 8 * st, neg ? qn - 1 : 0);
-                            } else {
-                                w = bcbit;
-                                qc -= st;
-                            }
-                            qf = face_w(gb - 4 * st, qc);
-                            g = face_w(gb, qc);
+                    for (int j = 0; j < 4; ++j) {
+                        const int u = 4 * k + j;
+                        ov[j] = lds_i(ob + (int)(min((uint32_t)qc, wn - 1u) << 2));
+                        const float d = (qf - qp) * qi;
+                        const float ds = quad_min(d);
+                        dsv[u] = ds;
+                        bool mv = d == ds, tie = false;
+                        if (__builtin_expect(careful, 0)) {
+                            const int e = mv ? 1 : 0;
+                            tie = (e & (quad_i<0xF9>(e) | quad_i<0xFE>(e))) != 0;   // (lanes a + 1 and a + 2)
+                            mv = mv && !tie;
                         }
-                        w = quad_max(w);
-                        const bool hit = w >= 0;
-                        wall = hit && u < lim ? w : wall;
-                        lim = hit ? min(lim, u + 1) : lim;
-                        qs = hit ? 0.0f : qs;
-                        qi = hit ? 0.0f : qi;
-                        live &= ~__ballot(hit);
-                        nlive = __popcll(live) >> 2;
-                        __builtin_amdgcn_s_waitcnt(0xC07F);   // (lgkmcnt(0) here, not on the common path)
+                        if (REC) {
+                            const int l = quad_sum(qc * qstride);
+                            lin[k] = a == j ? l : lin[k];
+                        }
+                        const float pn = tie ? qf : fmaf(ds, qs, qp);
+                        qp = mv ? qa : pn;
+                        nm += mv ? 1 : 0;
+                        qf = mv ? g : qf;
+                        g = mv ? h : g;
+                        qc = mv ? cn : qc;
+                        nout += (uint32_t)qc >= wn ? 1 : 0;
+                        cn = behind(qc, o1);
+                        qa = o1 ? wrapp : qf;
+                        h = face_w(xb, behind(cn, o2));
                     }
-                    h = face_w(gb + 4 * st, qc);
-                }
-                // the cells' field offsets: crossing 4 k + j to lane j
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const int ou = quad_sum(ax3 ? 0 : ov[j]);
-                    oid[k] = a == j ? ou : oid[k];
+                    for (int j = 0; j < 4; ++j) ov[j] = ax3 ? 0 : ov[j];   // (here, not on the chain: the reads have come)
+                    Tv[k] = load_T(qT, quad_spread(ov, a));
                 }
+                if (careful || !__ballot(run && quad_sum(nm) != kDrain)) break;
+                qp = qp0;
+                qf = qf0;
+                qc = qc0;
+            }
+            if (__ballot(nout > 0 && run)) {
+                // the first wall of the batch, if it comes before the step cap
+                const int uh = kDrain - nout, um = quad_min_i(uh);
+                const int w = quad_max(nout > 0 && uh == um ? bcbit : -1);
+                wall = um < lim ? w : -1;
+                lim = min(lim, um + 1);
             }
             if (__ballot(run && lim < kDrain)) {             // the step cap inside the batch
 #pragma unroll
                 for (int u = 0; u < kDrain; ++u) dsv[u] = u < lim ? dsv[u] : 0.0f;
             }
-            // the cells' temperatures and lookups
-            float Tv[kDrain / 4], kap[kDrain / 4], ibv[kDrain / 4], tk[kDrain / 4], dg[kDrain / 4];
-#pragma unroll
-            for (int k = 0; k < kDrain / 4; ++k) Tv[k] = load_T(qT, oid[k]);
+            // the lookups
+            float kap[kDrain / 4], ibv[kDrain / 4], tk[kDrain / 4], dg[kDrain / 4];
 #pragma unroll
             for (int k = 0; k < kDrain / 4; ++k) table_at(Tv[k], qkrow, qibrow, kap[k], ibv[k]);
             // optical depth in crossing order (every lane of the quad), kept by
