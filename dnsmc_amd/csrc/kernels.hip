@@ -1201,7 +1201,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     // crossings stops claiming, so that it reaches the drain below (over four
     // times faster per crossing) while the other waves trace the rest.  At most
     // retire_most waves of the launch do for rays beyond retire_steps (counted
-    // in claim word 16), as many beyond four times that for the waves that were
+    // in claim word 16), as many beyond twice that for the waves that were
     // refused (word 17), and so on up to word 19: the longest rays are not left
     // out, and the other waves remain to claim what is left.
     uint32_t last_c = 0, asked = 0;
@@ -1211,7 +1211,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
         uint32_t k = 0;
         if (lane == 0) k = atomicAdd(P.claim + 16u + asked, 1u);
         ++asked;
-        ask_at = asked < 4u ? 4 * ask_at : 0x7FFFFFFF;
+        ask_at = asked < 4u ? 2 * ask_at : 0x7FFFFFFF;
         return __builtin_amdgcn_readfirstlane(k) < P.retire_most;
     };
     // kappa and Ib of a ray's (band, g) rows at a field value (sliced tables:

@@ -636,16 +636,18 @@ static hipError_t launch_trace_t(bool amc, int ncu, int max_blocks, size_t lds, 
     int nb = per_cu * ncu;
     nb = std::min(nb, TAB == kTabSliced ? std::max(8, max_blocks / 4) : max_blocks);
     nb = std::max(8, nb / 8 * 8);
-    // retiring waves (kernels.hip): rays beyond 2048 crossings, in about the
-    // last 64 claims per wave, at most one wave of 16.  A 64x96x64 solve of 500
-    // rays/cell (94 claims per wave): 23.8 ms without, 18.1 / 18.4 / 21.9 ms
-    // beyond 1024 / 2048 / 4096 crossings, 22.1 / 21.0 / 18.1 / 17.1 / 24.1 ms
-    // in the last 16 / 32 / 64 / 128 / 256 claims; 384x256x256 at 100 rays/cell
-    // (1200 claims per wave) 398 ms either way, 440 ms when any wave may retire
-    // at any time.
+    // retiring waves (kernels.hip): rays beyond 1536 crossings, in about the
+    // last 64 claims per wave, at most one wave of 16 (and as many beyond each of
+    // the next three doublings).  A 64x96x64 solve of 500 rays/cell (94 claims
+    // per wave): 23.8 ms without; beyond 2048, 8192, ... crossings 21.5 ms (which
+    // of the rays that reach 2048 at about the same time win is chance, and
+    // 8192 crossings are 7 ms of the bulk's pace); in doublings from 1024 / 1536 /
+    // 2048 / 3072 on 18.1 / 18.1 / 19.2 / 19.5 ms.  384x256x256 at 100 rays/cell
+    // (1200 claims per wave) the same within 0.3 % either way, 440 against 398 ms
+    // when any wave may retire at any time.
     const long long waves = (long long)nb * (threads / 64);
     const long long nclaim = (((P.nrays + P.super - 1) / P.super + 7) / 8) * P.nsnap_launch;   // per XCD share
-    P.retire_steps = 2048;
+    P.retire_steps = 1536;
     P.retire_from = (unsigned)std::max(0ll, nclaim - 64 * waves / 8);
     P.retire_most = (unsigned)(waves / 16);
     hipLaunchKernelGGL(k, dim3(nb), dim3(threads), lds, st, P);
