@@ -2888,6 +2888,19 @@ __global__ void fill_u32(unsigned* p, long long n, unsigned v)
     if (i < n) p[i] = v;
 }
 
+// A run's start: the tallies and the two step counters, one launch (four fills
+// before; a solve of 2e5 rays waits for each launch).
+__global__ void clear_tallies(double* E, double* A, double* Q2, long long n, unsigned long long* nsteps)
+{
+    const long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (i < n) {
+        E[i] = 0.0;
+        A[i] = 0.0;
+        Q2[i] = 0.0;
+    }
+    if (i < 2) nsteps[i] = 0ull;
+}
+
 __global__ void fill_f64(double* p, long long n, double v)
 {
     long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x;

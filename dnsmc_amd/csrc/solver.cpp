@@ -41,6 +41,7 @@ template <typename V, int NS>
 __global__ void reduce_rays(const V* pray, int tally, long long nslots, int R, long long slot0, const int4* slotinfo,
                             double* E, double* A, double* Q2);
 __global__ void fill_f64(double* p, long long n, double v);
+__global__ void clear_tallies(double* E, double* A, double* Q2, long long n, unsigned long long* nsteps);
 __global__ void cand_scan(TraceArgs P, uint32_t nfin, uint32_t* list);
 // mlp.hip
 __global__ void mlp_proposal(GenArgs a, float* cdf);
@@ -919,14 +920,11 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     s->ev_used = 0;
     memset(&s->st, 0, sizeof s->st);
     s->t0 = std::chrono::steady_clock::now();
-    // counters are cleared by fill kernels (stream-ordered, capture-safe)
-    hipLaunchKernelGGL(fill_u32, dim3(1), dim3(64), 0, s->stream, (unsigned*)nsteps, 4ll, 0u);
+    // tallies and counters are cleared by kernels (stream-ordered, capture-safe)
     {
-        long long n = nslots * c.nsnap;
-        int nb = (int)((n + 255) / 256);
-        hipLaunchKernelGGL(fill_f64, dim3(nb), dim3(256), 0, s->stream, tE, n, 0.0);
-        hipLaunchKernelGGL(fill_f64, dim3(nb), dim3(256), 0, s->stream, tA, n, 0.0);
-        hipLaunchKernelGGL(fill_f64, dim3(nb), dim3(256), 0, s->stream, tQ2, n, 0.0);
+        const long long n = nslots * c.nsnap;
+        hipLaunchKernelGGL(clear_tallies, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s->stream, tE, tA, tQ2, n, nsteps);
+        HIPCHK(hipGetLastError());
     }
     HIPCHK(hipEventRecord(s->ev_ready, s->stream));
     for (int p = 1; p < npipes; ++p) HIPCHK(hipStreamWaitEvent(s->pipe[p].stream, s->ev_ready, 0));
