@@ -39,3 +39,23 @@ def test_compat_descriptors(oracle, ck_table_dir, srt, sobol, photmax):
             np.testing.assert_array_equal(got["w0"], ref["w0"])
             np.testing.assert_array_equal(got["w1"], ref["w1"])
             np.testing.assert_allclose(got["w"], ref["w"], rtol=2e-7)
+
+
+@pytest.mark.parametrize("photmax", [255, 256, 257, 700, 5000])
+@pytest.mark.parametrize("levels", [1, 2])
+def test_shared_slot_tallies(ck_table_dir, levels, photmax):
+    """The tallies of launches with 256 rays per slot and more (16 lanes' sums at
+    a time) and less, against the ordered FP64 sums of the same rays: only the
+    order of FP64 additions differs."""
+    res = {}
+    for tally in (0, 1):
+        cfg = workloads.channel_config((16, 4, 4), spectral=0, Tw=573.0, table_dir=ck_table_dir[0], mode=1, srt=0, sobol=1,
+                                       photmax=photmax, nvar=3, num_streams=16, grid_num=levels, tally=tally)
+        S = dnsmc_amd.Solver(cfg)
+        S.load_tables()
+        S.set_field(0, workloads.ghosted(workloads.field_profile_noise(7, (16, 4, 4))))
+        S.run()
+        res[tally] = (S.results(0), S.stats()["n_steps"])
+    assert res[0][1] == res[1][1]
+    for k in ("E", "A"):
+        np.testing.assert_allclose(res[0][0][k], res[1][0][k], rtol=1e-11, atol=0)
