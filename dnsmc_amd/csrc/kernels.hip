@@ -963,13 +963,14 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     if (SPEC == kSpecTable && TAB == kTabIbLds)
         for (int i = threadIdx.x; i < P.nB * P.nT; i += blockDim.x) s_ib[i] = P.Ib[i];
     if (SPEC == kSpecTable && TAB == kTabSliced) {
+        // (a slice that reaches the table's top may end with its last node again)
         for (int i = threadIdx.x; i < P.nB * nw; i += blockDim.x) {
             const int r = i / nw;
-            s_ib[i] = P.Ib[r * P.nT + P.tab_lo + (i - r * nw)];
+            s_ib[i] = P.Ib[r * P.nT + min(P.tab_lo + (i - r * nw), P.nT - 1)];
         }
         for (int i = threadIdx.x; i < P.nB * P.nQ * nw; i += blockDim.x) {
             const int r = i / nw;
-            s_kq[i] = P.kq[r * P.nT + P.tab_lo + (i - r * nw)];
+            s_kq[i] = P.kq[r * P.nT + min(P.tab_lo + (i - r * nw), P.nT - 1)];
         }
     }
     __syncthreads();

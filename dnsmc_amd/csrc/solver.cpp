@@ -990,13 +990,15 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             return std::min(t0, d.nT - 2);
         };
         const int lo = node(tlo), hi = node(thi);
-        const int nw = hi + 2 - lo;
+        // the sliced lookup takes coordinates below the slice's last node: where a
+        // coarse level's spline overshoots the table (level 0 may not reach its
+        // top), the table's last node is held twice
+        const int over = fmaf(thi, d.inv_dT, d.mT0) >= (float)(d.nT - 1) ? 1 : 0;
+        const int nw = hi + 2 - lo + over;
         const size_t sliced = lds_trace + sizeof(float) * (size_t)d.nB * (d.nQ + 1) * nw;
         const char* force = getenv("DNSMC_TABLES");   // "global": keep the tables out of LDS
         const bool allow = !(force && !strcmp(force, "global"));
-        // (the sliced lookup takes coordinates below the table's last node)
-        const bool below_top = fmaf(thi, d.inv_dT, d.mT0) < (float)(d.nT - 1);
-        if (allow && below_top && sliced <= s->lds_max) {
+        if (allow && sliced <= s->lds_max) {
             tab = kTabSliced;
             P.tab_lo = lo;
             P.tab_nw = nw;
@@ -1421,7 +1423,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     s->st.n_rays = nslots * (long long)R * c.nsnap;
     s->st.table_mode = tab;
     s->st.table_lo = P.tab_lo;
-    s->st.table_nw = P.tab_nw;
+    s->st.table_nw = std::min(P.tab_nw, d.nT - P.tab_lo);   // (the last node held twice counts once)
     s->st.n_pipes = npipes;
     s->st.Tmax = d.Tmax;
     s->st.kappamax = d.kappamax;
