@@ -189,7 +189,7 @@ struct dnsmc_solver {
     DevBuf<unsigned> d_lohi;
     DevBuf<double> d_slab;         // staging of the DNS coupling slabs
     DevBuf<float> d_stage;         // staging of host temperature fields
-    HostPipe pipe_host;            // copies from and to the caller's arrays
+    HostPipe pipe_host;            // copies to the caller's arrays
     DevBuf<float> d_T[kMaxLev];
     DevBuf<float> d_U[kMaxLev];    // table coordinates of the sliced-table traversal
     long long ncell[kMaxLev] = {0, 0, 0, 0, 0, 0};     // cells per level
@@ -1484,31 +1484,21 @@ static int fetch_perm(const T* dev, long long c, const std::vector<long long>& p
     return DNSMC_OK;
 }
 
-// The caller's array to the device, in stream order; the array is free again on
-// return unless HIP knows its memory (a copy in the stream then).
-static hipError_t upload_host(dnsmc_solver* s, void* dev, const void* host, size_t bytes)
-{
-    if (bytes < HostPipe::kParallel || !HostPipe::pageable(host))
-        return hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, s->stream);
-    const HostRows job = host_block(dev, host, bytes);
-    return s->pipe_host.run(s->dev, s->stream, true, &job, 1);
-}
-
-// Device ranges into the caller's arrays, done on return.
+// Device ranges into the caller's arrays, done on return.  (Small ones one plain
+// copy after the other: the runtime's staged copy of 49 KB takes 10 us, four of
+// them 47 with the call; through a pinned buffer and an event each 97.)
 static hipError_t download_host(dnsmc_solver* s, const HostRows* jobs, int n)
 {
+    size_t total = 0;
+    for (int i = 0; i < n; ++i) total += jobs[i].bytes;
+    hipError_t e = hipStreamSynchronize(s->stream);
     HostRows pg[4];
     int np = 0;
-    for (int i = 0; i < n; ++i) {
-        if (HostPipe::pageable(jobs[i].host)) {
-            pg[np++] = jobs[i];
-            continue;
-        }
-        const hipError_t e = hipMemcpyAsync(jobs[i].host, jobs[i].dev, jobs[i].bytes, hipMemcpyDeviceToHost, s->stream);
-        if (e != hipSuccess) return e;
+    for (int i = 0; i < n && e == hipSuccess; ++i) {
+        if (total >= HostPipe::kParallel && HostPipe::pageable(jobs[i].host)) pg[np++] = jobs[i];
+        else e = hipMemcpy(jobs[i].host, jobs[i].dev, jobs[i].bytes, hipMemcpyDeviceToHost);
     }
-    const hipError_t e = s->pipe_host.run(s->dev, s->stream, false, pg, np);
-    return e != hipSuccess ? e : hipStreamSynchronize(s->stream);
+    return e != hipSuccess ? e : s->pipe_host.run(s->dev, s->stream, pg, np);
 }
 
 // After the fine field of snapshot `snap` is on the device: coarse levels by
@@ -1729,7 +1719,7 @@ int dnsmc_set_field(dnsmc_solver* s, int snap, const float* T, int is_device)
     const float* src = T;
     if (!is_device) {
         HIPCHK(s->d_stage.ensure(gsz));
-        HIPCHK(upload_host(s, s->d_stage.p, T, gsz * sizeof(float)));
+        HIPCHK(hipMemcpyAsync(s->d_stage.p, T, gsz * sizeof(float), hipMemcpyHostToDevice, s->stream));
         src = s->d_stage.p;
     }
     const long long nc = (long long)n0 * n1 * n2;
@@ -1772,7 +1762,7 @@ int dnsmc_fix_temp_slab(dnsmc_solver* s, int snap, const double* cnew, const int
     // cnew(0:n0+1, nj, nk) of the rank, i fastest
     const size_t cnt = (size_t)(n[0] + 2) * len[1] * len[2];
     HIPCHK(s->d_slab.ensure(cnt));
-    HIPCHK(upload_host(s, s->d_slab.p, cnew, cnt * sizeof(double)));
+    HIPCHK(hipMemcpyAsync(s->d_slab.p, cnew, cnt * sizeof(double), hipMemcpyHostToDevice, s->stream));
     const long long nc = (long long)len[0] * len[1] * len[2];
     const int nb = (int)std::min<long long>((nc + 255) / 256, (long long)s->ncu * 16);
     hipLaunchKernelGGL(slab_to_field, dim3(nb), dim3(256), 0, s->stream, (const double*)s->d_slab.p, n[0], n[1], n[2],
@@ -1966,7 +1956,7 @@ int dnsmc_get_results_fortran(dnsmc_solver* s, int snap, float* resfort, float* 
         job.p1 = p1;
         job.p2 = p2;
         job.p3 = (const char*)varfort - (const char*)resfort;
-        HIPCHK(s->pipe_host.run(s->dev, s->stream, false, &job, 1));
+        HIPCHK(s->pipe_host.run(s->dev, s->stream, &job, 1));
         return DNSMC_OK;
     }
     // the caller's arrays round-trip through the device so that the entries

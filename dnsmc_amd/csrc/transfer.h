@@ -1,11 +1,16 @@
-// Copies between device buffers and the caller's pageable arrays.
+// Copies of device buffers into the caller's pageable arrays.
 //
-// A plain hipMemcpy of pageable memory stages through the runtime's buffers on
-// one thread, and a fresh array's page faults are taken there too: 7 to 15 GB/s.
-// Here chunks of 1 MiB go through pinned buffers of the solver, and from
-// kParallel bytes on several threads move them (two chunks in flight each).
-// Results of 384x256x256 cells (2 x 101 MB): 26 -> 8 ms, a field of them in 3 ms;
-// four FP64 results of 256x128x128 cells (134 MB): 20 -> 6 ms.
+// A plain hipMemcpy to pageable memory stages through the runtime's buffers on
+// one thread, and a fresh array's page faults are taken there too.  Here chunks
+// of 1 MiB go through pinned buffers of the solver, and from kParallel bytes on
+// several threads move them (two chunks in flight each).  Measured, plain -> four
+// threads, into an array used before (a fresh one): 2.1 MB 118 -> 118 us, 3.2 MB
+// 185 -> 193, 4.2 MB 237 -> 225, 6.3 MB 360 -> 290, 17 MB 0.97 -> 0.63 ms, 105 MB
+// 5.9 (24) -> 3.4 (8.2) ms: below kParallel the plain copy is used unless rows
+// have to be placed.  Results of 384x256x256 cells (2 x 101 MB): 26 -> 8 ms.
+// Uploads are plain copies: 3.2 / 26 / 105 MB take 0.11 / 0.71 / 3.5 ms so, and
+// took 0.19 / 0.92 / 3.45 through such buffers.  A solver's first copy pays for
+// the buffers: 0.35 ms for 8 MiB.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <string.h>
@@ -33,7 +38,7 @@ inline HostRows host_block(const void* dev, const void* host, size_t bytes)
 
 class HostPipe {
 public:
-    static constexpr size_t kChunk = 1u << 20, kParallel = 2u << 20;
+    static constexpr size_t kChunk = 1u << 20, kParallel = 4u << 20;
     static constexpr int kWorkers = 4;
 
     ~HostPipe() { release(); }
@@ -50,7 +55,7 @@ public:
     }
 
     // Moves the jobs' ranges in stream order; the host side is done on return.
-    hipError_t run(int device, hipStream_t st, bool up, const HostRows* jobs, int njobs)
+    hipError_t run(int device, hipStream_t st, const HostRows* jobs, int njobs)
     {
         std::vector<Chunk> ch;
         size_t total = 0;
@@ -69,12 +74,12 @@ public:
             for (; made < T; ++made)
                 th[made] = std::thread([&, made] {
                     err[made] = hipSetDevice(device);
-                    if (err[made] == hipSuccess) err[made] = work(st, up, ch, made, T);
+                    if (err[made] == hipSuccess) err[made] = work(st, ch, made, T);
                 });
         } catch (const std::system_error&) {   // no thread to be had: this one does the rest
         }
-        err[0] = work(st, up, ch, 0, T);
-        for (int t = made; t < T; ++t) err[t] = work(st, up, ch, t, T);
+        err[0] = work(st, ch, 0, T);
+        for (int t = made; t < T; ++t) err[t] = work(st, ch, t, T);
         for (int t = 1; t < made; ++t) th[t].join();
         for (int t = 0; t < T; ++t)
             if (err[t] != hipSuccess) return err[t];
@@ -113,51 +118,37 @@ private:
             }
         return hipSuccess;
     }
-    static void rows(const Chunk& c, char* pin, bool up)
+    static void rows(const Chunk& c, const char* pin)
     {
         const HostRows& j = *c.j;
         for (size_t o = c.off; o < c.off + c.len;) {
             const long long r = (long long)(o / j.row);
             const size_t in = o - (size_t)r * j.row, n = std::min(j.row - in, c.off + c.len - o);
-            char* h = j.host + (r % j.n1) * j.p1 + (r / j.n1 % j.n2) * j.p2 + (r / (j.n1 * j.n2)) * j.p3 + in;
-            if (up) memcpy(pin + (o - c.off), h, n);
-            else memcpy(h, pin + (o - c.off), n);
+            memcpy(j.host + (r % j.n1) * j.p1 + (r / j.n1 % j.n2) * j.p2 + (r / (j.n1 * j.n2)) * j.p3 + in, pin + (o - c.off), n);
             o += n;
         }
     }
     // worker t of T: chunks t, t + T, ..., alternating between its two slots
-    hipError_t work(hipStream_t st, bool up, const std::vector<Chunk>& ch, int t, int T)
+    hipError_t work(hipStream_t st, const std::vector<Chunk>& ch, int t, int T)
     {
         hipError_t e = hipSuccess;
         const size_t n = ch.size();
         auto slot = [&](size_t c) { return 2 * t + (int)((c / T) & 1); };
         auto pin = [&](size_t c) { return pin_ + (size_t)slot(c) * kChunk; };
         auto issue = [&](size_t c) -> hipError_t {
-            char* d = ch[c].j->dev + ch[c].off;
-            hipError_t r = up ? hipMemcpyAsync(d, pin(c), ch[c].len, hipMemcpyHostToDevice, st)
-                              : hipMemcpyAsync(pin(c), d, ch[c].len, hipMemcpyDeviceToHost, st);
+            const hipError_t r = hipMemcpyAsync(pin(c), ch[c].j->dev + ch[c].off, ch[c].len, hipMemcpyDeviceToHost, st);
             return r != hipSuccess ? r : hipEventRecord(ev_[slot(c)], st);
         };
-        if (!up && (size_t)t < n) e = issue(t);
-        size_t c = t;
-        for (; c < n && e == hipSuccess; c += T) {
-            if (up) {
-                if (c >= 2 * (size_t)T && (e = hipEventSynchronize(ev_[slot(c)])) != hipSuccess) break;
-                rows(ch[c], pin(c), true);
-                e = issue(c);
-            } else {
-                if (c + T < n && (e = issue(c + T)) != hipSuccess) break;
-                if ((e = hipEventSynchronize(ev_[slot(c)])) != hipSuccess) break;
-                rows(ch[c], pin(c), false);
-            }
+        if ((size_t)t < n) e = issue(t);
+        for (size_t c = t; c < n && e == hipSuccess; c += T) {
+            if (c + T < n && (e = issue(c + T)) != hipSuccess) break;
+            if ((e = hipEventSynchronize(ev_[slot(c)])) != hipSuccess) break;
+            rows(ch[c], pin(c));
         }
-        // the slots are free again when the call returns (an event never recorded
-        // counts as complete)
-        if (up || e != hipSuccess)
-            for (int i = 2 * t; i < std::min(2 * t + 2, slots_); ++i) {
-                const hipError_t r = hipEventSynchronize(ev_[i]);
-                if (e == hipSuccess) e = r;
-            }
+        // after an error the slots are free again when the call returns (an event
+        // never recorded counts as complete)
+        if (e != hipSuccess)
+            for (int i = 2 * t; i < std::min(2 * t + 2, slots_); ++i) (void)hipEventSynchronize(ev_[i]);
         return e;
     }
 };
