@@ -600,7 +600,7 @@ __device__ __forceinline__ float dot2bf(uint32_t a, uint32_t b, float c)
 
 __device__ __forceinline__ uint32_t readlane_u(uint32_t v, int l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, l); }
 
-// The trace kernel's argument block (its only argument, at offset 0 of the
+// A traversal kernel's argument block (its first argument, at offset 0 of the
 // kernel argument segment) through a pointer the compiler cannot see through:
 // fields read through it are loaded (scalar loads from the constant segment)
 // where they are used instead of being hoisted to the kernel's start and held
@@ -1996,8 +1996,13 @@ __device__ __forceinline__ double quad_min_d(double v)
     return min_f64(v, quad_d<kQuadXor2>(v));
 }
 
-// Work: waves claim `super` consecutive rays at a time and start new ones when
-// 16 lanes are idle.  The drain below is the FP32 traversal's: when nothing is
+// Work (LONG): the rays are cut into a share per XCD; a wave takes `super` rays
+// of its XCD's share by its place, then claims as many at a time from a counter
+// per share, the others' when its own is used up, and starts new rays when 16
+// lanes are idle.  (One counter for all, the first chunks claimed too: its
+// atomics, 11 ns each, were a quarter of a launch of 4e5 short rays: 4e5 rays of
+// 3.3 crossings 0.275 -> 0.227 ms, 8e5 of 3.6 on three levels 0.545 -> 0.465.)
+// The drain below is the FP32 traversal's: when nothing is
 // left to hand out and at most 16 of a wave's rays run on, all on the last
 // level, four lanes follow a ray, kDrain crossings ahead, with the loop's
 // arithmetic and order (a crossing past the ray's end has length 0).
@@ -2005,10 +2010,14 @@ __device__ __forceinline__ double quad_min_d(double v)
 // Such a launch waits for its longest ray: one crossing after another takes
 // about 700 ns here (faces, field, table and exponential one behind the other).
 // 1024 cells x 8192 rays of a 64x96x64 channel, 9.1e7 crossings, longest ray
-// 16000: 12.1 ms with a thread per ray, 4.0 ms with the drain (the bulk about
+// 16000: 12.2 ms with a thread per ray, 3.6 ms with the drain (the bulk about
 // 1 ms of it).
-template <int SPEC, bool REC>
-__global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64, int super)
+//
+// Grey rays of few hundred crossings at most (!LONG, the host's rule) have no
+// long chain among them: a thread per ray, without the drain's registers (four
+// waves per SIMD instead of three).
+template <int SPEC, bool REC, bool LONG>
+__global__ __launch_bounds__(256, LONG ? 1 : 4) void trace_f64(TraceArgs P, double2* pray64)
 {
     extern __shared__ float lds[];
     int* s_lev = (int*)lds;
@@ -2183,32 +2192,74 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64, i
         }
         capped();
     };
-    unsigned long long cb = 0, ce = 0;   // the wave's claimed rays
+    auto count_steps = [&]() {
+        for (int off = 32; off > 0; off >>= 1) steps_t += __shfl_xor(steps_t, off);
+        if (lane == 0) atomicAdd(P.nsteps, steps_t);
+    };
+    if (!LONG) {
+        for (long long r = blockIdx.x * (long long)blockDim.x + threadIdx.x; r < P.nrays; r += (long long)gridDim.x * blockDim.x) {
+            q = (uint32_t)r;
+            start();
+            while (alive) cross();
+        }
+        count_steps();
+        return;
+    }
+    // the wave's rays cb..ce: at first a chunk by its place among the waves of
+    // its XCD's share, then claimed ones
+    uint32_t cb = 0, ce = 0;
+    auto waves = [&](uint32_t X) -> uint32_t { return ((gridDim.x + 7u - X) >> 3) * 4u; };
+    // chunk c (of S rays) of share X (p rays): its waves' places come first, then
+    // its counter's claims
+    auto take_chunk = [&](uint32_t X, uint32_t c, uint32_t S, uint32_t nrays, uint32_t p) -> bool {
+        const uint32_t n = X * p < nrays ? min(p, nrays - X * p) : 0u;
+        if (c * S >= n) return false;
+        cb = readlane_u(X * p + c * S, 0);
+        ce = readlane_u(cb + min(S, n - c * S), 0);
+        return true;
+    };
+    auto share = [](uint32_t nrays) -> uint32_t { return ((nrays + 7u) / 8u + 63u) / 64u * 64u; };
+    uint32_t home = (blockIdx.x & 7u) | 8u;  // its XCD; bit 3 while that share may have rays left
+    // one try: false when no share has rays left (cb == ce: another wave was first);
+    // readlane: the compiler then keeps the hand-out in scalar registers
+    auto claim = [&]() -> bool {
+        const KArgs* K = kernel_args();      // (read here, not held through the traversal)
+        const uint32_t nrays = (uint32_t)__builtin_amdgcn_readfirstlane((int)K->nrays);
+        const uint32_t S = (uint32_t)__builtin_amdgcn_readfirstlane(K->super), p = share(nrays);
+        uint32_t X = home & 7u;
+        if (!(home & 8u)) {
+            bool has = false;                // lane x: share x has rays left
+            if (lane < 8 && lane * p < nrays)
+                has = S * (waves(lane) + __hip_atomic_load(K->claim + 32 * lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) <
+                      min(p, nrays - lane * p);
+            const uint32_t left = readlane_u((uint32_t)__ballot(has), 0);
+            if (!left) return false;
+            X = (X + (uint32_t)__builtin_ctz((left | (left << 8)) >> X)) & 7u;
+        }
+        uint32_t c = 0;
+        if (lane == 0) c = atomicAdd(K->claim + 32u * X, 1u);
+        if (!take_chunk(X, waves(X) + (uint32_t)__builtin_amdgcn_readfirstlane((int)c), S, nrays, p)) home = readlane_u(home & 7u, 0);
+        return true;
+    };
+    take_chunk(home & 7u, (blockIdx.x >> 3) * 4u + (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6)), (uint32_t)P.super,
+               (uint32_t)P.nrays, share((uint32_t)P.nrays));
     bool more = true;
     for (;;) {
         unsigned long long idle = __ballot(!alive);
         if (more && __popcll(idle) >= 16) {
             while (idle) {
-                if (cb >= ce) {
-                    unsigned long long r = 0;
-                    if (lane == 0) r = atomicAdd((unsigned long long*)P.claim, (unsigned long long)super);
-                    r = ((unsigned long long)(uint32_t)__builtin_amdgcn_readfirstlane((int)(r >> 32)) << 32) |
-                        (uint32_t)__builtin_amdgcn_readfirstlane((int)r);
-                    if (r >= (unsigned long long)P.nrays) {
-                        more = false;
-                        break;
-                    }
-                    cb = r;
-                    ce = min(r + (unsigned long long)super, (unsigned long long)P.nrays);
+                if (cb >= ce && !claim()) {
+                    more = false;
+                    break;
                 }
                 const int rank = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
                                                                 __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
-                const int take = (int)min((unsigned long long)__popcll(idle), ce - cb);
-                if (!alive && rank < take) {
-                    q = (uint32_t)(cb + (unsigned long long)rank);
+                const uint32_t take = min((uint32_t)__popcll(idle), ce - cb);
+                if (!alive && (uint32_t)rank < take) {
+                    q = cb + (uint32_t)rank;
                     start();
                 }
-                cb += (unsigned long long)take;
+                cb += take;
                 idle = __ballot(!alive);
             }
         }
@@ -2430,13 +2481,14 @@ __global__ __launch_bounds__(256) void trace_f64(TraceArgs P, double2* pray64, i
         }
         __builtin_amdgcn_s_setprio(0);
     }
-    for (int off = 32; off > 0; off >>= 1) steps_t += __shfl_xor(steps_t, off);
-    if (lane == 0) atomicAdd(P.nsteps, steps_t);
+    count_steps();
 }
-template __global__ void trace_f64<kSpecTable, false>(TraceArgs, double2*, int);
-template __global__ void trace_f64<kSpecTable, true>(TraceArgs, double2*, int);
-template __global__ void trace_f64<kSpecGreyT4, false>(TraceArgs, double2*, int);
-template __global__ void trace_f64<kSpecGreyT4, true>(TraceArgs, double2*, int);
+#define DN_TRACE64_INST(S, R, D) template __global__ void trace_f64<S, R, D>(TraceArgs, double2*);
+#define DN_TRACE64_INST2(S, R) DN_TRACE64_INST(S, R, false) DN_TRACE64_INST(S, R, true)
+DN_TRACE64_INST(kSpecTable, false, true)
+DN_TRACE64_INST(kSpecTable, true, true)
+DN_TRACE64_INST2(kSpecGreyT4, false)
+DN_TRACE64_INST2(kSpecGreyT4, true)
 
 #define DN_TRACE_INST(S, I, T, R, A, G) template __global__ void trace<S, I, T, R, A, G>(TraceArgs);
 #define DN_TRACE_INST2(S, I, T, R, G) DN_TRACE_INST(S, I, T, R, false, G) DN_TRACE_INST(S, I, T, R, true, G)

@@ -31,8 +31,8 @@ __global__ void t_range(RangeArgs a);
 __global__ void raygen_plain(GenArgs a);
 __global__ void raygen_compat(GenArgs a);
 __global__ void raygen_compat_sorted(GenArgs a);
-template <int SPEC, bool REC>
-__global__ void trace_f64(TraceArgs P, double2* pray64, int super);
+template <int SPEC, bool REC, bool LONG>
+__global__ void trace_f64(TraceArgs P, double2* pray64);
 __global__ void finalize(const double* E, const double* A, const double* Q2, long long nemit, int spe, int R,
                          int compat, double* Q, double* Eo, double* Ao, double* sd);
 template <int AXIS>
@@ -739,6 +739,27 @@ static FeatArgs feat_args(dnsmc_solver* s, const Derived& d)
     return f;
 }
 
+// Most crossings a grey ray can have: tau_cut / kappa of path in the smallest
+// cells, at most maxs on each level but the last.  The FP64 traversal takes a
+// thread per ray up to 384: 4e5 rays of at most 30 / 300 crossings 0.15 / 0.20 ms
+// so and 0.18 / 0.21 with claims and drain, 3e6 of at most 129 / 310 0.68 / 0.96
+// and 0.77 / 1.0, 8e5 of at most 460 0.44 and 0.43, 3e6 of at most 1290 2.5 and 2.1.
+static double most_grey_crossings(const dnsmc_solver* s, float tau_cut)
+{
+    double most = 0.0;
+    for (size_t l = 0; l < s->lev.size(); ++l) {
+        double path = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            const std::vector<float>& f = s->lev[l].faces[a];
+            float dmin = s->cfg.L[a];
+            for (size_t i = 1; i < f.size(); ++i) dmin = std::min(dmin, f[i] - f[i - 1]);
+            path += (double)tau_cut / s->cfg.kappa_grey / dmin;
+        }
+        most += l + 1 < s->lev.size() ? std::min(path, (double)s->lev[l].maxs) : path;
+    }
+    return most;
+}
+
 // The whole solve, queued.  With `na` (dnsmc_run_noalloc) nothing is
 // allocated: the fused plain path only, counters and tallies in the scratch
 // array, results into the caller's arrays, no timing events.
@@ -1379,13 +1400,15 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             HIPCHK(hipEventRecord(et.a, st));
             if (f64) {
                 const size_t lds64 = sizeof(float) * (6 * kLevWords + P.nfaces + P.noffs + P.ncent + 6 * (size_t)d.nB);
-                // three waves per SIMD (registers); about four claims per wave
-                const int nb = (int)std::min<long long>((nr + 255) / 256, (long long)s->ncu * 3);
-                const int super = (int)std::max(64ll, std::min<long long>(512, nr / (16ll * nb) / 64 * 64));
-                void (*k)(TraceArgs, double2*, int) =
-                    spec == kSpecGreyT4 ? (rec ? trace_f64<kSpecGreyT4, true> : trace_f64<kSpecGreyT4, false>)
-                                        : (rec ? trace_f64<kSpecTable, true> : trace_f64<kSpecTable, false>);
-                hipLaunchKernelGGL(k, dim3(nb), dim3(256), lds64, st, P, pp.d_pray64.p, super);
+                // three waves per SIMD (registers); about four chunks per wave
+                const bool longer = spec != kSpecGreyT4 || most_grey_crossings(s, P.tau_cut) > 384.0;
+                const int nb = (int)std::min<long long>((nr + 255) / 256, (long long)s->ncu * (longer ? 3 : 16));
+                P.super = (int)std::max(64ll, std::min<long long>(512, nr / (16ll * nb) / 64 * 64));
+                void (*k)(TraceArgs, double2*) =
+                    spec != kSpecGreyT4 ? (rec ? trace_f64<kSpecTable, true, true> : trace_f64<kSpecTable, false, true>)
+                    : longer            ? (rec ? trace_f64<kSpecGreyT4, true, true> : trace_f64<kSpecGreyT4, false, true>)
+                                        : (rec ? trace_f64<kSpecGreyT4, true, false> : trace_f64<kSpecGreyT4, false, false>);
+                hipLaunchKernelGGL(k, dim3(nb), dim3(256), lds64, st, P, pp.d_pray64.p);
             } else {
                 HIPCHK(launch_trace(spec, tab, false, det, rec, amc, s->ncu, tb_cap, lds_trace, st, P));
             }
