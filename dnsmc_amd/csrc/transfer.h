@@ -16,9 +16,7 @@
 #include <string.h>
 
 #include <algorithm>
-#include <system_error>
 #include <thread>
-#include <vector>
 
 namespace dn {
 
@@ -57,15 +55,15 @@ public:
     // Moves the jobs' ranges in stream order; the host side is done on return.
     hipError_t run(int device, hipStream_t st, const HostRows* jobs, int njobs)
     {
-        std::vector<Chunk> ch;
+        Chunks ch{jobs, njobs, 0};
         size_t total = 0;
         for (int j = 0; j < njobs; ++j) {
             total += jobs[j].bytes;
-            for (size_t o = 0; o < jobs[j].bytes; o += kChunk) ch.push_back(Chunk{jobs + j, o, std::min(kChunk, jobs[j].bytes - o)});
+            ch.n += Chunks::of(jobs[j]);
         }
-        if (ch.empty()) return hipSuccess;
+        if (ch.n == 0) return hipSuccess;
         const int T = total < kParallel ? 1 : kWorkers;
-        hipError_t e = ensure(T == 1 && ch.size() == 1 ? 1 : 2 * T);
+        hipError_t e = ensure(T == 1 && ch.n == 1 ? 1 : 2 * T);
         if (e != hipSuccess) return e;
         hipError_t err[kWorkers] = {hipSuccess, hipSuccess, hipSuccess, hipSuccess};
         std::thread th[kWorkers];
@@ -76,7 +74,7 @@ public:
                     err[made] = hipSetDevice(device);
                     if (err[made] == hipSuccess) err[made] = work(st, ch, made, T);
                 });
-        } catch (const std::system_error&) {   // no thread to be had: this one does the rest
+        } catch (...) {   // no thread to be had, or no memory for one: this one does the rest
         }
         err[0] = work(st, ch, 0, T);
         for (int t = made; t < T; ++t) err[t] = work(st, ch, t, T);
@@ -90,6 +88,18 @@ private:
     struct Chunk {
         const HostRows* j;
         size_t off, len;
+    };
+    struct Chunks {   // the jobs' ranges in pieces of kChunk (nothing allocated)
+        const HostRows* jobs;
+        int njobs;
+        size_t n;
+        static size_t of(const HostRows& j) { return (j.bytes + kChunk - 1) / kChunk; }
+        Chunk operator[](size_t c) const
+        {
+            const HostRows* j = jobs;
+            for (; c >= of(*j); ++j) c -= of(*j);
+            return Chunk{j, c * kChunk, std::min(kChunk, j->bytes - c * kChunk)};
+        }
     };
     char* pin_ = nullptr;
     int slots_ = 0;
@@ -129,14 +139,15 @@ private:
         }
     }
     // worker t of T: chunks t, t + T, ..., alternating between its two slots
-    hipError_t work(hipStream_t st, const std::vector<Chunk>& ch, int t, int T)
+    hipError_t work(hipStream_t st, const Chunks& ch, int t, int T)
     {
         hipError_t e = hipSuccess;
-        const size_t n = ch.size();
+        const size_t n = ch.n;
         auto slot = [&](size_t c) { return 2 * t + (int)((c / T) & 1); };
         auto pin = [&](size_t c) { return pin_ + (size_t)slot(c) * kChunk; };
         auto issue = [&](size_t c) -> hipError_t {
-            const hipError_t r = hipMemcpyAsync(pin(c), ch[c].j->dev + ch[c].off, ch[c].len, hipMemcpyDeviceToHost, st);
+            const Chunk k = ch[c];
+            const hipError_t r = hipMemcpyAsync(pin(c), k.j->dev + k.off, k.len, hipMemcpyDeviceToHost, st);
             return r != hipSuccess ? r : hipEventRecord(ev_[slot(c)], st);
         };
         if ((size_t)t < n) e = issue(t);
