@@ -651,6 +651,11 @@ static hipError_t launch_trace_t(bool amc, int ncu, int max_blocks, size_t lds, 
     P.retire_steps = 1536;
     P.retire_from = (unsigned)std::max(0ll, nclaim - 64 * waves / 8);
     P.retire_most = (unsigned)(waves / 16);
+    if (const char* rt = getenv("DNSMC_RETIRE")) {   // beyond n crossings, at any time; 0: never
+        P.retire_steps = std::max(1, std::min(atoi(rt), 1 << 26));
+        P.retire_from = 0;
+        if (atoi(rt) <= 0) P.retire_most = 0;
+    }
     hipLaunchKernelGGL(k, dim3(nb), dim3(threads), lds, st, P);
     return hipGetLastError();
 }
@@ -2034,6 +2039,13 @@ int dnsmc_get_array(dnsmc_solver* s, const char* name, int level, float* out, lo
                 for (int j = 0; j < ln[1]; ++j)
                     for (int i = 0; i < ln[0]; ++i)
                         v[o++] = b[(size_t)sn * s->tstride[level] + brick_index(i, j, k, s->nbx[level], s->nby[level])];
+    } else if (nm == "retired") {
+        // claim words 16 to 19 of the last traversal launch on the main stream: the
+        // waves that asked to stop claiming beyond 1, 2, 4 and 8 times the threshold
+        if (s->last_nemit == 0) return fail(DNSMC_ESTATE, "run the solver first");
+        unsigned asks[4];
+        HIPCHK(hipMemcpy(asks, s->pipe[0].d_claim.p + 16, sizeof asks, hipMemcpyDeviceToHost));
+        v.assign(asks, asks + 4);
     } else if (nm == "qcdf") {
         // the learned proposal's cumulative weights of the last batch, one row
         // of mlp_noutp(nB*nQ) per slot, rows in emitter order (the batch must

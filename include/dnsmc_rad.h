@@ -243,6 +243,9 @@ int dnsmc_set_emitters_list(dnsmc_solver *s, const int *cells, int ncells);
  *                     launches of a solve also stay on one stream)
  *   DNSMC_TABLES=global  keep kappa / Planck tables out of LDS
  *   DNSMC_REFILL_K=k  idle lanes of a wave before it starts new rays
+ *   DNSMC_RETIRE=n    a wave with a ray beyond n crossings may stop claiming
+ *                     rays at any time (default: beyond 1536 near the end of
+ *                     the launch; 0: never)
  *   DNSMC_SUPER=n     rays per claimed super-chunk (multiple of 64)
  *   DNSMC_BLOCK=n     threads per block of the traversal with LDS table
  *                     slices (default 1024: one block and 16 waves per CU)
@@ -283,8 +286,9 @@ int dnsmc_get_stats(dnsmc_solver *s, dnsmc_stats *st);
 
 /* Test and training hooks. */
 /* Derived arrays: name in {"faces0","faces1",..,"centres","T1".."T5","cdf_band","cdf_g",
- * "inv_emax","Ib","kq","Ibw","scalars","p_bg","pcdf","qcdf","lrows","features"}; copies up to n
- * floats, returns count.  "qcdf": the learned proposal's cumulative weights of the
+ * "inv_emax","Ib","kq","Ibw","scalars","p_bg","pcdf","qcdf","lrows","features","retired"}; copies
+ * up to n floats, returns count.  "retired": how many waves of the last traversal launch on the
+ * solver's main stream asked to stop claiming, beyond 1, 2, 4 and 8 times the threshold.  "qcdf": the learned proposal's cumulative weights of the
  * last batch, a row per slot in emitter order (the batch must cover every slot);
  * "features": the proposal's 6 input features per slot of the last run, emitter order. */
 int dnsmc_get_array(dnsmc_solver *s, const char *name, int level, float *out, long long n);
