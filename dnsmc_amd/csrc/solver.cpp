@@ -1225,7 +1225,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
                 s->first_batch_rays = nslots * (long long)R;
             }
         }
-        // long rays first (the plain in-kernel draw; DNSMC_LONG_FIRST=0: off)
+        // long rays first (the plain in-kernel draw; DNSMC_LONG_FIRST: 0 off, 1 on)
         bool long_first = !lfused;
         // a grey ray ends after tau_cut / kappa of path: with few crossings at
         // most there is no long ray to list; nor is there an order to choose
@@ -1241,7 +1241,7 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
             if (cross < 4096.0) long_first = false;
         }
         if (nslots * (long long)R * c.nsnap <= 16ll * 64 * s->ncu) long_first = false;
-        if (const char* lf = getenv("DNSMC_LONG_FIRST")) long_first = long_first && atoi(lf) != 0;
+        if (const char* lf = getenv("DNSMC_LONG_FIRST")) long_first = !lfused && atoi(lf) != 0;
         // the listed part, the final 1/long_part of each XCD range of the last
         // snapshot: a half in launches of several snapshots, a quarter in
         // one-snapshot launches (measured on 384x256x256: 8 snapshots 3200 /

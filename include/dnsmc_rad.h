@@ -232,7 +232,10 @@ int dnsmc_set_emitters_list(dnsmc_solver *s, const int *cells, int ncells);
  *   DNSMC_FUSED=0     batched generation for the plain estimator too
  *   DNSMC_FUSED_SLOTS=n  at most n slots per fused launch
  *   DNSMC_LONG_FIRST=0   fused launches trace in claim order only (no
- *                     list of the rays along the walls traced first)
+ *                     list of the rays along the walls traced first); 1:
+ *                     with the list also where it is off by default (grey
+ *                     gas of few crossings, launches whose rays all start
+ *                     at once)
  *   DNSMC_LONG_PART=k    list those rays from the final 1/k of each XCD's
  *                     share of the last snapshot (default 2 with several
  *                     snapshots per launch, 4 with one)
