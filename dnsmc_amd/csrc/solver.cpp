@@ -1139,6 +1139,8 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
     const size_t lds_gen = sizeof(float) * ((size_t)d.nB + (size_t)d.nB * d.nQ + (gib ? (size_t)d.nB * d.nT : 0) + 64);
     const bool sorted = c.mode == DNSMC_MODE_COMPAT && d.sorted;
     const size_t lds_sorted = sizeof(float) * (2 * (size_t)d.nB + 3 * (size_t)d.nB * d.nQ + 64);
+    // (the table sizes that reference sampling takes are those of the other
+    // generators; its own kernel would need less)
     if (c.mode == DNSMC_MODE_COMPAT && !sorted && lds_gen > s->lds_max)
         return fail(DNSMC_EDEVICE, "reference sampling: too many (band, g) bins for the proposal's CDFs in LDS");
     const int compat_threads = std::min(256, (c.photmax + 64 * std::max(1, G.run_len) - 1) / (64 * std::max(1, G.run_len)) * 64);
