@@ -18,7 +18,6 @@ struct LevParams {
     int n[3];
     int foff[3];      // offsets of the face arrays in the packed face buffer
     int maxs;
-    int nbx, nby;        // 4x4x4 bricks along x and y
     int ooff[3];         // offsets of the brick-offset tables in the packed table buffer
     long long tstride;   // floats of this level per snapshot (bricked, padded)
 };

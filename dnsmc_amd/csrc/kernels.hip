@@ -723,14 +723,6 @@ __device__ __forceinline__ bool long_candidate(const A& P, uint32_t q, uint32_t 
            mt - (1u << 23) + P.cand_w < 2u * P.cand_w;
 }
 
-// The long-ray candidates of a fused launch: each ray of the final part of
-// the 8 XCD ranges of the launch's last snapshot (nfin rays per range from
-// cand_from on, those below nrays) gets the plain draw's Philox block, and
-// the rays that pass long_candidate go to their range's list (list x at
-// x * cand_cap, its count at cand_cnt[64 x]; every hit is counted, also past
-// cand_cap).  A block takes tiles of kCandTile rays of one range and stages
-// the tile's hits in LDS: one global atomic per tile.
-constexpr uint32_t kCandTile = 4096;
 // Crossings per iteration of the traversal, their field loads in flight together
 // (a wave's lanes meet an L2 miss nearly every crossing, and only four waves
 // per SIMD hide it).  A ray that ends inside an iteration wastes the rest.
@@ -812,6 +804,15 @@ __device__ __forceinline__ int quad_min_i(int v)
     v = min(v, quad_i<kQuadXor1>(v));
     return min(v, quad_i<kQuadXor2>(v));
 }
+
+// The long-ray candidates of a fused launch: each ray of the final part of
+// the 8 XCD ranges of the launch's last snapshot (nfin rays per range from
+// cand_from on, those below nrays) gets the plain draw's Philox block, and
+// the rays that pass long_candidate go to their range's list (list x at
+// x * cand_cap, its count at cand_cnt[64 x]; every hit is counted, also past
+// cand_cap).  A block takes tiles of kCandTile rays of one range and stages
+// the tile's hits in LDS: one global atomic per tile.
+constexpr uint32_t kCandTile = 4096;
 __global__ __launch_bounds__(256) void cand_scan(TraceArgs P, uint32_t nfin, uint32_t* list)
 {
     __shared__ uint32_t s_q[kCandTile];
@@ -875,11 +876,13 @@ __global__ __launch_bounds__(256) void cand_scan(TraceArgs P, uint32_t nfin, uin
 // another slot.  TMODE 1 writes each ray's (E, A) for the deterministic
 // reduce_rays pass.
 //
-// One step: the kappa gather of the current cell is issued first, the
-// geometry (distances, face snap, move, boundary) runs while it is in flight,
-// the next cell's field load is issued at the end of the geometry, and the
-// optical depth / transmissivity / tally update consumes kappa last.  With
-// the kappa/Ib slice in LDS the field holds table coordinates (t_to_u).
+// One iteration: a lane first walks kAhead crossings (distances, face snap,
+// move, boundary; which cells a ray crosses does not depend on the field) with
+// each next cell's field load issued as its offsets are known, then the table
+// lookups, optical depth, transmissivity and gathered emission of the same
+// crossings follow in order, each taking the field value of the crossing
+// before.  With the kappa/Ib slice in LDS the field holds table coordinates
+// (t_to_u).  A wave's last rays are followed by four lanes each (the drain).
 //
 // GEN: the rays are drawn in the kernel instead of read from descriptors
 // (1: the plain estimator's Philox draw, bit-identical to raygen_plain; 2:
@@ -928,16 +931,15 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     for (int i = threadIdx.x; i < P.nlev; i += blockDim.x) {
         int* L = s_lev + i * kLevWords;
         L[0] = P.lev[i].n[0]; L[1] = P.lev[i].n[1]; L[2] = P.lev[i].n[2];
-        // per axis: LDS address of face 0, and from a cell's low face (word
-        // c - 1 of 1-based cell c) to its word of the brick-offset table
+        // per axis: LDS address of face 0
         L[3] = face0 + 4 * P.lev[i].foff[0]; L[4] = face0 + 4 * P.lev[i].foff[1]; L[5] = face0 + 4 * P.lev[i].foff[2];
         L[6] = P.lev[i].maxs;
         const float* tb = P.T[i] + (size_t)P.snap * P.lev[i].tstride;
         unsigned long long u = (unsigned long long)tb;
         L[7] = (int)(uint32_t)u;
         L[8] = (int)(uint32_t)(u >> 32);
-        L[9] = P.lev[i].nbx;
-        L[10] = P.lev[i].nby;
+        // from a cell's low face (word c - 1 of 1-based cell c) to its word of the
+        // brick-offset table
         for (int a = 0; a < 3; ++a) L[11 + a] = off0 - face0 + 4 * (P.lev[i].ooff[a] - P.lev[i].foff[a]);
         L[14] = (int)P.lev[i].tstride;
         int before = 0;                          // crossings on the finer levels
@@ -1241,8 +1243,9 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     };
     // Retiring: a wave asked to claim more work near the launch's end (its last
     // claim at retire_from or later) while one of its rays is beyond ask_at
-    // crossings stops claiming, so that it reaches the drain below (over four
-    // times faster per crossing) while the other waves trace the rest.  At most
+    // crossings stops claiming, so that it reaches the drain below (105 ns per
+    // crossing against some 850 at the bulk's pace) while the other waves trace
+    // the rest.  At most
     // retire_most waves of the launch do for rays beyond retire_steps (counted
     // in claim word 16), as many beyond twice that for the waves that were
     // refused (word 17), and so on up to word 19: the longest rays are not left

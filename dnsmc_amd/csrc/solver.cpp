@@ -965,8 +965,6 @@ static int do_run(dnsmc_solver* s, const NoAlloc* na)
         }
         P.lev[l].maxs = s->lev[l].maxs;
         P.lev[l].tstride = s->tstride[l];
-        P.lev[l].nbx = s->nbx[l];
-        P.lev[l].nby = s->nby[l];
         for (int a = 0; a < 3; ++a) P.lev[l].ooff[a] = s->ooff[l][a];
         P.T[l] = s->d_T[l].p;
     }
