@@ -1050,9 +1050,13 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     // The finished rays of all lanes.  Where they share one slot and its ring
     // entry, the sum of each 16 lanes is added once: the atomics of lanes on one
     // address take the LDS one lane after the other.  For descriptor launches of
-    // at least 256 rays per slot, where most refills meet one slot: 3.7e8 rays of
-    // 20000 per slot and 2.6 crossings 12.4 -> 10.6 ms (quads: 10.9); at 100 per
-    // slot 0.8 % slower, and a fused launch of 500 per slot no faster.
+    // at least 256 rays per slot, where most refills meet one slot.  Traversal of
+    // reference sampling without and with it, by rays per slot (three levels,
+    // sorted bands): 100 10.3 / 10.3 ms, 160 11.7 / 11.7, 256 19.5 / 18.9, 800
+    // 7.33 / 7.03, 5000 34.0 / 31.0, 20000 (2.6 crossings) 12.4 / 10.7 (quads: 10.9);
+    // learned rays on four levels: 100 and 160 the same, 256 4.79 / 4.63, 400 7.70 /
+    // 7.26, 1600 27.4 / 25.1; on one level the same within 1 % up to 1600.  A fused
+    // launch of 500 per slot is no faster.
     const bool wide = QUEUE && GEN == 0 && P.rays_per_slot >= 256;
     auto ring_tally_wave = [&](bool f, float er, float ar) {
         const unsigned long long fm = __ballot(f);
@@ -1721,7 +1725,7 @@ __global__ __launch_bounds__(TAB == kTabSliced ? 1024 : 256) void trace(TraceArg
     // follow in crossing order with the main loop's arithmetic (a crossing
     // past the ray's end has length 0 and adds 0): 122 ns per crossing with
     // a branch per crossing for walls, wraps and ties, 105 ns without (below):
-    // a solve bound by one ray of 16000 crossings 2.22 -> 2.05 ms.  Batches of
+    // a launch bound by one ray of 16000 crossings 2.23 -> 2.04 ms.  Batches of
     // 8, 16, 24 and 32 crossings: 2.34, 2.03, 2.18 and 2.22 ms there.  The
     // first solve 46 -> 22 ms (18 with retiring waves, above).
     if (__ballot(alive)) {
@@ -2013,8 +2017,8 @@ __device__ __forceinline__ double quad_min_d(double v)
 // Such a launch waits for its longest ray: one crossing after another takes
 // about 700 ns here (faces, field, table and exponential one behind the other).
 // 1024 cells x 8192 rays of a 64x96x64 channel, 9.1e7 crossings, longest ray
-// 16000: 12.2 ms with a thread per ray, 3.6 ms with the drain (the bulk about
-// 1 ms of it).
+// 16000, on three temperature fields: 12.2, 8.5 and 8.8 ms with a thread per ray,
+// 3.9, 2.7 and 2.7 ms with the drain (the bulk about 1 ms of it).
 //
 // Grey rays of few hundred crossings at most (!LONG, the host's rule) have no
 // long chain among them: a thread per ray, without the drain's registers (four

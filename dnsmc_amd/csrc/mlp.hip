@@ -144,13 +144,14 @@ __device__ __forceinline__ void put_w3_tile(const uint4& r0, const uint4& r1, ui
 // 256 of them: 115 MB each way, 0.42 ms per step of 16384 rows (320 us of tile
 // kernel at one block per CU, 79 us of reduction, 19 us of weight sum).  Here
 // W3's part (96 % of the parameters) is kept in registers over the rows of a
-// split: 0.14 ms for the same step (462 -> 142 us with the update; kernels 75 us
-// for the rows, two blocks per CU, bound by the exponentials and LDS reads of
-// the two passes over W3's columns, 27 us for dW3, 11 us for the sums).  Every
-// sum over rows, columns and blocks below W3 keeps the first form's order, so
-// those gradients are bit for bit what they were.  dZ leaves the logits'
-// accumulators in the layout of the next product's operand (rows
-// 4 (l / 16) + i, column l % 16), so dW3 = H2^T dZ takes it from registers.
+// split: 0.14 ms for the same step (462 -> 142 us with the update; kernels 73 us
+// for the rows, a block per CU and so one wave per SIMD, bound by that wave's
+// chain through two passes over W3's columns (VALU at 0.40 of its issue peak);
+// 26 us for dW3, 11 us for the sums).  Every sum over rows, columns and blocks
+// below W3 keeps the first form's order, so those gradients are bit for bit what
+// they were.  dZ leaves the logits' accumulators in the layout of the next
+// product's operand (rows 4 (l / 16) + i, column l % 16), so dW3 = H2^T dZ takes
+// it from registers.
 
 // Four BF16 of consecutive k as an MFMA operand, from an 8-byte aligned address.
 __device__ __forceinline__ s4v frag8(const uint16_t* p)
